@@ -38,3 +38,14 @@ def test_inference_tensors_have_no_order(pkg, oracle):
         pk = pkg.ops.make_packed(*t, 64, 0)
         pk.find_order()
     assert pk.order is None
+
+
+def test_copies_made_under_inference_mode(pkg, oracle):
+    """A serving process copies layers in that mode; the copy's tensors count no writes."""
+    qw, qz, sc, gi = oracle.make_gptq(256, 64, 64, seed=5, sym=False, act_order=True)
+    t = [torch.from_numpy(np.ascontiguousarray(a.view(np.int32) if a.dtype == np.uint32 else a)) for a in (qw, qz, sc, gi)]
+    pk = pkg.ops.make_packed(*t, 64, 0)
+    pk.find_order()
+    with torch.inference_mode():
+        new = copy.deepcopy(pk)
+    assert torch.equal(new.g_idx, pk.g_idx) and new.regroup(2048, 0, False) == 0

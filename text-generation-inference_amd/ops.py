@@ -95,7 +95,8 @@ class PackedWeight:
             copy.deepcopy(self.qweight, memo), copy.deepcopy(self.qzeros, memo), copy.deepcopy(self.scales, memo),
             copy.deepcopy(self.g_idx, memo), self.K, self.N, self.groupsize, self.num_groups, self.layout,
             copy.deepcopy(self.perm, memo), _plans=dict(self._plans))
-        if self.order is not None and self.g_idx._version == self._order_version:
+        # (under inference_mode the copy is an inference tensor, which counts no writes: no order for it)
+        if self.order is not None and not new.g_idx.is_inference() and self.g_idx._version == self._order_version:
             new.order, new._order_version = copy.deepcopy(self.order, memo), new.g_idx._version
         return new
 
