@@ -22,12 +22,10 @@ def to_dev(a, gpu):
 def build(pkg, oracle, gpu, K, N, gs, seed):
     qw, qz, sc, gi = oracle.make_gptq(K, N, gs, seed=seed, sym=False, act_order=True)
     pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), to_dev(gi, gpu), gs, 0)
-    pk.find_order()
-    assert pk.order is not None
     return (qw, qz, sc, gi), pk
 
 
-def call(pkg, pk, x, act=-1, order=None):
+def call(pkg, pk, x, act=-1):
     lib, L = pkg._lib.load(), pkg._lib
     M, code = x.shape[0], pkg.ops._DTYPES[x.dtype]
     need = ctypes.c_size_t(0)
@@ -35,8 +33,7 @@ def call(pkg, pk, x, act=-1, order=None):
     assert need.value > 0
     ws = torch.zeros(need.value, dtype=torch.uint8, device=x.device)
     y = torch.empty((M, pk.N // (2 if act >= 0 else 1)), dtype=x.dtype, device=x.device)
-    order = pk.order if order is None else order
-    args = [ctypes.byref(pk.struct()), order.data_ptr(), x.data_ptr(), None, y.data_ptr(), M, code, act, ws.data_ptr()]
+    args = [ctypes.byref(pk.struct()), x.data_ptr(), None, y.data_ptr(), M, code, act, ws.data_ptr()]
     assert lib.q4_linear_regroup(*args, need.value - 1, pkg.ops._stream_handle(x.device)) == L.ERR_WORKSPACE
     L.check(lib.q4_linear_regroup(*args, need.value, pkg.ops._stream_handle(x.device)))
     return y
@@ -66,18 +63,94 @@ def test_regrouped_call_matches_oracle(pkg, oracle, gpu, K, N, gs, M, dtype):
     assert np.abs(got - want).max() <= 4 * (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) * np.abs(want).max()
 
 
-@pytest.mark.parametrize("K,N,M,regroups", [(512, 32768, 48, False), (4096, 28672, 48, True), (4096, 28672, 130, True)])
+@pytest.mark.parametrize("K,N,M,regroups", [(512, 32768, 48, False), (4096, 28672, 48, False), (4096, 28672, 130, True), (4096, 4096, 1024, False), (4096, 6144, 1536, True)])
 def test_layers_regroup_from_the_librarys_row_count_on(pkg, oracle, gpu, K, N, M, regroups):
     """The tensor calls take the regrouped route by the library's rule; gated and plain agree with the
     kernels that read through g_idx (the same weights, sums in another order)."""
     _, pk = build(pkg, oracle, gpu, K, N, 128, seed=N)
-    plain = pkg.ops.make_packed(pk.qweight, pk.qzeros, pk.scales, pk.g_idx, 128, 0)
     x = torch.randn((M, K), device=gpu, dtype=torch.float16) * 0.1
     assert (pk.regroup(M, 0, False) > 0) == regroups
-    for f in (lambda w: pkg.ops.linear(w, x), lambda w: pkg.ops.linear_gate_up(w, x)):
-        a, b = f(pk).float(), f(plain).float()
-        assert ((a - b).norm() / b.norm()).item() <= 2e-3
+    plain = pkg.ops.linear(pk, x, path=2)
+    for a, b in ((pkg.ops.linear(pk, x), plain), (pkg.ops.linear_gate_up(pk, x), pkg.ops.act_mul(plain))):
+        assert ((a.float() - b.float()).norm() / b.float().norm()).item() <= 2e-3
     assert pkg.ops.linear(pk, x[:0]).shape == (0, N)
-    order = pk.order.clone()
-    order[0], order[1] = -5, K + 7  # clamped: a wrong row, never outside
-    assert call(pkg, pk, x, order=order).shape == (M, N)
+
+
+# On the size below, 48 rows: the batch decode kernel on the copy; 200: the prefill kernels
+ROWS = [48, 200]
+
+
+def big(pkg, gpu, seed):
+    K, N, gs = 8192, 32768, 128
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    words = lambda *s: torch.randint(-(2**31), 2**31 - 1, s, dtype=torch.int32, device=gpu, generator=gen)  # noqa: E731
+    scales = (torch.rand((K // gs, N), device=gpu, generator=gen) * 0.019 + 0.001).half()
+    g_idx = (torch.arange(K, device=gpu) // gs)[torch.randperm(K, device=gpu, generator=gen)].int()
+    return pkg.ops.make_packed(words(K // 8, N), words(K // gs, N // 8), scales, g_idx, gs, 0)
+
+
+def against_g_idx(pkg, pk, x, plain=None, gated=None):
+    """Both calls against the kernels that read g_idx as it is in memory now."""
+    want = pkg.ops.linear(pk, x, path=2)
+    plain = pkg.ops.linear(pk, x) if plain is None else plain
+    gated = pkg.ops.linear_gate_up(pk, x) if gated is None else gated
+    for a, b in ((plain, want), (gated, pkg.ops.act_mul(want))):
+        assert ((a.float() - b.float()).norm() / b.float().norm()).item() <= 2e-3
+
+
+@pytest.mark.parametrize("M", ROWS)
+def test_a_call_reads_g_idx_when_it_runs(pkg, gpu, M):
+    """Entries written after the layer was prepared, counted by torch (copy_) or not (.data), are the ones used."""
+    pk = big(pkg, gpu, M)
+    pk.prepare()
+    assert pk.regroup(M, 0, False) > 0 and pk.regroup(M, 0, True) > 0
+    x = torch.randn((M, pk.K), device=gpu, dtype=torch.float16) * 0.1
+    against_g_idx(pkg, pk, x)
+    pk.g_idx.data.copy_(pk.g_idx[torch.randperm(pk.K, device=gpu)])
+    against_g_idx(pkg, pk, x)
+    pk.g_idx.copy_(pk.g_idx.flip(0))
+    against_g_idx(pkg, pk, x)
+
+
+@pytest.mark.parametrize("M", ROWS)
+def test_a_captured_call_reads_g_idx_when_it_is_replayed(pkg, gpu, M):
+    """Another checkpoint is copied into the buffers of a captured layer, as load_state_dict does it."""
+    pk = big(pkg, gpu, M)
+    pk.prepare()
+    x = torch.randn((M, pk.K), device=gpu, dtype=torch.float16) * 0.1
+    pkg.ops.linear(pk, x), pkg.ops.linear_gate_up(pk, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plain, gated = pkg.ops.linear(pk, x), pkg.ops.linear_gate_up(pk, x)
+    for seed in range(3):
+        src = big(pkg, gpu, seed)
+        for name in ("qweight", "qzeros", "scales", "g_idx"):
+            getattr(pk, name).copy_(getattr(src, name))
+        pk.prepare()
+        graph.replay()
+        torch.cuda.synchronize()
+        against_g_idx(pkg, pk, x, plain, gated)
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_uneven_groups_are_looked_up(pkg, gpu, M, dtype):
+    """Groups of other sizes, which only the device sees: the very kernels that read through g_idx."""
+    pk = big(pkg, gpu, M)
+    x = (torch.randn((M, pk.K), device=gpu) * 0.1).to(dtype)
+    for entries in (pk.g_idx.clamp(max=pk.num_groups - 2), torch.zeros_like(pk.g_idx), pk.g_idx - 1, pk.g_idx + 1):
+        pk.g_idx.copy_(entries)
+        want = pkg.ops.linear(pk, x, path=2)
+        assert torch.equal(pkg.ops.linear(pk, x), want)
+        assert torch.equal(pkg.ops.linear_gate_up(pk, x), pkg.ops.act_mul(want))
+
+
+@pytest.mark.parametrize("K,N,gs,M", [(128, 64, 32, 130), (2048, 272, 64, 33), (38400, 136, 128, 20), (1024, 8192, 1024, 64)])
+def test_uneven_groups_without_a_prefill_kernel(pkg, oracle, gpu, K, N, gs, M):
+    """Sizes that the library never regroups by itself, one group and columns in no whole tile among them."""
+    _, pk = build(pkg, oracle, gpu, K, N, gs, seed=K)
+    x = torch.randn((M, K), device=gpu, dtype=torch.float16) * 0.1
+    pk.g_idx.copy_(pk.g_idx.clamp(max=pk.num_groups // 2 - 1) if pk.num_groups > 1 else pk.g_idx - 1)
+    want = pkg.ops.linear(pk, x, path=2 if N % 128 == 0 else 3)
+    assert torch.equal(call(pkg, pk, x), want)

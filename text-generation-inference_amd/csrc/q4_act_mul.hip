@@ -7,7 +7,9 @@ namespace q4 {
 
 template <int DTYPE>
 __global__ __launch_bounds__(256) void act_mul_kernel(const uint16_t* __restrict__ gate_up,
-                                                      uint16_t* __restrict__ y, int M, int inter, int act) {
+                                                      uint16_t* __restrict__ y, int M, int inter, int act,
+                                                      const int32_t* __restrict__ only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   const int vec_per_row = inter >> 3;  // 8 values per 16-byte vector
   const long total = (long)M * vec_per_row;
   for (long v = (long)blockIdx.x * blockDim.x + threadIdx.x; v < total; v += (long)gridDim.x * blockDim.x) {
@@ -33,7 +35,8 @@ __global__ __launch_bounds__(256) void act_mul_kernel(const uint16_t* __restrict
 
 namespace q4host {
 
-int launch_act_mul(const void* gate_up, void* y, int M, int inter, int dtype, int act, hipStream_t stream) {
+int launch_act_mul(const void* gate_up, void* y, int M, int inter, int dtype, int act, hipStream_t stream,
+                   const int32_t* only_if) {
   if (inter % 8 != 0) {
     set_error("q4_act_mul: the intermediate size %d must be a multiple of 8", inter);
     return Q4_ERR_UNSUPPORTED;
@@ -44,10 +47,10 @@ int launch_act_mul(const void* gate_up, void* y, int M, int inter, int dtype, in
   if (blocks < 1) blocks = 1;
   if (dtype == Q4_DTYPE_F16)
     hipLaunchKernelGGL(q4::act_mul_kernel<Q4_DTYPE_F16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)gate_up, (uint16_t*)y, M, inter, act);
+                       (const uint16_t*)gate_up, (uint16_t*)y, M, inter, act, only_if);
   else
     hipLaunchKernelGGL(q4::act_mul_kernel<Q4_DTYPE_BF16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)gate_up, (uint16_t*)y, M, inter, act);
+                       (const uint16_t*)gate_up, (uint16_t*)y, M, inter, act, only_if);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     set_error("q4_act_mul: launch failed: %s", hipGetErrorString(err));

@@ -454,8 +454,28 @@ static q4_weight in_group_order(const q4_weight* w, const void* qweight) {
   return seq;
 }
 
-static size_t regroup_offset(int M, int K, int N) {
-  return (q4_workspace_bytes_perm(M, K, N) + 255) & ~(size_t)255;
+// Whether q4_linear_regroup can run at all: the groups' sizes add up to K, a panel of columns fits LDS, and there
+// is a kernel that reads through g_idx for the case that the groups turn out uneven.
+static bool regroup_runs(const q4_weight* w, int M, int dtype) {
+  if (w->g_idx == nullptr || (long)w->num_groups * w->groupsize != w->K || !regroup_supported(w->K, w->N)) return false;
+  return gemm_awq_supported(w, M, dtype) ? (long)(M + 127) / 128 * (w->N / 128) * 16 <= 0x7fffffffL : M <= 4 * 65535;
+}
+
+// Workspace of q4_linear_regroup behind that of the calls on the copy: the flag, one word per group, the row order,
+// and the copy, whose room also takes the [M, N] sums of a gated call through g_idx.
+struct RegroupLayout {
+  size_t any_uneven, uneven, perm, copy, bytes;
+};
+static RegroupLayout regroup_layout(const q4_weight* w, int M, bool gate_up) {
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  RegroupLayout l;
+  l.any_uneven = up(q4_workspace_bytes_perm(M, w->K, w->N));
+  l.uneven = l.any_uneven + 256;
+  l.perm = up(l.uneven + (size_t)w->num_groups * 4);
+  l.copy = up(l.perm + (size_t)w->K * 4);
+  const size_t copy = (size_t)w->K * w->N / 2, sums = gate_up ? (size_t)M * w->N * 2 : 0;
+  l.bytes = l.copy + (copy > sums ? copy : sums);
+  return l;
 }
 
 int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, size_t* workspace_bytes) {
@@ -467,9 +487,7 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
     return Q4_ERR_INVALID_ARGUMENT;
   }
   *workspace_bytes = 0;
-  if (M == 0 || w->N == 0 || w->g_idx == nullptr || (long)w->num_groups * w->groupsize != w->K ||
-      !regroup_supported(w->K, w->N))
-    return 0;
+  if (M == 0 || w->N == 0 || !regroup_runs(w, M, dtype)) return 0;
   const q4_weight seq = in_group_order(w, w->qweight);
   if (gate_up) {
     int fused = 0;
@@ -477,47 +495,83 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
     if (rc != Q4_OK) return rc;
     if (!fused) return 0;
   }
-  *workspace_bytes = regroup_offset(M, w->K, w->N) + (size_t)w->K * w->N / 2;
-  // The pass over the weights (8192 x 57344 131 us, 4096 x 4096 7) and the gather of x come back as rows and
-  // weights multiply.  Regrouped / through g_idx, us, groups of 128: 4096 x 6144 at M = 384 44 / 42, at 512 53 / 59;
-  // 8192 x 8192 at 128 59 / 46, at 192 68 / 74, at 1024 154 / 186; 14336 x 4096 at 256 70 / 67, at 300 1.2 times
-  // faster; 4096 x 4096 at 1024 60 / 65; 8192 x 57344 at 192 355 / 459; 28672 x 8192 at 1024 532 / 816.  Groups of
-  // 32, whose table does not fit LDS: 8192 x 8192 at 384 rows 2.0 times faster.  Up to 128 rows the kernels that
-  // read through g_idx hold one row block, flat in M.
+  *workspace_bytes = regroup_layout(w, M, gate_up != 0).bytes;
+  // (uneven groups then cost what they always did)
+  if (q4_select_path(w, M, dtype) != Q4_PATH_GEMM) return 0;
+  // Sorting g_idx (3 us), the pass over the weights (8192 x 57344 131 us, 4096 x 4096 7), the gather of x and the
+  // launches that end at the flag (3-7 us) come back as rows and weights multiply; the kernels that read through g_idx
+  // hold row blocks of 128 and 256, in which they are flat in M.  Time through g_idx over time regrouped, MI355X, 23
+  // layer shapes, groups of 32 to 128, 17 row counts, both data types, plain and gated:
+  //   33-64 rows    the batch decode kernel on the copy: 8192 x 57344 1.14-1.30; 4096 x 28672 0.94-1.06, 3584 x 37888
+  //                 0.91-1.05, narrower ones down to 0.6
+  //   N >= 2 K      4096 x 22016 .. 8192 x 57344: 129-192 rows 1.02-1.66, from 320 on 1.06-1.70; 193-256 rows 0.95-1.08
+  //                 below 1.3e8 weights, 1.03-1.40 above; 4096 x 12288 from 320 rows on 0.99-1.46, below 0.89-1.08
+  //   other shapes  from 6e10 rows x weights on 1.00-1.77 (28672 x 8192 at 256 rows, 6e10, 0.89: from 320 on), below
+  //                 0.66-1.48 (13824 x 5120 at 768 0.94, 4096 x 4096 at 1024 0.91); 1536 rows and more 1.04-1.50 from 2.5e7
+  //                 weights on, 4096 x 4096 0.97-1.10
+  //   no table      (too many groups for LDS) 129 rows and more, 14336 x 4096 1.14-2.08, 28672 x 8192 0.99-2.15
   const double weights = (double)w->K * w->N;
-  if (M > 128 && M * weights >= 1.25e10) return 1;
-  // 33 to 64 rows: the batch decode kernel on the copy, on wide matrices (us: 4096 x 28672 at M = 33 55 / 63, at 64
-  // 60 / 62; 3584 x 37888 at 48 65 / 77; 8192 x 57344 at 33 187 / 235, at 64 204 / 248; not 28672 x 8192 132 / 118)
-  return M >= Q4_REGROUP_MIN_ROWS && M <= 64 && w->N / 4 >= w->K && weights >= (M <= 48 ? 6.4e7 : 2.6e8);
+  if (M <= 128) return M >= Q4_REGROUP_MIN_ROWS && M <= 64 && w->N / 4 >= w->K && weights >= 2.6e8;
+  if (!gemm_act_order_table(w)) return weights >= 5e7;
+  if (w->N / 2 >= w->K && weights >= (M >= 320 ? 5e7 : (M <= 192 ? 8.5e7 : 1.3e8))) return 1;
+  return (M >= 320 && M * weights >= 6e10) || (M >= 1536 && weights >= 2.4e7);
 }
 
-int q4_linear_regroup(const q4_weight* w, const int32_t* perm, const void* x, const void* bias, void* y, int M,
-                      int dtype, int act, void* workspace, size_t workspace_bytes, void* stream) {
+int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
+                      void* workspace, size_t workspace_bytes, void* stream) {
   int rc = validate_weight(w, "q4_linear_regroup");
+  if (rc == Q4_OK) rc = validate_dtype(dtype, "q4_linear_regroup");
   if (rc != Q4_OK) return rc;
-  if (w->g_idx == nullptr || perm == nullptr || M < 0) {
-    set_error("q4_linear_regroup: bad M=%d, null perm, or a weight that is not act-order", M);
+  if (w->g_idx == nullptr || M < 0 || act < -1 || act > Q4_ACT_GELU) {
+    set_error("q4_linear_regroup: bad M=%d or act=%d, or a weight that is not act-order", M, act);
     return Q4_ERR_INVALID_ARGUMENT;
   }
   if (M == 0 || w->N == 0) return Q4_OK;
-  if ((long)w->num_groups * w->groupsize != w->K || !regroup_supported(w->K, w->N)) {
-    set_error("q4_linear_regroup: no kernel for K=%d N=%d with %d groups of %d rows", w->K, w->N, w->num_groups,
+  if (y == nullptr || x == nullptr) {
+    set_error("q4_linear_regroup: null x or y");
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
+  if ((((uintptr_t)x | (uintptr_t)y) & 15u) != 0 || ((uintptr_t)bias & 1u) != 0) {
+    set_error("q4_linear_regroup: x and y must be 16-byte aligned (bias: 2-byte)");
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
+  const q4_weight plain = in_group_order(w, w->qweight);
+  int fused = 1;
+  if (act >= 0) rc = q4_linear_gate_up_plan(&plain, M, dtype, &fused);
+  if (rc != Q4_OK) return rc;
+  if (!fused || !regroup_runs(w, M, dtype)) {
+    set_error("q4_linear_regroup: no kernel for M=%d K=%d N=%d with %d groups of %d rows", M, w->K, w->N, w->num_groups,
               w->groupsize);
     return Q4_ERR_UNSUPPORTED;
   }
-  const size_t offset = regroup_offset(M, w->K, w->N);
-  const size_t need = offset + (size_t)w->K * w->N / 2;
-  if (workspace == nullptr || ((uintptr_t)workspace & 15u) != 0 || workspace_bytes < need) {
+  const RegroupLayout l = regroup_layout(w, M, act >= 0);
+  if (workspace == nullptr || ((uintptr_t)workspace & 15u) != 0 || workspace_bytes < l.bytes) {
     set_error("q4_linear_regroup: 16-byte aligned workspace of %zu bytes needed (q4_linear_regroup_plan), %zu given",
-              need, workspace_bytes);
+              l.bytes, workspace_bytes);
     return Q4_ERR_WORKSPACE;
   }
-  uint32_t* qweight = (uint32_t*)((char*)workspace + offset);
-  const q4_weight seq = in_group_order(w, qweight);
-  rc = launch_regroup(w->qweight, perm, qweight, w->K, w->N, (hipStream_t)stream);
+  char* base = (char*)workspace;
+  int32_t* any_uneven = (int32_t*)(base + l.any_uneven);
+  int32_t* uneven = (int32_t*)(base + l.uneven);
+  int32_t* perm = (int32_t*)(base + l.perm);
+  uint32_t* copy = (uint32_t*)(base + l.copy);
+  hipStream_t s = (hipStream_t)stream;
+  rc = launch_group_order(w->g_idx, perm, uneven, w->K, w->num_groups, w->groupsize, s);
+  if (rc == Q4_OK) rc = launch_regroup(w->qweight, perm, uneven, w->num_groups, any_uneven, copy, w->K, w->N, s);
   if (rc != Q4_OK) return rc;
-  if (act >= 0) return q4_linear_gate_up_perm(&seq, perm, x, bias, y, M, dtype, act, workspace, offset, stream);
-  return q4_linear_perm(&seq, perm, x, bias, y, M, dtype, workspace, offset, Q4_PATH_AUTO, stream);
+  const q4_weight seq = in_group_order(w, copy);
+  if (act >= 0) rc = q4_linear_gate_up_perm(&seq, perm, x, bias, y, M, dtype, act, workspace, l.any_uneven, stream);
+  else rc = q4_linear_perm(&seq, perm, x, bias, y, M, dtype, workspace, l.any_uneven, Q4_PATH_AUTO, stream);
+  if (rc != Q4_OK) return rc;
+  // Groups of other sizes than groupsize (only the device knows): the kernels that look every row's group up write y
+  // again.  Otherwise these launches end at the flag.
+  void* sums = act >= 0 ? (void*)copy : y;
+  if (gemm_awq_supported(w, M, dtype))
+    rc = launch_gemm_awq(w, x, bias, sums, M, dtype, workspace, l.any_uneven, s, nullptr, any_uneven);
+  else
+    rc = launch_generic(w, x, bias, sums, M, dtype, s, any_uneven);
+  if (rc == Q4_OK && act >= 0) rc = launch_act_mul(sums, y, M, w->N / 2, dtype, act, s, any_uneven);
+  return rc;
 }
 
 int q4_linear_gate_up(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,

@@ -208,8 +208,9 @@ __device__ __forceinline__ int moe_enter(Problem& p, const MoeView& mv, int e) {
 namespace q4host {
 void set_error(const char* fmt, ...);
 int launch_dequant(const q4_weight* w, void* w_out, int dtype, hipStream_t stream);
+// (only_if, here and below: device flag or nullptr; the launch does nothing while the flag is 0)
 int launch_generic(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
-                   hipStream_t stream);
+                   hipStream_t stream, const int32_t* only_if = nullptr);
 struct GemvConfig {
   int wcol;    // waves across columns in a workgroup (one column tile each)
   int wk;      // waves across K in a workgroup
@@ -243,13 +244,17 @@ bool batch_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan
 int launch_batch(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act,
                  void* workspace, size_t workspace_bytes, const BatchPlan& plan, hipStream_t stream);
 bool gemv_gate_up_supported(const q4_weight* w, int M, int dtype);
-int launch_act_mul(const void* gate_up, void* y, int M, int inter, int dtype, int act, hipStream_t stream);
+int launch_act_mul(const void* gate_up, void* y, int M, int inter, int dtype, int act, hipStream_t stream,
+                   const int32_t* only_if = nullptr);
 bool gemm_gate_up_supported(const q4_weight* w, int M, int dtype);
 int launch_gemm_gate_up(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
                         hipStream_t stream);
 int launch_make_sequential(const uint32_t* qweight, const int32_t* perm, uint32_t* out, int K, int N, hipStream_t stream);
 bool regroup_supported(int K, int N);
-int launch_regroup(const uint32_t* qweight, const int32_t* perm, uint32_t* out, int K, int N, hipStream_t stream);
+int launch_group_order(const int32_t* g_idx, int32_t* perm, int32_t* uneven, int K, int num_groups, int groupsize,
+                       hipStream_t stream);
+int launch_regroup(const uint32_t* qweight, const int32_t* perm, const int32_t* uneven, int num_groups, int32_t* any_uneven,
+                   uint32_t* out, int K, int N, hipStream_t stream);
 int launch_gather_columns(const void* x, const int32_t* perm, void* out, int M, int K, hipStream_t stream);
 int launch_gptq_solve_block(float* W, const float* U, float* Q, float* Err, float* loss, float* scale, float* zero,
                             int rows, int K, int i1, int count, int groupsize, int G, int sym, hipStream_t stream);
@@ -268,7 +273,8 @@ struct MoeLaunch {
 };
 // moe != nullptr: grouped launch, M = moe->tokens, y and the partial tiles have moe->pairs rows
 int launch_gemm_awq(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
-                    void* workspace, size_t workspace_bytes, hipStream_t stream, const MoeLaunch* moe = nullptr);
+                    void* workspace, size_t workspace_bytes, hipStream_t stream, const MoeLaunch* moe = nullptr,
+                    const int32_t* only_if = nullptr);
 size_t gemm_awq_moe_workspace_bytes(const q4_weight* w, const MoeLaunch* moe);
 // AWQ layout, dense launches: the kernel that unpacks the checkpoint words in registers
 bool gemm_awq_direct_supported(const q4_weight* w, int M, int dtype);
@@ -299,5 +305,5 @@ int gemm_pick_splits(long tiles, int KT, int M, int N, double us_alone, double u
 bool gemm_act_order_table(const q4_weight* w);  // act-order GEMM reads its parameters from LDS
 int gemm_awq_splits(int M, int K, int N, bool one_per_cu, bool tall = false);
 void launch_gemm_reduce(const float* partials, const void* bias, void* y, int M, int N, int splits, int dtype,
-                        hipStream_t stream);
+                        hipStream_t stream, const int32_t* only_if = nullptr);
 }  // namespace q4host

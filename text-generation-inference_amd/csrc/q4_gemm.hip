@@ -170,16 +170,16 @@ int gemm_pick_splits(long tiles, int KT, int M, int N, double us_alone, double u
 }
 
 void launch_gemm_reduce(const float* partials, const void* bias, void* y, int M, int N, int splits, int dtype,
-                        hipStream_t stream) {
+                        hipStream_t stream, const int32_t* only_if) {
   const long quads = (long)M * (N / 4);
   long blocks = (quads + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   if (dtype == Q4_DTYPE_F16)
     hipLaunchKernelGGL(q4::gemm_reduce_kernel<Q4_DTYPE_F16>, dim3((unsigned)blocks), dim3(256), 0, stream, partials,
-                       bias, (uint16_t*)y, M, N, splits);
+                       bias, (uint16_t*)y, M, N, splits, only_if);
   else
     hipLaunchKernelGGL(q4::gemm_reduce_kernel<Q4_DTYPE_BF16>, dim3((unsigned)blocks), dim3(256), 0, stream, partials,
-                       bias, (uint16_t*)y, M, N, splits);
+                       bias, (uint16_t*)y, M, N, splits, only_if);
 }
 
 // fp32 partial tiles of the split-K variants: splits x M x N floats (upper bound over the

@@ -47,6 +47,7 @@ struct AwqGemmParams {
   int partial_rows;  // rows of one split's slice of `partials` (M; grouped launches: all pairs)
   Problem p;
   MoeView moe;  // grouped launches only (MOE kernels): blockIdx.y is the expert
+  const int32_t* __restrict__ only_if;  // act-order, may be nullptr: the launch does nothing while *only_if is 0
 };
 
 struct AwqSplice {
@@ -80,6 +81,7 @@ constexpr int kActNarrowGroupBytes = kABN * 3;  // 128 fp16 scales, then 128 zer
 template <int DTYPE, int MODE, bool MOE = false, int BM = kABM>
 __global__ __launch_bounds__(MODE == kModeAwq ? 256 : 512, 2) void gemm_awq_kernel(AwqGemmParams gp) {
   constexpr bool ACT = MODE != kModeAwq;
+  if (ACT && !MOE && gp.only_if != nullptr && *gp.only_if == 0) return;
   static_assert(BM == kABM || (BM == 2 * kABM && ACT), "256-row tiles: act-order only");
   // AWQ: 4 waves, 2 x 2, a 64 x 64 block each.  Act-order: 8 waves, 4 x 2, a 32 x 64 block each: the
   // parameter table leaves room for one workgroup per CU, and a single wave per SIMD cannot hide
@@ -592,7 +594,7 @@ size_t gemm_awq_moe_workspace_bytes(const q4_weight* w, const MoeLaunch* moe) {
 }
 
 int launch_gemm_awq(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
-                    void* workspace, size_t workspace_bytes, hipStream_t stream, const MoeLaunch* moe) {
+                    void* workspace, size_t workspace_bytes, hipStream_t stream, const MoeLaunch* moe, const int32_t* only_if) {
   using namespace q4;
   // dense AWQ launches go to the kernel that unpacks the words in registers where it applies
   if (moe == nullptr && gemm_awq_direct_supported(w, M, dtype))
@@ -617,6 +619,7 @@ int launch_gemm_awq(const q4_weight* w, const void* x, const void* bias, void* y
   gp.partial_rows = out_rows;
   gp.partials = splits > 1 ? (float*)((char*)workspace + Q4_WORKSPACE_COUNTER_BYTES) : nullptr;
   gp.moe = moe != nullptr ? moe->view : MoeView{};
+  gp.only_if = only_if;
   const long total = (long)((M + bm - 1) / bm) * (w->N / kABN) * splits;
   const long experts = moe != nullptr ? moe->num_experts : 1;
   if (total > 0x7fffffffL || experts > 65535) {
@@ -659,7 +662,7 @@ int launch_gemm_awq(const q4_weight* w, const void* x, const void* bias, void* y
     if (dtype == Q4_DTYPE_F16) launch_mode(F16{}, std::false_type{});
     else launch_mode(BF16{}, std::false_type{});
   }
-  if (splits > 1) launch_gemm_reduce(gp.partials, bias, y, out_rows, w->N, splits, dtype, stream);
+  if (splits > 1) launch_gemm_reduce(gp.partials, bias, y, out_rows, w->N, splits, dtype, stream, only_if);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     set_error("q4_linear(gemm/awq): launch failed: %s", hipGetErrorString(err));

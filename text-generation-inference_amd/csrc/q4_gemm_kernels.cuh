@@ -572,10 +572,13 @@ __global__ __launch_bounds__(256 * KG, (KG == 2 ? 1 : BM == 64 ? 3 : BM == 128 ?
 }
 
 // y[m][n] = round(sum over splits of partials[s][m][n]) (+ bias), four columns per thread.
+// only_if, when given: nothing happens while *only_if is 0.
 template <int DTYPE>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ partials,
                                                           const void* __restrict__ bias, uint16_t* __restrict__ y,
-                                                          int M, int N, int splits) {
+                                                          int M, int N, int splits,
+                                                          const int32_t* __restrict__ only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   const long quads = (long)M * (N >> 2);
   const size_t stride = (size_t)M * N;
   for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += (long)gridDim.x * blockDim.x) {

@@ -10,7 +10,8 @@ namespace q4 {
 constexpr int kGenericRows = 4;
 
 template <int DTYPE, int LAYOUT>
-__global__ __launch_bounds__(256) void generic_kernel(Problem p) {
+__global__ __launch_bounds__(256) void generic_kernel(Problem p, const int32_t* __restrict__ only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   const int m0 = blockIdx.y * kGenericRows;
   if (n >= p.N) return;
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(256) void generic_kernel(Problem p) {
 namespace q4host {
 
 int launch_generic(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
-                   hipStream_t stream) {
+                   hipStream_t stream, const int32_t* only_if) {
   using namespace q4;
   if (M == 0 || w->N == 0) return Q4_OK;
   Problem p{w->qweight, w->qzeros, (const half_t*)w->scales, w->g_idx, x, bias, y,
@@ -81,11 +82,11 @@ int launch_generic(const q4_weight* w, const void* x, const void* bias, void* y,
   dim3 grid((w->N + 255) / 256, gy);
   const bool awq = w->layout == Q4_LAYOUT_AWQ;
   if (dtype == Q4_DTYPE_F16) {
-    if (awq) hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_F16, Q4_LAYOUT_AWQ>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_F16, Q4_LAYOUT_GPTQ>), grid, block, 0, stream, p);
+    if (awq) hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_F16, Q4_LAYOUT_AWQ>), grid, block, 0, stream, p, only_if);
+    else hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_F16, Q4_LAYOUT_GPTQ>), grid, block, 0, stream, p, only_if);
   } else {
-    if (awq) hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_BF16, Q4_LAYOUT_AWQ>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_BF16, Q4_LAYOUT_GPTQ>), grid, block, 0, stream, p);
+    if (awq) hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_BF16, Q4_LAYOUT_AWQ>), grid, block, 0, stream, p, only_if);
+    else hipLaunchKernelGGL((generic_kernel<Q4_DTYPE_BF16, Q4_LAYOUT_GPTQ>), grid, block, 0, stream, p, only_if);
   }
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {

@@ -25,18 +25,72 @@ __global__ __launch_bounds__(256) void make_sequential_kernel(const uint32_t* __
   out[(size_t)r * N + n] = word;
 }
 
+// The row order by group, found inside a forward call (q4_linear_regroup) from g_idx as it is in memory then.
+// Workgroup g scans all of g_idx (K entries from L2) and writes the rows of group g, ascending, to perm[g
+// groupsize ..]; uneven[g] says whether they were not exactly `groupsize`.  perm is valid whatever g_idx holds:
+// rows beyond a group's share are left out, missing ones become 0.
+__global__ __launch_bounds__(512) void group_order_kernel(const int32_t* __restrict__ g_idx, int32_t* __restrict__ perm,
+                                                          int32_t* __restrict__ uneven, int K, int groupsize) {
+  __shared__ int sums[8];
+  const int g = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int per = ((K >> 2) + 511) / 512 * 4;  // entries of a thread, contiguous
+  const int k0 = min(tid * per, K), k1 = min(k0 + per, K);
+  int count = 0;
+#pragma unroll 4
+  for (int k = k0; k < k1; k += 4) {
+    const uint4_t v = *(const uint4_t*)(g_idx + k);
+    count += ((int)v.x == g) + ((int)v.y == g) + ((int)v.z == g) + ((int)v.w == g);
+  }
+  int scan = count;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int below = __shfl_up(scan, d);
+    if (lane >= d) scan += below;
+  }
+  if (lane == 63) sums[tid >> 6] = scan;
+  __syncthreads();
+  int rank = scan - count, total = 0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    if (w < (tid >> 6)) rank += sums[w];
+    total += sums[w];
+  }
+  int32_t* dst = perm + (size_t)g * groupsize;
+  for (int k = k0; count > 0 && k < k1; k += 4) {
+    const uint4_t v = *(const uint4_t*)(g_idx + k);
+    const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if ((int)e[i] != g) continue;
+      if (rank < groupsize) dst[rank] = k + i;
+      ++rank;
+    }
+  }
+  for (int r = total + tid; r < groupsize; r += 512) dst[r] = 0;
+  if (tid == 0) uneven[g] = total != groupsize ? 1 : 0;
+}
+
 // The same for a whole matrix inside a forward call (q4_linear_regroup).  A source word's nibbles go to
 // eight different output words: one thread per word in output order reads everything eight times
 // (8192 x 10240: 33 us whether the last-level cache or the L2 serves it, 2.5 TB/s in and out).  Here a
 // workgroup holds a panel of C columns over all of K in LDS (K C / 2 bytes: 32 columns up to K = 9600, 16
 // or 8 beyond), so memory sees every word once in and once out, and gathers from there: a lane owns four
 // adjacent columns of an output row, eight 128-bit LDS reads and two operations per nibble.
+// Workgroup 0 also gathers what group_order_kernel found: *any_uneven is 1 if a group has not its share of rows.
 template <int C>
 __global__ __launch_bounds__(1024) void regroup_kernel(const uint32_t* __restrict__ qweight, const int32_t* __restrict__ perm,
-                                                       uint32_t* __restrict__ out, int K, int N) {
+                                                       const int32_t* __restrict__ uneven, int num_groups,
+                                                       int32_t* __restrict__ any_uneven, uint32_t* __restrict__ out, int K,
+                                                       int N) {
   extern __shared__ __align__(16) uint4_t panel[];  // [K / 8][C / 4]
   constexpr int UPR = C / 4;  // 16-byte units per row
   const int rows = K >> 3, units = rows * UPR;
+  if (blockIdx.x == 0) {
+    int bad = 0;
+    for (int g = threadIdx.x; g < num_groups; g += 1024) bad |= uneven[g];
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) *any_uneven = bad != 0 ? 1 : 0;
+  }
   // Panels narrower than a cache line: the ones that share lines run on one XCD (workgroup ids go to the 8
   // XCDs in turn), whose L2 then fetches a line once and collects its parts on the way out.
   constexpr int SHARE = 32 / C;
@@ -231,13 +285,25 @@ static int regroup_panel(int K, int N) {
 }
 bool regroup_supported(int K, int N) { return K % 8 == 0 && regroup_panel(K, N) != 0; }
 
-int launch_regroup(const uint32_t* qweight, const int32_t* perm, uint32_t* out, int K, int N, hipStream_t stream) {
+int launch_group_order(const int32_t* g_idx, int32_t* perm, int32_t* uneven, int K, int num_groups, int groupsize,
+                       hipStream_t stream) {
+  hipLaunchKernelGGL(q4::group_order_kernel, dim3((unsigned)num_groups), dim3(512), 0, stream, g_idx, perm, uneven, K, groupsize);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) {
+    set_error("q4_linear_regroup: launch failed: %s", hipGetErrorString(err));
+    return Q4_ERR_LAUNCH;
+  }
+  return Q4_OK;
+}
+
+int launch_regroup(const uint32_t* qweight, const int32_t* perm, const int32_t* uneven, int num_groups, int32_t* any_uneven,
+                   uint32_t* out, int K, int N, hipStream_t stream) {
   const int c = regroup_panel(K, N);
   const size_t smem = (size_t)K * c / 2;
   const dim3 grid((unsigned)(N / (c > 0 ? c : 1)));
   auto launch = [&](auto k) {
     if (smem > 64 * 1024) (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    hipLaunchKernelGGL(k, grid, dim3(1024), smem, stream, qweight, perm, out, K, N);
+    hipLaunchKernelGGL(k, grid, dim3(1024), smem, stream, qweight, perm, uneven, num_groups, any_uneven, out, K, N);
   };
   if (c == 32) launch(q4::regroup_kernel<32>);
   else if (c == 16) launch(q4::regroup_kernel<16>);

@@ -75,13 +75,6 @@ class PackedWeight:
     # Rows in group order (make_sequential): packed row i holds checkpoint row perm[i] and the
     # kernels take the activation columns in that order; None for checkpoint order.
     perm: Optional[torch.Tensor] = None
-    # Act-order weight in checkpoint order whose groups all hold `groupsize` rows: the row order by
-    # group (the stable argsort of g_idx), with which calls of many rows regroup on the way
-    # (q4_linear_regroup).  Found by prepare(); None where it does not apply.  It holds for the g_idx it was
-    # read from: entries written in place afterwards (load_state_dict) leave it behind, and until the next
-    # prepare() such a weight is read through g_idx like any other.
-    order: Optional[torch.Tensor] = None
-    _order_version: int = field(default=-1, repr=False, compare=False)
     # (M, dtype code) -> (kernel path, workspace bytes): a pure function of the weight's geometry,
     # asked of the library once and kept (one library call per forward afterwards)
     _plans: dict = field(default_factory=dict, repr=False, compare=False)
@@ -91,14 +84,10 @@ class PackedWeight:
         import copy
 
         # the cached ctypes struct holds device addresses: a copy gets its own, on first use
-        new = PackedWeight(
+        return PackedWeight(
             copy.deepcopy(self.qweight, memo), copy.deepcopy(self.qzeros, memo), copy.deepcopy(self.scales, memo),
             copy.deepcopy(self.g_idx, memo), self.K, self.N, self.groupsize, self.num_groups, self.layout,
-            copy.deepcopy(self.perm, memo), _plans=dict(self._plans))
-        # (under inference_mode the copy is an inference tensor, which counts no writes: no order for it)
-        if self.order is not None and not new.g_idx.is_inference() and self.g_idx._version == self._order_version:
-            new.order, new._order_version = copy.deepcopy(self.order, memo), new.g_idx._version
-        return new
+            copy.deepcopy(self.perm, memo), dict(self._plans), None)
 
     def struct(self) -> Q4Weight:
         if self._struct is None:
@@ -125,17 +114,9 @@ class PackedWeight:
             self._plans[key] = got
         return got
 
-    def find_order(self) -> None:
-        """Set `order` from the g_idx as it is now.  Inference tensors do not count their writes: none for them."""
-        if self.g_idx is None or self.g_idx.is_inference():
-            self.order = None
-        elif self.order is None or self.g_idx._version != self._order_version:
-            self._order_version = self.g_idx._version
-            self.order = _group_order(self)
-
     def regroup(self, M: int, dtype_code: int, gate_up: bool) -> int:
         """Workspace bytes of q4_linear_regroup where the library prefers it for M rows, else 0."""
-        if self.order is None or M < _lib.REGROUP_MIN_ROWS or self.g_idx._version != self._order_version:
+        if self.g_idx is None or M < _lib.REGROUP_MIN_ROWS:
             return 0
         key = ("regroup", M, dtype_code, gate_up)
         got = self._plans.get(key)
@@ -156,7 +137,6 @@ class PackedWeight:
         graph)."""
         if not self.qweight.is_cuda:
             return
-        self.find_order()
         if rows is None:
             rows = tuple(M for M in _PLAN_ROWS if M <= max(max_rows, 16))
             if max_rows > 16 and max_rows not in rows:
@@ -230,19 +210,6 @@ def make_packed(qweight, qzeros, scales, g_idx, groupsize: int, layout: int) -> 
     )
 
 
-def _group_order(w: PackedWeight) -> Optional[torch.Tensor]:
-    """The stable argsort of an act-order weight's g_idx (int32), or None unless every group holds
-    exactly `groupsize` rows (one device->host sync for the check)."""
-    K = w.K
-    if w.g_idx is None or w.perm is not None or K == 0 or K % 8 or w.num_groups * w.groupsize != K:
-        return None
-    groups, perm = torch.sort(w.g_idx, stable=True)
-    expect = torch.arange(K, device=groups.device, dtype=groups.dtype).div_(w.groupsize, rounding_mode="floor")
-    if not torch.equal(groups, expect):
-        return None
-    return perm.to(torch.int32)
-
-
 def make_sequential(w: PackedWeight) -> Optional[PackedWeight]:
     """Act-order weight with its rows put into group order, or None when that is not possible.
 
@@ -258,10 +225,14 @@ def make_sequential(w: PackedWeight) -> Optional[PackedWeight]:
     if w.g_idx is None or w.layout != LAYOUT_GPTQ or w.perm is not None:
         return None
     _require_cuda(w.qweight, "qweight")
-    perm32 = _group_order(w)
-    if perm32 is None:
-        return None
     K = w.K
+    if K == 0 or K % 8 or w.num_groups * w.groupsize != K:
+        return None
+    groups, perm = torch.sort(w.g_idx, stable=True)
+    expect = torch.arange(K, device=groups.device, dtype=groups.dtype).div_(w.groupsize, rounding_mode="floor")
+    if not torch.equal(groups, expect):
+        return None
+    perm32 = perm.to(torch.int32)
     out = torch.empty_like(w.qweight)
     with torch.cuda.device(w.qweight.device):
         _lib.check(_lib.load().q4_gptq_make_sequential(
@@ -461,7 +432,7 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev) -> int:
     # decode: split-K partial sums, tickets, accumulation cells; prefill GEMM: split-K
     # partial tiles when the tile grid alone would leave CUs idle
     planned_path, need, tuned = w.plan(M, code)
-    regroup = w.order is not None and path == PATH_AUTO and gemv_config is None and w.regroup(M, code, False)
+    regroup = w.regroup(M, code, False) if path == PATH_AUTO and gemv_config is None else 0
     if path == PATH_AUTO and gemv_config is None:
         path = planned_path
         if tuned is not None and w.perm is None:
@@ -477,8 +448,7 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev) -> int:
         return lib.q4_gemv_tuned(st, x.data_ptr(), bias_ptr, y.data_ptr(), M, code, ws.data_ptr(), ws.numel(),
                                  wcol, wk, splits, words, stream)
     if regroup and ws.numel() >= regroup:
-        return lib.q4_linear_regroup(st, w.order.data_ptr(), x.data_ptr(), bias_ptr, y.data_ptr(), M, code, -1,
-                                     ws.data_ptr(), ws.numel(), stream)
+        return lib.q4_linear_regroup(st, x.data_ptr(), bias_ptr, y.data_ptr(), M, code, -1, ws.data_ptr(), ws.numel(), stream)
     if w.perm is not None:
         return lib.q4_linear_perm(st, w.perm.data_ptr(), x.data_ptr(), bias_ptr, y.data_ptr(), M, code,
                                   ws.data_ptr(), ws.numel(), path, stream)
@@ -668,7 +638,7 @@ def linear_gate_up(
             ws = _workspace_for_call(x.device, regroup, stream)
             if ws.numel() >= regroup:
                 _lib.check(_lib.load().q4_linear_regroup(
-                    ctypes.byref(w.struct()), w.order.data_ptr(), x.data_ptr(),
+                    ctypes.byref(w.struct()), x.data_ptr(),
                     bias.contiguous().data_ptr() if bias is not None else None,
                     y.data_ptr(), M, _DTYPES[x.dtype], _lib.ACTIVATIONS[act], ws.data_ptr(), ws.numel(), stream))
                 return y
