@@ -155,19 +155,21 @@ int q4_linear_gate_up_perm(const q4_weight* w, const int32_t* perm, const void* 
                            int dtype, int act, void* workspace, size_t workspace_bytes, void* stream);
 /*
  * q4_linear (act = -1) or q4_linear_gate_up (act = Q4_ACT_*) for an act-order weight (g_idx set) as it is in
- * the checkpoint, by putting its rows into group order on the way: the call sorts g_idx, qweight goes through that
- * order into the workspace, then the call is q4_linear_perm / q4_linear_gate_up_perm on that copy.  One more pass over
+ * the checkpoint, by putting its rows into group order on the way: the call sorts g_idx, copies qweight and x in that
+ * order into the scratch, then runs q4_linear / q4_linear_gate_up on the copies.  One more pass over
  * the weight buys kernels that look no group up, which pays with many rows.  g_idx is read when the call runs, so a
  * captured call follows what is written into it between replays.  Where its groups do not all hold `groupsize` rows,
  * which only the device can tell, the kernels that read through g_idx compute y instead.
- * q4_linear_regroup_plan: 1 where this measured faster than the kernels that read through g_idx, else 0,
- * and the workspace bytes the call needs (0: it cannot run); the workspace's head is the zero-initialised
- * area of q4_workspace_bytes.  Never preferred for fewer than Q4_REGROUP_MIN_ROWS rows.
+ * q4_linear_regroup_plan: 1 where this measured faster than the kernels that read through g_idx, else 0, and the bytes
+ * the call needs (scratch 0: it cannot run).  The workspace is that of q4_linear; the scratch holds nothing between
+ * calls and needs no initialisation (K * N / 2 + 2 * M * K bytes and a little more), so that a caller need not keep it.
+ * Never preferred for fewer than Q4_REGROUP_MIN_ROWS rows.
  */
 #define Q4_REGROUP_MIN_ROWS 33
-int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, size_t* workspace_bytes);
+int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, size_t* workspace_bytes,
+                           size_t* scratch_bytes);
 int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
-                      void* workspace, size_t workspace_bytes, void* stream);
+                      void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, void* stream);
 /*
  * One block of the GPTQ solver's column loop (GPTQ.fasterquant,
  * server/text_generation_server/layers/gptq/quantize.py:294-331; the quantizer's range rule,

@@ -28,14 +28,15 @@ def build(pkg, oracle, gpu, K, N, gs, seed):
 def call(pkg, pk, x, act=-1):
     lib, L = pkg._lib.load(), pkg._lib
     M, code = x.shape[0], pkg.ops._DTYPES[x.dtype]
-    need = ctypes.c_size_t(0)
-    L.check(lib.q4_linear_regroup_plan(ctypes.byref(pk.struct()), M, code, int(act >= 0), ctypes.byref(need)))
-    assert need.value > 0
+    need, room = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    L.check(lib.q4_linear_regroup_plan(ctypes.byref(pk.struct()), M, code, int(act >= 0), ctypes.byref(need), ctypes.byref(room)))
+    assert room.value > 0
     ws = torch.zeros(need.value, dtype=torch.uint8, device=x.device)
+    scratch = torch.full((room.value,), 0xA5, dtype=torch.uint8, device=x.device)
     y = torch.empty((M, pk.N // (2 if act >= 0 else 1)), dtype=x.dtype, device=x.device)
-    args = [ctypes.byref(pk.struct()), x.data_ptr(), None, y.data_ptr(), M, code, act, ws.data_ptr()]
-    assert lib.q4_linear_regroup(*args, need.value - 1, pkg.ops._stream_handle(x.device)) == L.ERR_WORKSPACE
-    L.check(lib.q4_linear_regroup(*args, need.value, pkg.ops._stream_handle(x.device)))
+    args = [ctypes.byref(pk.struct()), x.data_ptr(), None, y.data_ptr(), M, code, act, ws.data_ptr(), need.value, scratch.data_ptr()]
+    assert lib.q4_linear_regroup(*args, room.value - 1, pkg.ops._stream_handle(x.device)) == L.ERR_WORKSPACE
+    L.check(lib.q4_linear_regroup(*args, room.value, pkg.ops._stream_handle(x.device)))
     return y
 
 
@@ -69,7 +70,7 @@ def test_layers_regroup_from_the_librarys_row_count_on(pkg, oracle, gpu, K, N, M
     kernels that read through g_idx (the same weights, sums in another order)."""
     _, pk = build(pkg, oracle, gpu, K, N, 128, seed=N)
     x = torch.randn((M, K), device=gpu, dtype=torch.float16) * 0.1
-    assert (pk.regroup(M, 0, False) > 0) == regroups
+    assert (pk.regroup(M, 0, False)[1] > 0) == regroups
     plain = pkg.ops.linear(pk, x, path=2)
     for a, b in ((pkg.ops.linear(pk, x), plain), (pkg.ops.linear_gate_up(pk, x), pkg.ops.act_mul(plain))):
         assert ((a.float() - b.float()).norm() / b.float().norm()).item() <= 2e-3
@@ -103,7 +104,7 @@ def test_a_call_reads_g_idx_when_it_runs(pkg, gpu, M):
     """Entries written after the layer was prepared, counted by torch (copy_) or not (.data), are the ones used."""
     pk = big(pkg, gpu, M)
     pk.prepare()
-    assert pk.regroup(M, 0, False) > 0 and pk.regroup(M, 0, True) > 0
+    assert pk.regroup(M, 0, False)[1] > 0 and pk.regroup(M, 0, True)[1] > 0
     x = torch.randn((M, pk.K), device=gpu, dtype=torch.float16) * 0.1
     against_g_idx(pkg, pk, x)
     pk.g_idx.data.copy_(pk.g_idx[torch.randperm(pk.K, device=gpu)])
@@ -154,3 +155,39 @@ def test_uneven_groups_without_a_prefill_kernel(pkg, oracle, gpu, K, N, gs, M):
     pk.g_idx.copy_(pk.g_idx.clamp(max=pk.num_groups // 2 - 1) if pk.num_groups > 1 else pk.g_idx - 1)
     want = pkg.ops.linear(pk, x, path=2 if N % 128 == 0 else 3)
     assert torch.equal(call(pkg, pk, x), want)
+
+
+def test_the_copy_lasts_for_one_call(pkg, gpu, monkeypatch):
+    """Preparing a layer and calling it leaves no copy of the weight behind; without memory for one, or with `out` under
+    capture, where nothing may be allocated, the call goes through g_idx."""
+    pk = big(pkg, gpu, 1)
+    x = torch.randn((200, pk.K), device=gpu, dtype=torch.float16) * 0.1
+    pkg.ops.linear(pk, x[:1]), pkg.ops.linear(pk, x, path=2)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    pk.prepare(rows=(1, 48, 200))
+    got = pkg.ops.linear(pk, x), pkg.ops.linear_gate_up(pk, x)
+    kept = sum(t.numel() * t.element_size() for t in got)
+    assert torch.cuda.memory_allocated() - before - kept < pk.K * pk.N // 2
+    want = pkg.ops.linear(pk, x, path=2)
+    out = torch.empty_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = torch.cuda.memory_allocated()
+        pkg.ops.linear(pk, x, out=out)
+        assert torch.cuda.memory_allocated() == held
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    empty = torch.empty
+
+    def full(*args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8:
+            raise torch.cuda.OutOfMemoryError("no memory for the copy")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert torch.equal(pkg.ops.linear(pk, x), want) and torch.equal(pkg.ops.linear_gate_up(pk, x), pkg.ops.act_mul(want))

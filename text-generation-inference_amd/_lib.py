@@ -97,9 +97,9 @@ SIGNATURES = {
     "q4_workspace_bytes_perm": (c_size_t, [c_int, c_int, c_int]),
     "q4_linear_gate_up_perm": (c_int, [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                         c_void_p, c_size_t, c_void_p]),
-    "q4_linear_regroup_plan": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int, POINTER(c_size_t)]),
+    "q4_linear_regroup_plan": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int, POINTER(c_size_t), POINTER(c_size_t)]),
     "q4_linear_regroup": (c_int, [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t,
-                                  c_void_p]),
+                                  c_void_p, c_size_t, c_void_p]),
     "q4_gptq_solve_block": (c_int, [c_void_p] * 7 + [c_int] * 7 + [c_void_p]),
     "q4_moe_gather_columns": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "q4_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),

@@ -461,32 +461,34 @@ static bool regroup_runs(const q4_weight* w, int M, int dtype) {
   return gemm_awq_supported(w, M, dtype) ? (long)(M + 127) / 128 * (w->N / 128) * 16 <= 0x7fffffffL : M <= 4 * 65535;
 }
 
-// Workspace of q4_linear_regroup behind that of the calls on the copy: the flag, one word per group, the row order,
-// and the copy, whose room also takes the [M, N] sums of a gated call through g_idx.
+// Scratch of q4_linear_regroup: the flag, one word per group, the row order, x in that order, and the copy, whose
+// room also takes the [M, N] sums of a gated call through g_idx.
 struct RegroupLayout {
-  size_t any_uneven, uneven, perm, copy, bytes;
+  size_t any_uneven, uneven, perm, x_seq, copy, bytes;
 };
 static RegroupLayout regroup_layout(const q4_weight* w, int M, bool gate_up) {
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   RegroupLayout l;
-  l.any_uneven = up(q4_workspace_bytes_perm(M, w->K, w->N));
-  l.uneven = l.any_uneven + 256;
+  l.any_uneven = 0;
+  l.uneven = 256;
   l.perm = up(l.uneven + (size_t)w->num_groups * 4);
-  l.copy = up(l.perm + (size_t)w->K * 4);
+  l.x_seq = up(l.perm + (size_t)w->K * 4);
+  l.copy = up(l.x_seq + (size_t)M * w->K * 2);
   const size_t copy = (size_t)w->K * w->N / 2, sums = gate_up ? (size_t)M * w->N * 2 : 0;
   l.bytes = l.copy + (copy > sums ? copy : sums);
   return l;
 }
 
-int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, size_t* workspace_bytes) {
+int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, size_t* workspace_bytes,
+                           size_t* scratch_bytes) {
   int rc = validate_weight(w, "q4_linear_regroup_plan");
   if (rc == Q4_OK) rc = validate_dtype(dtype, "q4_linear_regroup_plan");
   if (rc != Q4_OK) return rc;
-  if (M < 0 || workspace_bytes == nullptr) {
+  if (M < 0 || workspace_bytes == nullptr || scratch_bytes == nullptr) {
     set_error("q4_linear_regroup_plan: negative M=%d or null output pointer", M);
     return Q4_ERR_INVALID_ARGUMENT;
   }
-  *workspace_bytes = 0;
+  *workspace_bytes = *scratch_bytes = 0;
   if (M == 0 || w->N == 0 || !regroup_runs(w, M, dtype)) return 0;
   const q4_weight seq = in_group_order(w, w->qweight);
   if (gate_up) {
@@ -495,7 +497,9 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
     if (rc != Q4_OK) return rc;
     if (!fused) return 0;
   }
-  *workspace_bytes = regroup_layout(w, M, gate_up != 0).bytes;
+  const size_t own = q4_workspace_bytes_for(w, M), copy = q4_workspace_bytes_for(&seq, M);
+  *workspace_bytes = own > copy ? own : copy;
+  *scratch_bytes = regroup_layout(w, M, gate_up != 0).bytes;
   // (uneven groups then cost what they always did)
   if (q4_select_path(w, M, dtype) != Q4_PATH_GEMM) return 0;
   // Sorting g_idx (3 us), the pass over the weights (8192 x 57344 131 us, 4096 x 4096 7), the gather of x and the
@@ -518,7 +522,7 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
 }
 
 int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
-                      void* workspace, size_t workspace_bytes, void* stream) {
+                      void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, void* stream) {
   int rc = validate_weight(w, "q4_linear_regroup");
   if (rc == Q4_OK) rc = validate_dtype(dtype, "q4_linear_regroup");
   if (rc != Q4_OK) return rc;
@@ -531,8 +535,8 @@ int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void*
     set_error("q4_linear_regroup: null x or y");
     return Q4_ERR_INVALID_ARGUMENT;
   }
-  if ((((uintptr_t)x | (uintptr_t)y) & 15u) != 0 || ((uintptr_t)bias & 1u) != 0) {
-    set_error("q4_linear_regroup: x and y must be 16-byte aligned (bias: 2-byte)");
+  if ((((uintptr_t)x | (uintptr_t)y | (uintptr_t)workspace) & 15u) != 0 || ((uintptr_t)bias & 1u) != 0) {
+    set_error("q4_linear_regroup: x, y and the workspace must be 16-byte aligned (bias: 2-byte)");
     return Q4_ERR_INVALID_ARGUMENT;
   }
   const q4_weight plain = in_group_order(w, w->qweight);
@@ -545,29 +549,31 @@ int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void*
     return Q4_ERR_UNSUPPORTED;
   }
   const RegroupLayout l = regroup_layout(w, M, act >= 0);
-  if (workspace == nullptr || ((uintptr_t)workspace & 15u) != 0 || workspace_bytes < l.bytes) {
-    set_error("q4_linear_regroup: 16-byte aligned workspace of %zu bytes needed (q4_linear_regroup_plan), %zu given",
-              l.bytes, workspace_bytes);
+  if (scratch == nullptr || ((uintptr_t)scratch & 15u) != 0 || scratch_bytes < l.bytes) {
+    set_error("q4_linear_regroup: 16-byte aligned scratch of %zu bytes needed (q4_linear_regroup_plan), %zu given", l.bytes,
+              scratch_bytes);
     return Q4_ERR_WORKSPACE;
   }
-  char* base = (char*)workspace;
+  char* base = (char*)scratch;
   int32_t* any_uneven = (int32_t*)(base + l.any_uneven);
   int32_t* uneven = (int32_t*)(base + l.uneven);
   int32_t* perm = (int32_t*)(base + l.perm);
+  void* x_seq = base + l.x_seq;
   uint32_t* copy = (uint32_t*)(base + l.copy);
   hipStream_t s = (hipStream_t)stream;
   rc = launch_group_order(w->g_idx, perm, uneven, w->K, w->num_groups, w->groupsize, s);
   if (rc == Q4_OK) rc = launch_regroup(w->qweight, perm, uneven, w->num_groups, any_uneven, copy, w->K, w->N, s);
+  if (rc == Q4_OK) rc = launch_gather_columns(x, perm, x_seq, M, w->K, s);
   if (rc != Q4_OK) return rc;
   const q4_weight seq = in_group_order(w, copy);
-  if (act >= 0) rc = q4_linear_gate_up_perm(&seq, perm, x, bias, y, M, dtype, act, workspace, l.any_uneven, stream);
-  else rc = q4_linear_perm(&seq, perm, x, bias, y, M, dtype, workspace, l.any_uneven, Q4_PATH_AUTO, stream);
+  if (act >= 0) rc = q4_linear_gate_up(&seq, x_seq, bias, y, M, dtype, act, workspace, workspace_bytes, stream);
+  else rc = q4_linear_ex(&seq, x_seq, bias, y, M, dtype, workspace, workspace_bytes, Q4_PATH_AUTO, stream);
   if (rc != Q4_OK) return rc;
   // Groups of other sizes than groupsize (only the device knows): the kernels that look every row's group up write y
   // again.  Otherwise these launches end at the flag.
   void* sums = act >= 0 ? (void*)copy : y;
   if (gemm_awq_supported(w, M, dtype))
-    rc = launch_gemm_awq(w, x, bias, sums, M, dtype, workspace, l.any_uneven, s, nullptr, any_uneven);
+    rc = launch_gemm_awq(w, x, bias, sums, M, dtype, workspace, workspace_bytes, s, nullptr, any_uneven);
   else
     rc = launch_generic(w, x, bias, sums, M, dtype, s, any_uneven);
   if (rc == Q4_OK && act >= 0) rc = launch_act_mul(sums, y, M, w->N / 2, dtype, act, s, any_uneven);

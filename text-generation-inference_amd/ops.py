@@ -109,22 +109,23 @@ class PackedWeight:
                 # weight in group order: x is gathered into the tail of the workspace (all but the
                 # shortest decode calls, which gather inside the kernel)
                 nbytes = max(nbytes, int(lib.q4_workspace_bytes_perm(M, self.K, self.N)))
-            nbytes = max(nbytes, self.regroup(M, dtype_code, False))  # (the gated call takes as much or nothing)
+            nbytes = max(nbytes, self.regroup(M, dtype_code, False)[0])
             got = (int(path.value), nbytes, None)
             self._plans[key] = got
         return got
 
-    def regroup(self, M: int, dtype_code: int, gate_up: bool) -> int:
-        """Workspace bytes of q4_linear_regroup where the library prefers it for M rows, else 0."""
+    def regroup(self, M: int, dtype_code: int, gate_up: bool) -> tuple:
+        """(workspace, scratch) bytes of q4_linear_regroup where the library prefers it for M rows, else (0, 0)."""
         if self.g_idx is None or M < _lib.REGROUP_MIN_ROWS:
-            return 0
+            return 0, 0
         key = ("regroup", M, dtype_code, gate_up)
         got = self._plans.get(key)
         if got is None:
-            need = ctypes.c_size_t(0)
-            rc = _lib.load().q4_linear_regroup_plan(ctypes.byref(self.struct()), M, dtype_code, int(gate_up), ctypes.byref(need))
+            need, scratch = ctypes.c_size_t(0), ctypes.c_size_t(0)
+            rc = _lib.load().q4_linear_regroup_plan(ctypes.byref(self.struct()), M, dtype_code, int(gate_up),
+                                                    ctypes.byref(need), ctypes.byref(scratch))
             _lib.check(rc)
-            got = int(need.value) if rc == 1 else 0
+            got = (int(need.value), int(scratch.value)) if rc == 1 else (0, 0)
             self._plans[key] = got
         return got
 
@@ -349,6 +350,18 @@ def _workspace_for_call(device: torch.device, need: int, stream: int) -> torch.T
     return reserve_workspace(device, need, stream)
 
 
+def _regroup_scratch(w: PackedWeight, nbytes: int, out_given: bool) -> Optional[torch.Tensor]:
+    """Memory of one regrouped call: a copy of the packed weight and of x, freed (on the call's stream) when it returns
+    and nothing to keep between calls.  None where there is none: the kernels that read through g_idx need no copy.  Under
+    capture it comes from the graph's pool; a call with `out` allocates nothing there, as `linear` promises."""
+    if out_given and torch.cuda.is_current_stream_capturing():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=w.qweight.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def workspace_bytes(M: int, K: int, N: int) -> int:
     return int(_lib.load().q4_workspace_bytes(int(M), int(K), int(N)))
 
@@ -410,10 +423,10 @@ def linear(
         return y
     fused_bias = bias is not None and bias.dtype == x.dtype and bias.is_cuda and bias.numel() == w.N
     if dev.index is None or _current_device() == dev.index:
-        rc = _launch_linear(w, x, bias.contiguous() if fused_bias else None, y, M, code, path, gemv_config, dev)
+        rc = _launch_linear(w, x, bias.contiguous() if fused_bias else None, y, M, code, path, gemv_config, dev, out is not None)
     else:
         with torch.cuda.device(dev):
-            rc = _launch_linear(w, x, bias.contiguous() if fused_bias else None, y, M, code, path, gemv_config, dev)
+            rc = _launch_linear(w, x, bias.contiguous() if fused_bias else None, y, M, code, path, gemv_config, dev, out is not None)
     if rc < 0:
         _lib.check(rc)
     if bias is not None and not fused_bias:
@@ -424,7 +437,7 @@ def linear(
     return y
 
 
-def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev) -> int:
+def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev, out_given) -> int:
     """The library call of `linear` on the current stream of `dev`, the current device."""
     lib = _lib.load()
     stream = _stream_handle(dev)
@@ -432,7 +445,7 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev) -> int:
     # decode: split-K partial sums, tickets, accumulation cells; prefill GEMM: split-K
     # partial tiles when the tile grid alone would leave CUs idle
     planned_path, need, tuned = w.plan(M, code)
-    regroup = w.regroup(M, code, False) if path == PATH_AUTO and gemv_config is None else 0
+    scratch = w.regroup(M, code, False)[1] if path == PATH_AUTO and gemv_config is None else 0
     if path == PATH_AUTO and gemv_config is None:
         path = planned_path
         if tuned is not None and w.perm is None:
@@ -447,8 +460,9 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev) -> int:
             ws = _workspace_for_call(dev, need, stream)
         return lib.q4_gemv_tuned(st, x.data_ptr(), bias_ptr, y.data_ptr(), M, code, ws.data_ptr(), ws.numel(),
                                  wcol, wk, splits, words, stream)
-    if regroup and ws.numel() >= regroup:
-        return lib.q4_linear_regroup(st, x.data_ptr(), bias_ptr, y.data_ptr(), M, code, -1, ws.data_ptr(), ws.numel(), stream)
+    if scratch and (mem := _regroup_scratch(w, scratch, out_given)) is not None:
+        return lib.q4_linear_regroup(st, x.data_ptr(), bias_ptr, y.data_ptr(), M, code, -1, ws.data_ptr(), ws.numel(),
+                                     mem.data_ptr(), mem.numel(), stream)
     if w.perm is not None:
         return lib.q4_linear_perm(st, w.perm.data_ptr(), x.data_ptr(), bias_ptr, y.data_ptr(), M, code,
                                   ws.data_ptr(), ws.numel(), path, stream)
@@ -631,16 +645,17 @@ def linear_gate_up(
     if M == 0 or inter == 0:
         return y
     fusable_bias = bias is None or (bias.dtype == x.dtype and bias.is_cuda and bias.numel() == w.N)
-    regroup = w.regroup(M, _DTYPES[x.dtype], True) if fused is None and fusable_bias else 0
-    if regroup:
+    need, scratch = w.regroup(M, _DTYPES[x.dtype], True) if fused is None and fusable_bias else (0, 0)
+    if scratch:
         with _on_device(x.device):
-            stream = _stream_handle(x.device)
-            ws = _workspace_for_call(x.device, regroup, stream)
-            if ws.numel() >= regroup:
+            mem = _regroup_scratch(w, scratch, out is not None)
+            if mem is not None:
+                stream = _stream_handle(x.device)
+                ws = _workspace_for_call(x.device, need, stream)
                 _lib.check(_lib.load().q4_linear_regroup(
-                    ctypes.byref(w.struct()), x.data_ptr(),
-                    bias.contiguous().data_ptr() if bias is not None else None,
-                    y.data_ptr(), M, _DTYPES[x.dtype], _lib.ACTIVATIONS[act], ws.data_ptr(), ws.numel(), stream))
+                    ctypes.byref(w.struct()), x.data_ptr(), bias.contiguous().data_ptr() if bias is not None else None,
+                    y.data_ptr(), M, _DTYPES[x.dtype], _lib.ACTIVATIONS[act], ws.data_ptr(), ws.numel(), mem.data_ptr(),
+                    mem.numel(), stream))
                 return y
     if fused is None and not _gate_up_fused_preferred(w, M, _DTYPES[x.dtype]):
         fused = False  # no fused kernel here, or the two launches measured faster (the library's rule)
