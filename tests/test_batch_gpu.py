@@ -102,7 +102,18 @@ def test_weights_are_not_rounded(pkg, oracle, gpu, layout, N, M, dtype):
     """Against 64-bit sums of scale * (q - z) only the output's rounding is left: its relative 2-norm is
     0.41 to 0.43 u (u = 2^-11, 2^-8; values spread over their binade), with rounded weights 0.59 u; the bar
     is half way."""
-    K, gs = 2048, 128
+    _unrounded(pkg, oracle, gpu, layout, 2048, N, M, dtype)
+
+
+@pytest.mark.parametrize("K,N,M", [(768, 17408, 33), (512, 16640, 48), (896, 17408, 40)])
+def test_weights_of_small_wide_matrices_are_not_rounded(pkg, oracle, gpu, K, N, M):
+    """Three row blocks on matrices small enough for the decode kernels, which carry the scale to the sums."""
+    assert pkg.ops.select_path(pkg.ops.make_packed(*[to_dev(a, gpu) for a in oracle.make_gptq(K, N, 128, seed=1)[:3]], None, 128, 0), M) == "gemv"
+    _unrounded(pkg, oracle, gpu, "gptq", K, N, M, "f16")
+
+
+def _unrounded(pkg, oracle, gpu, layout, K, N, M, dtype):
+    gs = 128
     if layout == "awq":
         qw, qz, sc = oracle.make_awq(K, N, gs, seed=N + M)
         deq = oracle.dequant_awq
@@ -115,4 +126,23 @@ def test_weights_are_not_rounded(pkg, oracle, gpu, layout, N, M, dtype):
     xt = to_dev(x, gpu, bf16=dtype == "bf16")
     want = xt.double().cpu().numpy() @ (ints * np.repeat(sc.astype(np.float64), gs, axis=0))
     err = np.linalg.norm(pkg.ops.linear(pk, xt).double().cpu().numpy() - want) / np.linalg.norm(want)
+    assert err <= 0.51 * (2.0**-8 if dtype == "bf16" else 2.0**-11)
+
+
+@pytest.mark.parametrize("T,E,dtype", [(52, 4, "f16"), (64, 4, "bf16"), (30, 2, "f16"), (48, 2, "bf16")])
+def test_weights_of_few_experts_are_not_rounded(pkg, oracle, gpu, T, E, dtype):
+    """Grouped launches of up to 64 tokens with three and four row blocks an expert, on wide matrices."""
+    K, N, gs, topk = 1024, 16384, 128, 2
+    parts = [oracle.make_gptq(K, N, gs, seed=E + e, sym=False)[:3] for e in range(E)]
+    packed = pkg.ops.make_packed_moe(*[torch.stack([to_dev(p[i], gpu) for p in parts]) for i in range(3)], gs)
+    x = to_dev(oracle.make_x(T, K, seed=T, dtype=dtype), gpu, bf16=dtype == "bf16")
+    routing = pkg.ops.moe_route(torch.randn((T, E), device=gpu, generator=torch.Generator(device=gpu).manual_seed(T)), topk)
+    got = pkg.ops.moe_linear(packed, x, routing, gather=True).double().cpu().numpy()
+    rows, offsets = routing.sorted_tokens.cpu().numpy(), routing.expert_offsets.cpu().numpy()
+    want = np.empty_like(got)
+    for e, (qw, qz, sc) in enumerate(parts):
+        w = np.asarray(oracle.dequant_gptq(qw, qz, np.ones_like(sc), None, gs, "f16")).astype(np.float64) * np.repeat(sc.astype(np.float64), gs, axis=0)
+        own = slice(offsets[e], offsets[e + 1])
+        want[own] = x.double().cpu().numpy()[rows[own]] @ w
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err <= 0.51 * (2.0**-8 if dtype == "bf16" else 2.0**-11)

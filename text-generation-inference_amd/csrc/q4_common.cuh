@@ -260,6 +260,7 @@ int launch_gptq_solve_block(float* W, const float* U, float* Q, float* Err, floa
                             int rows, int K, int i1, int count, int groupsize, int G, int sym, hipStream_t stream);
 int launch_moe_gather_columns(const void* x, const int32_t* x_rows, const int32_t* offsets, const int32_t* perms,
                               void* out, int num_experts, int pairs, int K, hipStream_t stream);
+bool moe_decode_tokens(const q4_weight* e0, int tokens);  // whether the grouped decode kernels' row limit holds them
 bool batch_moe_default(const q4_moe_weight* w, int tokens, int topk, bool gate_up);
 int launch_batch_moe_linear(const q4_moe_weight* w, const q4::MoeView& view, const void* x, void* y, int tokens, int topk,
                             int dtype, int gate_up_act, void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -43,7 +43,9 @@ static long batch_units(bool awq, int nq, bool gate_up, long rows) {
 // measured decomposition on average, 11 % at worst.
 // Grouped launches: `experts` that receive rows multiply the tiles, M is all their rows, mt the row
 // blocks of one workgroup.
-static bool batch_plan(const q4_weight* w, int M, int mt, int experts, bool gate_up, BatchPlan* plan) {
+// unrounded: only wave tiles on which the scale multiplies the sums (batch_late), for calls that the decode kernels
+// would hold, which carry the scale to the sums as well.
+static bool batch_plan(const q4_weight* w, int M, int mt, int experts, bool gate_up, bool unrounded, BatchPlan* plan) {
   const bool awq = w->layout == Q4_LAYOUT_AWQ, grouped = experts > 0;
   const int chunks = w->K / 128, wn = awq && gate_up ? 2 : 1;
   if (!grouped) experts = 1;
@@ -55,10 +57,12 @@ static bool batch_plan(const q4_weight* w, int M, int mt, int experts, bool gate
   double best = -1.0;
   for (int nq = awq ? 2 : 1; nq <= 2; ++nq) {
     if (w->N % (64 * nq * wn) != 0) continue;
+    if (unrounded && !q4::batch_late(awq ? q4::kBatchAwq : q4::kBatchGptq, mt, nq)) continue;
     const int tiles = w->N / (64 * nq * wn);
     // (128-column tiles that make two rounds on their own: their x traffic is half; 4096 x 28672 in four
     // experts, one row each: 44.8 us against 50.2)
-    if (nq == 1 && w->N % 128 == 0 && (long)tiles / 2 * experts >= 512) continue;
+    if (nq == 1 && w->N % 128 == 0 && (long)tiles / 2 * experts >= 512 && !(unrounded && !q4::batch_late(q4::kBatchGptq, mt, 2)))
+      continue;
     for (int wk = wn == 2 ? 4 : 8; wk >= 4; wk -= 4) {
       for (int sp = 1; sp <= 8; sp *= 2) {
         // every wave walks a chunk; the exchange cells fit; 128-column tiles that nearly fill the chip are
@@ -118,7 +122,9 @@ bool batch_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan
     if (dtype == Q4_DTYPE_BF16 && M <= 3 && weights >= (1L << 26) && !short_groups) return false;
     if (M > 48 && w->K > 8192 && weights >= (1L << 26)) return false;
   }
-  return batch_plan(w, M, (M + 15) / 16, 0, gate_up, plan);
+  // (33 rows and more that the decode kernels would hold, which carry the scale to the sums: small matrices)
+  const bool unrounded = M > 32 && q4_select_path(w, M, dtype) == Q4_PATH_GEMV;
+  return batch_plan(w, M, (M + 15) / 16, 0, gate_up, unrounded, plan);
 }
 
 static void batch_fill(BatchParams& bp, const q4_weight* w, int wk, int splits) {
@@ -183,15 +189,19 @@ static int batch_moe_blocks(int num_experts, int pairs) {
 // MFMA tiles, reduction and elementwise launch) / this one: first projection with its activation 1 token
 // 27.0 / 26.1, 16 tokens 111 / 82, 48 146 / 98, 64 194 / 101, 128 156 / 123, 256 (64 rows each) 232 / 229;
 // second 1 18.7 / 15.2, 16 76 / 40, 48 70 / 48, 64 73 / 47, 128 86 / 58, 256 112 / 111.
+static bool batch_moe_plan(const q4_moe_weight* w, int tokens, int pairs, bool gate_up, BatchPlan* plan) {
+  const q4_weight* e0 = &w->expert0;
+  return batch_plan(e0, pairs, batch_moe_blocks(w->num_experts, pairs), pairs < w->num_experts ? pairs : w->num_experts, gate_up,
+                    moe_decode_tokens(e0, tokens), plan);
+}
+
 bool batch_moe_default(const q4_moe_weight* w, int tokens, int topk, bool gate_up) {
   const long pairs = (long)tokens * topk;
   const q4_weight* e0 = &w->expert0;
   if (e0->layout != Q4_LAYOUT_GPTQ || tokens < 1 || pairs > 48L * w->num_experts || w->num_experts > 65535) return false;
   const long row_blocks = (tokens + 15) / 16;
   BatchPlan plan;
-  const int active = pairs < w->num_experts ? (int)pairs : w->num_experts;
-  return row_blocks * 8 <= 65535 && batch_supported(e0, (int)pairs, gate_up) &&
-         batch_plan(e0, (int)pairs, batch_moe_blocks(w->num_experts, (int)pairs), active, gate_up, &plan);
+  return row_blocks * 8 <= 65535 && batch_supported(e0, (int)pairs, gate_up) && batch_moe_plan(w, tokens, (int)pairs, gate_up, &plan);
 }
 
 // The rows of y, and of x without a row map, are the token-expert pairs sorted by expert.
@@ -201,7 +211,7 @@ int launch_batch_moe_linear(const q4_moe_weight* w, const q4::MoeView& view, con
   const int pairs = tokens * topk, mt = batch_moe_blocks(w->num_experts, pairs);
   const bool fuse = gate_up_act != 0;
   BatchPlan plan;
-  if (!batch_plan(e0, pairs, mt, pairs < w->num_experts ? pairs : w->num_experts, fuse, &plan)) {
+  if (!batch_moe_plan(w, tokens, pairs, fuse, &plan)) {
     set_error("q4_moe_linear(batch decode kernel): unsupported problem");
     return Q4_ERR_UNSUPPORTED;
   }

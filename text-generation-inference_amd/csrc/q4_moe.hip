@@ -253,8 +253,7 @@ MoeGemvPlan moe_gemv_plan(const q4_moe_weight* w, int tokens, int topk, int dtyp
   const bool awq = e0->layout == Q4_LAYOUT_AWQ;
   const bool act = !awq && e0->g_idx != nullptr;
   const int rows = tokens < kRowsPerBlock ? tokens : kRowsPerBlock;
-  const int max_tokens = (awq || act || e0->K > 8192) ? kMoeDecodeMaxTokensLongK : kMoeDecodeMaxTokens;
-  if (tokens > max_tokens || !gemv_supported(e0, rows, dtype)) return pl;
+  if (!moe_decode_tokens(e0, tokens) || !gemv_supported(e0, rows, dtype)) return pl;
   // fused epilogue: one token only (Mixtral gate_up, two experts: 33.5 us fused against 36.4 us with the
   // separate activation kernel; two tokens, four experts: 46.0 against 40.7 us)
   if (gate_up && (tokens > 1 || !gemv_gate_up_supported(e0, tokens, dtype))) return pl;
@@ -380,6 +379,11 @@ MoeView make_view(const q4_moe_weight* w, const int32_t* x_rows, const int32_t* 
 }
 
 }  // namespace
+
+bool moe_decode_tokens(const q4_weight* e0, int tokens) {
+  const bool narrow = e0->layout == Q4_LAYOUT_AWQ || e0->g_idx != nullptr || e0->K > 8192;
+  return tokens <= (narrow ? kMoeDecodeMaxTokensLongK : kMoeDecodeMaxTokens);
+}
 
 // Upper bound over the kernels a grouped launch of this weight can take (for any dtype the
 // plans are the same except that act-order bf16 has no decode kernel and goes to the MFMA one).
