@@ -93,9 +93,21 @@ int q4_dequant(const q4_weight* w, void* w_out, int dtype, void* stream);
 int q4_linear(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
               void* workspace, size_t workspace_bytes, void* stream);
 
-/* Same as q4_linear with the kernel path forced (Q4_PATH_*); for tests and benchmarks. */
+/*
+ * Same as q4_linear with the kernel path forced (Q4_PATH_*); for tests and benchmarks.  The batch decode kernel and the
+ * prefill kernels whose tiles follow the row count belong to neither path: they run under Q4_PATH_AUTO only.
+ */
 int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
                  void* workspace, size_t workspace_bytes, int path, void* stream);
+/*
+ * Which kernels q4_linear (gate_up = 0) or q4_linear_gate_up (gate_up = 1) run for this problem: a Q4_PATH_* or one of
+ * the Q4_KERNEL_* below (an answer only, no path to ask for); Q4_PATH_AUTO when no gated kernel takes it.  A pure
+ * function of (w's geometry, M, dtype).
+ */
+#define Q4_KERNEL_BATCH 4 /* up to 64 rows, GPTQ (contiguous groups) and AWQ */
+#define Q4_KERNEL_TALL 5  /* prefill, tiles of 96 to 256 rows, one wave per SIMD */
+#define Q4_KERNEL_BLOCK 6 /* prefill, tiles of 256 x 256, fp16 */
+int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);
 
 /*
  * First half of a gated MLP in one launch: W packs [gate | up] along N and

@@ -205,6 +205,31 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     assert lib.q4_linear_noalloc(ctypes.byref(w), None, None, None, 0, 0, None) == 0  # no rows: nothing to do
 
 
+@pytest.mark.parametrize("K,N,gs,layout,g_idx,M,dtype,gate_up,want", [
+    # decode: one to four fp16 rows keep their own kernels, the gated epilogue and bf16 start at one
+    (4096, 6144, 128, 0, False, 1, "f16", 0, "gemv"), (4096, 6144, 128, 0, False, 5, "f16", 0, "batch"),
+    (4096, 28672, 128, 0, False, 1, "f16", 1, "batch"), (3584, 37888, 128, 0, False, 13, "bf16", 0, "batch"),
+    (4096, 28672, 128, 0, False, 3, "bf16", 0, "gemv"), (8192, 57344, 128, 0, False, 16, "f16", 1, "none"),
+    (14336, 4096, 64, 0, False, 1, "f16", 0, "batch"), (4096, 14336, 32, 0, False, 37, "f16", 0, "gemm"),
+    (4608, 28672, 384, 0, False, 1, "f16", 1, "gemv"), (4096, 6144, 128, 0, False, 64, "f16", 0, "batch"),
+    (14336, 4096, 128, 0, False, 49, "f16", 0, "batch"), (14336, 8192, 128, 0, False, 49, "f16", 0, "gemm"),
+    (4096, 28672, 128, 1, False, 1, "f16", 0, "gemv"), (4096, 28672, 128, 1, False, 16, "f16", 1, "batch"),
+    (4096, 4096, 128, 1, False, 1, "f16", 0, "batch"), (14336, 4096, 128, 1, False, 33, "f16", 0, "gemm"),
+    (8192, 10240, 128, 0, True, 4, "f16", 0, "gemv"), (8192, 10240, 128, 0, True, 33, "f16", 0, "gemm"),
+    # prefill
+    (4096, 6144, 128, 0, False, 2048, "bf16", 0, "gemm"), (4096, 28672, 128, 0, False, 2048, "bf16", 1, "gemm"),
+    (4096, 28672, 128, 0, False, 301, "f16", 1, "tall"), (14336, 4096, 128, 0, False, 301, "f16", 0, "tall"),
+    (4096, 28672, 128, 0, False, 1000, "f16", 1, "block"), (14336, 4096, 128, 1, False, 1000, "f16", 0, "block"),
+    (14336, 4096, 128, 1, False, 1000, "bf16", 0, "tall"), (4096, 28672, 32, 0, False, 301, "f16", 0, "gemm"),
+    (4104, 4104, 8, 0, False, 16, "f16", 0, "generic"), (4104, 4104, 8, 0, False, 16, "f16", 1, "none"),
+])
+def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, want):
+    """Which kernels the library's own choice runs (the sides of the measured crossovers); a forced path runs its own."""
+    w = _weight(pkg, K, N, gs, layout, g_idx)
+    rc = pkg._lib.load().q4_linear_kernel(ctypes.byref(w), M, 1 if dtype == "bf16" else 0, gate_up)
+    assert pkg._lib.KERNEL_NAMES[rc] == want
+
+
 def test_path_selection_and_workspace(pkg):
     lib = pkg._lib.load()
     L = pkg._lib
@@ -217,6 +242,7 @@ def test_path_selection_and_workspace(pkg):
         w2 = _weight(pkg, K, N, 128)
         assert lib.q4_select_path(ctypes.byref(w2), last_gemv, 0) == L.PATH_GEMV, (K, N)
         assert lib.q4_select_path(ctypes.byref(w2), last_gemv + 1, 0) == L.PATH_GEMM, (K, N)
+    assert int(dict(re.findall(r"#define\s+(Q4_KERNEL_[A-Z]+)\s+(\d+)", HEADER.read_text()))["Q4_KERNEL_BATCH"]) == L.KERNEL_BATCH
     odd = _weight(pkg, 4104, 4104, 8)
     assert lib.q4_select_path(ctypes.byref(odd), 1, 0) == L.PATH_GENERIC
     assert lib.q4_select_path(ctypes.byref(odd), 512, 0) == L.PATH_GENERIC

@@ -19,7 +19,7 @@ TOL_BF16 = 8e-3
 
 
 def _case(pkg, oracle, gpu, K, N, gs, M, act="silu", dtype="f16", layout="gptq", act_order=False, bias=False,
-          fused=None, seed=0):
+          fused=None, seed=0, tol=None):
     bf = dtype == "bf16"
     if layout == "gptq":
         qw, qz, sc, gi = oracle.make_gptq(K, N, gs, seed=seed, sym=False, act_order=act_order)
@@ -45,9 +45,10 @@ def _case(pkg, oracle, gpu, K, N, gs, M, act="silu", dtype="f16", layout="gptq",
     assert np.isfinite(g).all()
     ref = oracle.to_f32(want, dtype)
     err = max_rel_err(g, ref)
-    assert err <= (TOL_BF16 if bf else TOL), f"max rel err {err:.3e}"
+    tol = tol or (TOL_BF16 if bf else TOL)
+    assert err <= tol, f"max rel err {err:.3e}"
     # and against the unrounded fp32 chain
-    assert max_rel_err(g, exact) <= (TOL_BF16 if bf else TOL)
+    assert max_rel_err(g, exact) <= tol
     return g
 
 
@@ -72,6 +73,18 @@ def test_decode_small_shapes_split_k(pkg, oracle, gpu, K, N, gs, M):
 def test_decode_fused_ragged_k_partition(pkg, oracle, gpu, M):
     """43 chunks of 128 rows do not divide over the wave slots of the fused kernel."""
     _case(pkg, oracle, gpu, 43 * 128, 512, 128, M, fused=True, seed=M + 5)
+
+
+@pytest.mark.parametrize("K,N,gs", [(256, 256, 128), (384, 1024, 384), (1152, 512, 384), (2304, 1024, 1152)])
+@pytest.mark.parametrize("M,dtype", [(1, "f16"), (2, "f16"), (1, "bf16"), (2, "bf16")])
+def test_decode_slab_kernel(pkg, oracle, gpu, K, N, gs, M, dtype):
+    """What the batch decode kernel does not take (K below 512 rows, groups that are no power of two times 64) runs on the
+    slab kernel's gated epilogue.  Its weights are unrounded, so each of the three roundings can fall on the neighbouring
+    value: 3 x 2^-8 in bf16, 3 x 2^-11 (inside the bar) in fp16."""
+    pk = pkg.ops.make_packed(*[to_dev(a, gpu) for a in oracle.make_gptq(K, N, gs, seed=1)[:3]], None, gs, 0)
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if dtype == "bf16" else torch.float16, gate_up=True) == "gemv"
+    _case(pkg, oracle, gpu, K, N, gs, M, dtype=dtype, bias=True, fused=True, seed=K + M,
+          tol=1.2e-2 if dtype == "bf16" else None)
 
 
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "gelu", "gelu_fast", "gelu_pytorch_tanh"])

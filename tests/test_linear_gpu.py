@@ -201,6 +201,49 @@ def test_generic_path(pkg, oracle, gpu, layout, act, M):
          layout=layout, sym=False, act=act, bias=True, path=3, seed=M + 50)
 
 
+@pytest.mark.parametrize("layout", ["gptq", "awq"])
+@pytest.mark.parametrize("M", [8, 37])
+def test_a_forced_path_runs_its_own_kernels(pkg, oracle, gpu, layout, M):
+    """The prefill kernels round every weight, the batch decode kernel that the library picks for these rows does not:
+    against 64-bit sums of the rounded weights (whose relative 2-norm from the unrounded sums is about 0.4 u) only the
+    output's rounding, 0.43 u, is left on the forced path, and sqrt(0.43^2 + 0.4^2) u = 0.59 u on the batch kernel; the
+    bar is half way.  The forced decode path agrees with both but runs the sums in an order of its own."""
+    K, N, gs = 2048, 1024, 128
+    if layout == "awq":
+        qw, qz, sc = oracle.make_awq(K, N, gs, seed=M)
+        w = oracle.dequant_awq(qw, qz, sc, gs, "f16")
+    else:
+        qw, qz, sc, _ = oracle.make_gptq(K, N, gs, seed=M, sym=False)
+        w = oracle.dequant_gptq(qw, qz, sc, None, gs, "f16")
+    pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), None, gs, 1 if layout == "awq" else 0)
+    assert pkg.ops.kernel_of(pk, M) == "batch"
+    x = oracle.make_x(M, K, seed=M)
+    xt = to_dev(x, gpu)
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    gemv, gemm, auto = (pkg.ops.linear(pk, xt, None, path=p) for p in (1, 2, 0))
+    err = np.linalg.norm(gemm.double().cpu().numpy() - want) / np.linalg.norm(want)
+    assert err <= 0.51 * 2.0**-11
+    assert not torch.equal(gemm, auto) and not torch.equal(gemv, auto) and not torch.equal(gemv, gemm)
+    assert max_rel_err(to_f32(gemv), to_f32(gemm)) <= TOL
+
+
+@pytest.mark.parametrize("layout", ["gptq", "awq"])
+def test_a_forced_prefill_path_keeps_its_tiles(pkg, oracle, gpu, layout):
+    """Where the library picks the kernel whose tiles follow the row count, the forced path runs its own tiles and
+    K splits: other bits, the same sums."""
+    K, N, gs, M = (5504, 4096, 128, 301) if layout == "awq" else (4096, 4096, 128, 700)
+    if layout == "awq":
+        qw, qz, sc = oracle.make_awq(K, N, gs, seed=M)
+    else:
+        qw, qz, sc, _ = oracle.make_gptq(K, N, gs, seed=M, sym=False)
+    pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), None, gs, 1 if layout == "awq" else 0)
+    assert pkg.ops.kernel_of(pk, M) == "tall"
+    xt = to_dev(oracle.make_x(M, K, seed=M), gpu)
+    gemm, auto = pkg.ops.linear(pk, xt, None, path=2), pkg.ops.linear(pk, xt)
+    assert not torch.equal(gemm, auto)
+    assert max_rel_err(to_f32(auto), to_f32(gemm)) <= 1e-3
+
+
 # --------------------------------------------------------------------------- prefill GEMM
 
 

@@ -35,6 +35,8 @@ def test_row_tiles(pkg, oracle, gpu, layout, M, K, dtype):
     N = 28672
     pk, w = _weight(pkg, oracle, gpu, layout, K, N, 64, K + M, dtype)
     bf = dtype == "bf16"
+    dt = torch.bfloat16 if bf else torch.float16
+    assert all(pkg.ops.kernel_of(pk, M, dt, gate_up) in ("tall", "block") for gate_up in (False, True))
     x = oracle.make_x(M, K, seed=M, dtype=dtype)
     b32 = np.random.default_rng(M).standard_normal(N).astype(np.float32)
     bias = oracle.f32_to_bf16_bits(b32) if bf else b32.astype(np.float16)
@@ -59,6 +61,23 @@ def test_splits(pkg, oracle, gpu, layout, M, K, N, gs, dtype):
     got = pkg.ops.linear(pk, xt)
     again = pkg.ops.linear(pk, xt)
     assert torch.equal(got, again)
+    assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
+
+
+# ... and where the library picks these kernels for them, the 256 x 256 one included; K in 32 and 86 K tiles
+@pytest.mark.parametrize("layout,M,K,N,gs,dtype", [
+    ("gptq", 66, 2048, 256, 128, "f16"), ("gptq", 700, 4096, 1024, 256, "f16"), ("gptq", 301, 5504, 2048, 128, "bf16"),
+    ("gptq", 1000, 2048, 512, 2048, "bf16"), ("awq", 66, 2048, 256, 128, "f16"), ("awq", 301, 5504, 4096, 64, "f16"),
+    ("awq", 1000, 5504, 4096, 128, "f16"), ("awq", 512, 5504, 2048, 64, "bf16"), ("awq", 100, 2048, 512, 2048, "bf16")])
+def test_splits_of_the_picked_kernels(pkg, oracle, gpu, layout, M, K, N, gs, dtype):
+    pk, w = _weight(pkg, oracle, gpu, layout, K, N, gs, K + M, dtype)
+    bf = dtype == "bf16"
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16) in ("tall", "block")
+    x = oracle.make_x(M, K, seed=M, dtype=dtype)
+    y32, _ = oracle.linear_forward(x, w, None, dtype)
+    xt = to_dev(x, gpu, bf16=bf)
+    got = pkg.ops.linear(pk, xt)
+    assert torch.equal(got, pkg.ops.linear(pk, xt))
     assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
 
 

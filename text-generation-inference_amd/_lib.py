@@ -24,6 +24,10 @@ PATH_GEMV = 1
 PATH_GEMM = 2
 PATH_GENERIC = 3
 PATH_NAMES = {PATH_GEMV: "gemv", PATH_GEMM: "gemm", PATH_GENERIC: "generic"}
+KERNEL_BATCH = 4
+KERNEL_TALL = 5
+KERNEL_BLOCK = 6
+KERNEL_NAMES = {**PATH_NAMES, PATH_AUTO: "none", KERNEL_BATCH: "batch", KERNEL_TALL: "tall", KERNEL_BLOCK: "block"}
 WORKSPACE_COUNTER_BYTES = 4210688
 
 ERR_INVALID_ARGUMENT = -1
@@ -78,6 +82,7 @@ SIGNATURES = {
         c_int,
         [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_size_t, c_int, c_void_p],
     ),
+    "q4_linear_kernel": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int]),
     "q4_gemv_tuned": (
         c_int,
         [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_size_t, c_int, c_int, c_int, c_int, c_void_p],

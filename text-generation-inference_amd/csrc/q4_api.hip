@@ -241,6 +241,28 @@ size_t q4_workspace_bytes(int M, int K, int N) {
   return (size_t)Q4_WORKSPACE_COUNTER_BYTES + (decode > prefill ? decode : prefill);
 }
 
+int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up) {
+  int rc = validate_weight(w, "q4_linear_kernel");
+  if (rc == Q4_OK) rc = validate_dtype(dtype, "q4_linear_kernel");
+  if (rc != Q4_OK) return rc;
+  if (M < 0) {
+    set_error("q4_linear_kernel: negative M=%d", M);
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
+  if (M == 0 || w->K == 0 || w->N == 0) return gate_up ? Q4_PATH_AUTO : Q4_PATH_GENERIC;
+  if (gate_up && (w->N & 1)) return Q4_PATH_AUTO;
+  const int path = q4_select_path(w, M, dtype);
+  BatchPlan batch;
+  if ((gate_up || path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) && batch_default(w, M, dtype, gate_up != 0, &batch))
+    return Q4_KERNEL_BATCH;
+  TallPlan tall;
+  if (path == Q4_PATH_GEMM && gemm_tall_default(w, M, dtype, gate_up != 0, &tall))
+    return tall.block ? Q4_KERNEL_BLOCK : Q4_KERNEL_TALL;
+  if (!gate_up) return path;
+  if (path == Q4_PATH_GEMV) return gemv_gate_up_supported(w, M, dtype) ? path : Q4_PATH_AUTO;
+  return path == Q4_PATH_GEMM && gemm_gate_up_supported(w, M, dtype) ? path : Q4_PATH_AUTO;
+}
+
 int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
                  void* workspace, size_t workspace_bytes, int path, void* stream) {
   int rc = validate_weight(w, "q4_linear");
@@ -259,18 +281,22 @@ int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, i
     set_error("q4_linear: x, y and the workspace must be 16-byte aligned (bias: 2-byte)");
     return Q4_ERR_INVALID_ARGUMENT;
   }
-  if (path == Q4_PATH_AUTO) path = q4_select_path(w, M, dtype);
-  // a batch of decode rows: one kernel, whichever of the two paths the row count belongs to
-  BatchPlan batch;
-  if ((path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) && batch_default(w, M, dtype, false, &batch))
-    return launch_batch(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, batch, (hipStream_t)stream);
+  // The kernels that belong to neither path run where the caller leaves the choice: a batch of decode rows is one
+  // kernel's, whichever of the two paths the row count belongs to.
+  if (path == Q4_PATH_AUTO) {
+    path = q4_select_path(w, M, dtype);
+    BatchPlan batch;
+    if ((path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) && batch_default(w, M, dtype, false, &batch))
+      return launch_batch(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, batch, (hipStream_t)stream);
+    TallPlan tall;
+    if (path == Q4_PATH_GEMM && gemm_tall_default(w, M, dtype, false, &tall))
+      return launch_gemm_tall(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, tall, (hipStream_t)stream);
+  }
   switch (path) {
     case Q4_PATH_GEMV:
       return launch_gemv(w, x, bias, y, M, dtype, workspace, workspace_bytes, nullptr,
                          (hipStream_t)stream);
     case Q4_PATH_GEMM:
-      if (TallPlan tall; gemm_tall_default(w, M, dtype, false, &tall))
-        return launch_gemm_tall(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, tall, (hipStream_t)stream);
       if (w->layout == Q4_LAYOUT_AWQ || w->g_idx != nullptr)
         return launch_gemm_awq(w, x, bias, y, M, dtype, workspace, workspace_bytes, (hipStream_t)stream);
       return launch_gemm(w, x, bias, y, M, dtype, workspace, workspace_bytes, (hipStream_t)stream);
@@ -352,14 +378,14 @@ int q4_linear_perm(const q4_weight* w, const int32_t* perm, const void* x, const
     set_error("q4_linear_perm: x and y must be 16-byte aligned (bias: 2-byte)");
     return Q4_ERR_INVALID_ARGUMENT;
   }
-  if (path == Q4_PATH_AUTO) path = q4_select_path(w, M, dtype);
+  const int range = path == Q4_PATH_AUTO ? q4_select_path(w, M, dtype) : path;
   // Decode of a few rows with a short K: the kernel reads x through perm while it stages its
   // activation slab.  Every workgroup gathers its own copy, so the saved launch (~2.5 us) is
   // soon outweighed: measured against the separate pass at M = 1, 4096 x 4096 6.4 / 7.8 us,
   // 4096 x 28672 15.8 / 17.3, but 14336 x 4096 13.4 / 12.3, 28672 x 8192 29.0 / 26.0; at M = 4
   // 4096 x 4096 9.1 / 10.6, 4096 x 6144 9.8 / 10.7, but 4096 x 28672 20.2 / 19.2; at M = 8
   // 4096 x 6144 12.7 / 11.7; at M = 16 4096 x 6144 18.1 / 14.3, 14336 x 4096 37.9 / 20.0.
-  if (path == Q4_PATH_GEMV && w->K <= 4096 && (M <= 2 || (M <= 4 && w->N <= 8192)))
+  if (range == Q4_PATH_GEMV && w->K <= 4096 && (M <= 2 || (M <= 4 && w->N <= 8192)))
     return launch_gemv(w, x, bias, y, M, dtype, workspace, workspace_bytes, nullptr, (hipStream_t)stream, 0, perm);
   // otherwise one gather pass into the tail of the workspace, then the kernel of the plain call
   if (w->K % 8 != 0) {

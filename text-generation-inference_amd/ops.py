@@ -444,12 +444,10 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev, out_given) ->
     bias_ptr = bias.data_ptr() if bias is not None else None
     # decode: split-K partial sums, tickets, accumulation cells; prefill GEMM: split-K
     # partial tiles when the tile grid alone would leave CUs idle
-    planned_path, need, tuned = w.plan(M, code)
+    _, need, tuned = w.plan(M, code)
     scratch = w.regroup(M, code, False)[1] if path == PATH_AUTO and gemv_config is None else 0
-    if path == PATH_AUTO and gemv_config is None:
-        path = planned_path
-        if tuned is not None and w.perm is None:
-            gemv_config = tuned  # the decomposition a tuning pass measured fastest
+    if path == PATH_AUTO and gemv_config is None and tuned is not None and w.perm is None:
+        gemv_config = tuned  # the decomposition a tuning pass measured fastest
     ws = _workspace_for_call(dev, need, stream)
     st = w.struct()
     if gemv_config is not None:
@@ -559,7 +557,9 @@ def autotune(weights=None, rows=(1, 2, 3, 4, 8, 16), dtype: torch.dtype = torch.
                 need = max([ws[0].plan(M, code)[1]] + [
                     int(lib.q4_gemv_tuned_workspace_bytes(ctypes.byref(ws[0].struct()), M, code, *cfg)) for cfg in cands])
                 reserve_workspace(device, need, SHARED)
-                base = _time_graph_launches([(lambda w=w: linear(w, x, None, path=_lib.PATH_GEMV, out=y)) for w in rot], reps)
+                for w in ws:  # the library's own choice, without what an earlier pass has set
+                    w._plans[(M, code)] = w.plan(M, code)[:2] + (None,)
+                base = _time_graph_launches([(lambda w=w: linear(w, x, None, out=y)) for w in rot], reps)
                 best_t, best_cfg = base, None
                 for cfg in cands:
                     try:
@@ -676,6 +676,14 @@ def linear_gate_up(
     elif fused:
         raise ValueError("the fused kernel needs a bias of x's dtype with N entries (or none)")
     return act_mul(linear(w, x, bias), act, out=y)
+
+
+def kernel_of(w: PackedWeight, M: int, dtype: torch.dtype = torch.float16, gate_up: bool = False) -> str:
+    """The kernels that `linear` (or the fused `linear_gate_up`) runs for M rows by the library's own choice
+    (q4_linear_kernel); "none" where no fused kernel takes the problem."""
+    rc = _lib.load().q4_linear_kernel(w.struct(), int(M), _DTYPES[dtype], int(gate_up))
+    _lib.check(rc)
+    return _lib.KERNEL_NAMES[rc]
 
 
 def select_path(w: PackedWeight, M: int, dtype: torch.dtype = torch.float16) -> str:
