@@ -261,10 +261,11 @@ size_t q4_workspace_bytes(int M, int K, int N);
  */
 size_t q4_workspace_bytes_for(const q4_weight* w, int M);
 /*
- * Everything a caller needs to know before q4_linear_ex(w, ..., M, dtype, ...) in one call:
+ * Everything a caller needs to know before q4_linear(w, ..., M, dtype, ...) in one call:
  * *path = q4_select_path(w, M, dtype), *workspace_bytes = q4_workspace_bytes_for(w, M).  Both are
- * pure functions of (w's geometry, M, dtype): a caller may keep them per layer and batch size
- * and pass `path` to q4_linear_ex.  Replaces the per-layer sizing the reference does once at
+ * pure functions of (w's geometry, M, dtype): a caller may keep them per layer and batch size.  `path` says
+ * whether the row count is decode or prefill for this weight; passed to q4_linear_ex it leaves out the kernels
+ * that belong to neither path (Q4_KERNEL_*).  Replaces the per-layer sizing the reference does once at
  * Warmup (server/text_generation_server/layers/gptq/exllamav2.py:159-175, 233-240).
  */
 int q4_linear_plan(const q4_weight* w, int M, int dtype, int* path, size_t* workspace_bytes);

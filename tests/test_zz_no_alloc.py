@@ -16,7 +16,7 @@ from tests.util import bits_of, max_rel_err, to_dev, to_f32
 pytestmark = pytest.mark.gpu
 
 
-def _both(pkg, oracle, gpu, K, N, M, layout="gptq", dtype="f16", act=False, seed=0):
+def _both(pkg, oracle, gpu, K, N, M, layout="gptq", dtype="f16", act=False, seed=0, kernel=None):
     bf = dtype == "bf16"
     if layout == "gptq":
         qw, qz, sc, gi = oracle.make_gptq(K, N, 128, seed=seed, sym=False, act_order=act)
@@ -31,6 +31,7 @@ def _both(pkg, oracle, gpu, K, N, M, layout="gptq", dtype="f16", act=False, seed
     y32, _ = oracle.linear_forward(x, w, None, dtype)
     pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), to_dev(gi, gpu), 128, lay)
     xt = to_dev(x, gpu, bf16=bf)
+    assert kernel in (None, pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16))
     want = pkg.ops.linear(pk, xt, None)  # q4_linear_ex with a torch workspace
     got = torch.full_like(want, float("nan"))
     lib = pkg._lib.load()
@@ -50,15 +51,19 @@ def _both(pkg, oracle, gpu, K, N, M, layout="gptq", dtype="f16", act=False, seed
 def test_noalloc_matches_q4_linear_two_calls_in_a_row(pkg, oracle, gpu):
     assert pkg._lib.load().q4_noalloc_init() == 0
     # decode with K split over workgroups (fixed-point cells), then a smaller decode problem
-    _both(pkg, oracle, gpu, 4096, 4096, 1, seed=1)
-    _both(pkg, oracle, gpu, 2048, 1024, 1, seed=2)
-    # ticket path (several rows), then fewer rows on a smaller matrix
-    _both(pkg, oracle, gpu, 14336, 4096, 8, seed=3)
-    _both(pkg, oracle, gpu, 4096, 1024, 5, seed=4)
+    _both(pkg, oracle, gpu, 4096, 4096, 1, seed=1, kernel="gemv")
+    _both(pkg, oracle, gpu, 2048, 1024, 1, seed=2, kernel="gemv")
+    # several rows (batch decode kernel, exchange cells), then fewer rows on a smaller matrix
+    _both(pkg, oracle, gpu, 14336, 4096, 8, seed=3, kernel="batch")
+    _both(pkg, oracle, gpu, 4096, 1024, 5, seed=4, kernel="batch")
+    _both(pkg, oracle, gpu, 4096, 2048, 16, layout="awq", seed=8, kernel="batch")
+    # ticket path (act-order, bf16)
+    _both(pkg, oracle, gpu, 4096, 1024, 5, act=True, dtype="bf16", seed=9, kernel="gemv")
     # prefill: split-K partial tiles in the array, then a smaller prefill and a decode call
-    _both(pkg, oracle, gpu, 4096, 1024, 256, seed=5)
-    _both(pkg, oracle, gpu, 2048, 512, 96, seed=6)
-    _both(pkg, oracle, gpu, 2048, 512, 1, seed=7)
+    _both(pkg, oracle, gpu, 4096, 1024, 256, seed=5, kernel="tall")
+    _both(pkg, oracle, gpu, 4096, 1024, 300, layout="awq", seed=10, kernel="gemm")
+    _both(pkg, oracle, gpu, 2048, 512, 96, seed=6, kernel="tall")
+    _both(pkg, oracle, gpu, 2048, 512, 1, seed=7, kernel="gemv")
 
 
 @pytest.mark.parametrize("layout,act,dtype", [("awq", False, "f16"), ("gptq", True, "f16"), ("gptq", False, "bf16")])

@@ -791,7 +791,8 @@ int q4_linear_noalloc(const q4_weight* w, const void* x, const void* bias, void*
   }
   void* ptr = scratch_of_current_device("q4_linear_noalloc");
   if (ptr == nullptr) return Q4_ERR_LAUNCH;
-  return q4_linear_ex(w, x, bias, y, M, dtype, ptr, Q4_SCRATCH_BYTES, path, stream);
+  // (not `path`: a forced path leaves out the kernels that belong to neither)
+  return q4_linear_ex(w, x, bias, y, M, dtype, ptr, Q4_SCRATCH_BYTES, Q4_PATH_AUTO, stream);
 }
 
 int q4_linear(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
