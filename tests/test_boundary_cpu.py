@@ -221,6 +221,12 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     (4096, 28672, 128, 0, False, 301, "f16", 1, "tall"), (14336, 4096, 128, 0, False, 301, "f16", 0, "tall"),
     (4096, 28672, 128, 0, False, 1000, "f16", 1, "block"), (14336, 4096, 128, 1, False, 1000, "f16", 0, "block"),
     (14336, 4096, 128, 1, False, 1000, "bf16", 0, "tall"), (4096, 28672, 32, 0, False, 301, "f16", 0, "gemm"),
+    (4096, 28672, 128, 0, False, 2048, "bf16", 0, "gemm"), (4096, 28672, 128, 0, False, 1000, "bf16", 0, "tall"),
+    (4096, 12288, 128, 0, False, 2048, "f16", 0, "gemm"), (4096, 12288, 128, 0, False, 2048, "f16", 1, "gemm"),
+    (4096, 4096, 128, 0, False, 1400, "f16", 0, "gemm"), (4096, 4096, 128, 0, False, 700, "f16", 0, "tall"),
+    (1024, 8192, 128, 1, False, 1000, "f16", 0, "gemm"), (1024, 8192, 128, 1, False, 1000, "f16", 1, "tall"),
+    (1024, 8192, 128, 1, False, 512, "bf16", 1, "none"), (1024, 8192, 128, 1, False, 100, "bf16", 0, "tall"),
+    (1024, 8192, 128, 1, False, 2048, "f16", 0, "block"), (8192, 57344, 128, 0, False, 2048, "bf16", 0, "tall"),
     (4104, 4104, 8, 0, False, 16, "f16", 0, "generic"), (4104, 4104, 8, 0, False, 16, "f16", 1, "none"),
 ])
 def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, want):

@@ -65,11 +65,33 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
 // picked are 1 % above the best ones.  At 160 and 301 rows, where 128-row tiles pad most, 1.1-1.5.
 // GPTQ gate_up projections of several rounds stay with the 128 x 256 tiles, two workgroups per CU (4096 x 28672 at
 // 1400 rows 0.92-0.95, at 2048 0.92-0.99).
+// The estimates are off by up to 15 %.  Over 19 layer shapes x 17 row counts (65 .. 2048) these kernels are the pick in 626
+// cases: time of the others over theirs, geometric mean (least, most), GPTQ 1.13 (0.95, 1.55) in fp16, 1.16 (0.96, 1.60) in bf16,
+// gated 1.20 (1.00, 1.58) and 1.17 (0.99, 1.52); AWQ 1.15 (0.97, 1.39), 1.17 (0.98, 1.34), gated 1.11 (0.97, 1.40) and 1.06
+// (0.97, 1.26); the least is 8192 x 1280 at 512 rows.  What the estimates would give them beyond that, tall_outdone leaves to
+// the others (the same quotient):
+//   GPTQ, tiles below 256 rows, three rounds of the chip and more: every CU is at work, and these tiles unpack a weight as
+//     often as two 128-row workgroups: 4096 x 28672 at 1400 and 2048 rows 0.93-0.96, 4096 x 12288 at 2048 0.92, gated 0.95,
+//     8192 x 57344 at 1400 0.96; 256-row tiles in 3.5-7 rounds 0.97-1.06
+//   GPTQ, 96-row tiles for more than 1024 rows: 4096 x 4096 and 3584 x 3584 at 1400 0.93-0.94; at 700 0.97-1.07
+//   AWQ, K of at most 16 K tiles, where start and epilogue count as much as the tiles in between: 1024 x 8192 at 1000
+//     rows 0.90, gated bf16 at 512 to 1400 rows 0.86-1.02; up to 129 rows, in splits, 1.13-1.28, 256 x 256 tiles 1.20-1.34,
+//     gated fp16 0.97-1.08
+static bool tall_outdone(bool awq, int dtype, int M, int K, int N, bool gate_up, const TallPlan& plan) {
+  if (plan.block) return false;
+  if (awq) return K <= 1024 && M > 384 && (!gate_up || dtype == Q4_DTYPE_BF16);
+  const long tiles = (long)((M + 32 * plan.r - 1) / (32 * plan.r)) * (N / q4::kTallBN);
+  return (plan.r < 8 && tiles >= 3 * 256) || (plan.r == 3 && !gate_up && M > 1024);
+}
+
 bool gemm_tall_default(const q4_weight* w, int M, int dtype, bool gate_up, TallPlan* plan) {
   if (M <= 64 || !gemm_tall_supported(w, M)) return false;
   const bool awq = w->layout == Q4_LAYOUT_AWQ;
   auto others = [&](bool fused) { return awq ? gemm_awq_direct_estimate_us(w, M, dtype) : gemm_estimate_us(w, M, fused); };
-  if (!gate_up) return tall_plan(awq, dtype, M, w->K, w->N, false, plan) * 1.08 < others(false);
+  auto taken = [&](double other) {
+    return tall_plan(awq, dtype, M, w->K, w->N, gate_up, plan) * 1.08 < other && !tall_outdone(awq, dtype, M, w->K, w->N, gate_up, *plan);
+  };
+  if (!gate_up) return taken(others(false));
   const bool old_fused = gemm_gate_up_supported(w, M, dtype);
   if (old_fused && M > 1024 && (long)((M + 127) / 128) * (w->N / 256) > 1024) return false;
   double other = others(true);
@@ -80,7 +102,7 @@ bool gemm_tall_default(const q4_weight* w, int M, int dtype, bool gate_up, TallP
     other = others(false);
     other = (t < other ? t : other) + 4.0 + (double)M * w->N * 3e-6 / 5.0;
   }
-  return tall_plan(awq, dtype, M, w->K, w->N, true, plan) * 1.08 < other;
+  return taken(other);
 }
 
 // fp32 partial tiles of the largest split any layout and data type would pick
