@@ -216,6 +216,11 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     (4096, 28672, 128, 1, False, 1, "f16", 0, "gemv"), (4096, 28672, 128, 1, False, 16, "f16", 1, "batch"),
     (4096, 4096, 128, 1, False, 1, "f16", 0, "batch"), (14336, 4096, 128, 1, False, 33, "f16", 0, "gemm"),
     (8192, 10240, 128, 0, True, 4, "f16", 0, "gemv"), (8192, 10240, 128, 0, True, 33, "f16", 0, "gemm"),
+    (8192, 57344, 128, 1, False, 5, "f16", 0, "gemv"), (8192, 57344, 128, 1, False, 5, "bf16", 1, "none"),
+    (8192, 57344, 128, 1, False, 7, "f16", 0, "batch"), (8192, 57344, 128, 1, False, 7, "f16", 1, "batch"),
+    (3584, 37888, 128, 1, False, 32, "f16", 0, "batch"), (3584, 37888, 128, 1, False, 33, "f16", 0, "gemm"),
+    (3584, 37888, 128, 0, False, 49, "bf16", 0, "gemm"), (3584, 37888, 128, 0, False, 49, "bf16", 1, "batch"),
+    (3584, 37888, 128, 0, False, 49, "f16", 0, "batch"),
     # prefill
     (4096, 6144, 128, 0, False, 2048, "bf16", 0, "gemm"), (4096, 28672, 128, 0, False, 2048, "bf16", 1, "gemm"),
     (4096, 28672, 128, 0, False, 301, "f16", 1, "tall"), (14336, 4096, 128, 0, False, 301, "f16", 0, "tall"),

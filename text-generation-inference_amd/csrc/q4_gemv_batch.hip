@@ -93,34 +93,43 @@ static bool batch_plan(const q4_weight* w, int M, int mt, int experts, bool gate
 }
 
 // Where this kernel is the one to run, measured on MI355X against the kernels it takes over from
-// (24 layer shapes; time of theirs over time of this one, geometric mean and smallest):
-//   GPTQ fp16     8 rows 1.13 (1.01), 16 1.28 (1.10), 24 1.57 (1.27), 40 1.36 (1.08), 64 1.18 (0.90); four rows
-//                 and less 0.93-1.03: left to the short-launch kernel
-//   GPTQ bf16     1 row 1.17 (0.87: layers of 2^26 weights and more, left to the lean kernel up to 3
-//                 rows), 8 1.27, 16 1.36, 24 1.60, 40 1.40, 64 1.22
-//   gated epilogue against the plain launch and the elementwise kernel: from one row on 1.00-1.24
-//   AWQ           1 row 1.04 (1.4 on small layers, 0.79 on large: left out up to four rows), 8 1.39, 16 1.37, 24 1.22, 32 1.19,
-//                 48 1.10 (0.85)
+// (19 layer shapes; time of theirs over time of this one, geometric mean and smallest):
+//   GPTQ fp16     5 rows 1.10 (1.00), 8 1.13 (1.02), 16 1.24 (1.07), 24 1.53 (1.31), 32 1.49 (1.25), 48 1.30 (1.10), 64 1.14 (0.93);
+//                 four rows and less 0.93-1.03: left to the short-launch kernel
+//   GPTQ bf16     1 row 1.30 (0.96; 0.87 on layers of 2^26 weights and more, left to the lean kernel up to 3
+//                 rows), 8 1.26 (0.97), 16 1.34 (1.01), 24 1.55 (1.23), 32 1.53 (1.24), 48 1.34 (1.09), 64 1.20 (0.98)
+//   gated epilogue against the plain launch and the elementwise kernel: GPTQ 1 row 1.15 (0.98) and 1.61, 8 1.40 (1.26), 16 1.44
+//                 (1.22), 32 1.59 (1.24), 64 1.24 (1.08); AWQ 8 1.30 (1.03), 16 1.26 (1.02), 24 1.12 (0.99), 32 1.06 (0.88: 4096 x 12288)
+//   AWQ           1 row 1.19 (1.03; 0.79 on large layers: left out up to four rows), 5 1.30 (0.95), 8 1.35 (0.94), 16 1.33 (0.91),
+//                 24 1.18 (0.84), 32 1.17 (0.84), 48 1.16 (0.95)
 //   groups of 64  1-4 rows, plain launch, theirs / this one in us: fp16 4096 x 4096 6.06-6.65 / 5.25, 14336 x 4096
 //                 11.0-12.9 / 9.4, 4096 x 28672 16.2-17.7 / 14.4; bf16 4096 x 28672 21.5-23.0 / 16.7, 28672 x 8192
 //                 32.5-41.1 / 27.5; no slower on any of 12 shapes
 // The gated epilogue on 2^28 weights and more up to 16 rows stays with two launches (8192 x 57344, fp16, gated / two:
 // 1 row 51.8 / 43.8 us, 4 rows 54.6 / 49.0, 16 rows 64.2 / 57.8, 24 rows 58.4 / 59.1; 8192 x 28672 24.6 / 25.2).
 // 49-64 rows over a long K with many weights (13824 x 5120: 25.8 against 23.3 us) and AWQ beyond 32 rows
-// with the gated epilogue or a long K stay with the prefill kernels.
+// with the gated epilogue or a long K stay with the prefill kernels; so do 128-column tiles of which a few make a second
+// round, where either kernel rounds every weight (3584 x 37888, 296 tiles: AWQ 33 rows 36.4 / 32.3 us, 48 rows 37.9 / 34.6; bf16
+// GPTQ 49 rows 37.2 / 33.8).  AWQ on 2^28 weights and more up to 6 rows stays with the words-as-stored kernel (8192 x 57344, 5
+// rows 69.8 / 56.9 us, gated 72.9 / 60.4; 8 rows and more 0.92-1.06).
+// Slower than the kernel it took over from and kept, because the weights are unrounded here and rounded there: AWQ with 7 to 32
+// rows, 3584 x 37888 0.84-0.99, 8192 x 10240 0.85-0.98 (80 tiles: 160 workgroups); also 8192 x 10240 at 33-48 rows 0.91-0.96,
+// bf16 GPTQ 4096 x 28672 at 4-8 rows 0.96-0.97, fp16 1024 x 8192 at 49-64 rows 0.93-0.95.
 bool batch_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan) {
   if (M < 1 || M > 64 || !batch_supported(w, M, gate_up)) return false;
   const long weights = (long)w->K * w->N;
+  const bool second_round = w->N % 128 == 0 && w->N / 128 > 256 && w->N / 128 <= 320;
   if (w->layout == Q4_LAYOUT_AWQ) {
     if (M <= 4 && (gate_up || weights > (1L << 25))) return false;
-    if (M > 48 || (M > 32 && (gate_up || w->K > 8192))) return false;
+    if (M <= 6 && weights >= (1L << 28)) return false;
+    if (M > 48 || (M > 32 && (gate_up || w->K > 8192 || second_round))) return false;
   } else {
     if (gate_up && M <= 16 && weights >= (1L << 28)) return false;
     // (the kernels for a few rows are at their best from groups of 128 rows on)
     const bool short_groups = w->num_groups > 1 && w->groupsize < 128;
     if (dtype == Q4_DTYPE_F16 && !gate_up && M <= 4 && !short_groups) return false;
     if (dtype == Q4_DTYPE_BF16 && M <= 3 && weights >= (1L << 26) && !short_groups) return false;
-    if (M > 48 && w->K > 8192 && weights >= (1L << 26)) return false;
+    if (M > 48 && ((w->K > 8192 && weights >= (1L << 26)) || (second_round && !gate_up && dtype == Q4_DTYPE_BF16))) return false;
   }
   // (33 rows and more that the decode kernels would hold, which carry the scale to the sums: small matrices)
   const bool unrounded = M > 32 && q4_select_path(w, M, dtype) == Q4_PATH_GEMV;
