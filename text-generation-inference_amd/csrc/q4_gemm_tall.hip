@@ -74,12 +74,12 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
 //     often as two 128-row workgroups: 4096 x 28672 at 1400 and 2048 rows 0.93-0.96, 4096 x 12288 at 2048 0.92, gated 0.95,
 //     8192 x 57344 at 1400 0.96; 256-row tiles in 3.5-7 rounds 0.97-1.06
 //   GPTQ, 96-row tiles for more than 1024 rows: 4096 x 4096 and 3584 x 3584 at 1400 0.93-0.94; at 700 0.97-1.07
-//   AWQ, K of at most 16 K tiles, where start and epilogue count as much as the tiles in between: 1024 x 8192 at 1000
+//   AWQ, K of 9 to 16 K tiles (shorter ones not measured), where start and epilogue count as much as the tiles in between: 1024 x 8192 at 1000
 //     rows 0.90, gated bf16 at 512 to 1400 rows 0.86-1.02; up to 129 rows, in splits, 1.13-1.28, 256 x 256 tiles 1.20-1.34,
 //     gated fp16 0.97-1.08
 static bool tall_outdone(bool awq, int dtype, int M, int K, int N, bool gate_up, const TallPlan& plan) {
   if (plan.block) return false;
-  if (awq) return K <= 1024 && M > 384 && (!gate_up || dtype == Q4_DTYPE_BF16);
+  if (awq) return K > 512 && K <= 1024 && M > 384 && (!gate_up || dtype == Q4_DTYPE_BF16);
   const long tiles = (long)((M + 32 * plan.r - 1) / (32 * plan.r)) * (N / q4::kTallBN);
   return (plan.r < 8 && tiles >= 3 * 256) || (plan.r == 3 && !gate_up && M > 1024);
 }
