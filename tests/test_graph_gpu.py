@@ -67,8 +67,9 @@ def test_dense_paths_under_graph_replay(pkg, oracle, gpu):
 
     calls = [
         call(plain, 1), call(plain, 2),      # accumulation cells
-        call(plain, 8),                      # tickets
-        call(plain, 18),                     # two MFMA row blocks
+        call(plain, 8, path=1),              # accumulation cells, the rows dealt to the waves
+        call(plain, 18, path=1),             # two MFMA row blocks
+        call(plain, 8), call(plain, 40),     # exchange cells of the batch decode kernel
         call(plain, 40, path=2),             # split-K GEMM + reduction kernel
         call(plain, 300),
         call(seq, 1), call(seq, 8), call(seq, 300),   # fused gather, workspace gather, gather + GEMM
