@@ -85,7 +85,7 @@ int q4_dequant(const q4_weight* w, void* w_out, int dtype, void* stream);
  * server/text_generation_server/layers/awq/quantize/cuda.py:45-47).
  *
  * workspace: device buffer of at least q4_workspace_bytes(M, K, N) bytes whose first
- * Q4_WORKSPACE_COUNTER_BYTES bytes (split-K tickets, then fixed-point accumulation cells)
+ * Q4_WORKSPACE_COUNTER_BYTES bytes (split-K tickets, then the cells in which partial sums meet)
  * were zero before the first call that used it; the kernels leave them zero again.  The
  * rest holds fp32 partial sums and needs no initialisation.  Calls that share a workspace
  * must be ordered on one stream.
@@ -117,10 +117,11 @@ int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);
  * `gate_up_proj(x)` followed by `act(gate_up[:, 0]) * gate_up[:, 1]`
  * (server/text_generation_server/models/custom_modeling/flash_llama_modeling.py:400-404;
  * the reference fuses this only for unquantized ROCm decode, `ops.LLMM_Silu`, :378-397).
- * Fused in the decode kernel of the GPTQ layout with contiguous groups.  Returns
- * Q4_ERR_UNSUPPORTED otherwise (AWQ layout, g_idx, odd shapes, and M large enough for the
- * prefill GEMM, where the separate elementwise pass is the faster route): the caller then
- * runs q4_linear into an [M, N] buffer and q4_act_mul.
+ * Runs for contiguous groups, either layout, in the kernels that q4_linear_kernel(w, M, dtype, 1) names: up to 64
+ * rows the batch decode kernel (AWQ from five rows on; groups it does not take: the GPTQ decode kernel, one or
+ * two rows), above the prefill kernels.  Returns Q4_ERR_UNSUPPORTED where that answer is Q4_PATH_AUTO (g_idx, few
+ * AWQ rows, odd shapes, some sizes where the two launches measured faster): the caller then runs q4_linear into an
+ * [M, N] buffer and q4_act_mul.
  */
 #define Q4_ACT_SILU 0       /* x * sigmoid(x) */
 #define Q4_ACT_GELU_TANH 1  /* gelu(approximate="tanh"): "gelu_fast", "gelu_pytorch_tanh" */
@@ -252,7 +253,9 @@ size_t q4_gemv_tuned_workspace_bytes(const q4_weight* w, int M, int dtype, int w
  * (temp_dq_size / temp_fwd_size / scratch_space_fixed).
  */
 #define Q4_WORKSPACE_TICKET_BYTES 16384   /* split-K arrival tickets, one per column tile */
-#define Q4_WORKSPACE_CELL_BYTES 4194304   /* 64-bit fixed-point accumulation cells (fp16 decode: 16 rows x 32768 columns) */
+/* 64-bit cells: fixed-point accumulation (fp16 decode: 16 rows x 32768 columns), or two fp32 partial sums that wait for
+ * their partner's (batch decode kernel) */
+#define Q4_WORKSPACE_CELL_BYTES 4194304
 #define Q4_WORKSPACE_COUNTER_BYTES 4210688 /* = tickets + cells: the part that must start zero */
 size_t q4_workspace_bytes(int M, int K, int N);
 /*
@@ -331,16 +334,17 @@ int q4_moe_route_grouped(const void* gating, int gating_dtype, int tokens, int e
                          int32_t* sorted_tokens, int32_t* pair_slot, int32_t* expert_offsets, void* stream);
 
 /* y[r, :] = x[x_rows ? x_rows[r] : r, :] @ W_e for every sorted row r of every expert e.
- * y is [tokens*topk, N] in sorted order.  Up to 16 tokens (64 when K <= 8192) the decode
- * kernel runs once per expert and 16 rows it received; above, the MFMA kernel.  Workspace as for q4_linear, sized by
- * q4_moe_workspace_bytes, zero-initialised once. */
+ * y is [tokens*topk, N] in sorted order.  GPTQ weights with contiguous groups run on the batch decode kernel while an
+ * expert receives up to 48 rows on average; otherwise (AWQ, g_idx, groups it does not take) up to 16 tokens (64 when
+ * K <= 8192 and the groups are contiguous GPTQ) the decode kernel runs once per expert and 16 rows it received, above
+ * the MFMA kernel.  Workspace as for q4_linear, sized by q4_moe_workspace_bytes, zero-initialised once. */
 int q4_moe_linear(const q4_moe_weight* w, const void* x, const int32_t* x_rows, const int32_t* expert_offsets,
                   void* y, int tokens, int topk, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* First projection with the gated-MLP epilogue: every expert's W packs [gate | up] along N and
  * y[r, :] = act(x_r @ gate_e) * (x_r @ up_e), [tokens*topk, N/2] in sorted order.  One launch
- * where the fused decode kernel applies (one token, GPTQ layout with contiguous groups
- * of at least 128 rows); Q4_ERR_UNSUPPORTED otherwise -- then q4_moe_linear + q4_act_mul. */
+ * where the batch decode kernel takes the problem (see q4_moe_linear), or the GPTQ decode kernel for one token (groups
+ * in whole 128-row chunks); Q4_ERR_UNSUPPORTED otherwise -- then q4_moe_linear + q4_act_mul. */
 int q4_moe_linear_gate_up(const q4_moe_weight* w, const void* x, const int32_t* x_rows, const int32_t* expert_offsets,
                           void* y, int tokens, int topk, int dtype, int act, void* workspace, size_t workspace_bytes,
                           void* stream);

@@ -68,7 +68,8 @@ bool gemv_gate_up_supported(const q4_weight* w, int M, int dtype) {
   // kernel followed by the elementwise kernel: 16.1 / 18.2 us at M = 1, 17.2 / 18.4 us at
   // M = 2, 19.6 / 19.3 us at M = 4, 26.0 / 22.4 us at M = 8 (the fused workgroups are twice
   // as wide and stage twice the activation slab), so the fused kernel is offered for one and
-  // two rows.
+  // two rows.  By the library's own choice it runs where the batch decode kernel does not apply: fewer
+  // than four chunks of K, groups of 384, 640 .. rows (below 2^28 weights).
   return w->layout == Q4_LAYOUT_GPTQ && w->g_idx == nullptr && w->groupsize >= 128 && w->N % 128 == 0 &&
          M <= 2 && gemv_supported(w, M, dtype);
 }

@@ -1,6 +1,7 @@
 // Decode kernel instantiations with the gated-MLP epilogue (act(x @ gate) * (x @ up)), kept in
 // their own translation unit so that they compile in parallel with the plain ones.  The
-// launcher offers them for one and two activation rows only (grouped launches: tokens).
+// launcher offers them for one and two activation rows only (grouped launches: one token), and the batch decode
+// kernel (q4_gemv_batch.cuh) takes most of those: these serve the weights that it refuses.
 #include "q4_gemv_kernels.cuh"
 
 namespace q4host {

@@ -234,6 +234,8 @@ struct MoeGemvPlan {
   size_t slab_bytes, smem;
 };
 
+// (GPTQ weights with contiguous groups come here only where the batch decode kernel does not take them: other
+// groups and shapes, more than 48 rows per expert.)
 // The decode kernel takes 16 rows of an expert per workgroup; an expert can receive every
 // token, so the grid has ceil(tokens / 16) row blocks per expert, of which those past the
 // expert's count leave at once.  Each further block of an expert re-reads its weights (from

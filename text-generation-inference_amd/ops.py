@@ -470,9 +470,10 @@ def _launch_linear(w, x, bias, y, M, code, path, gemv_config, dev, out_given) ->
 def apply_linear(w: PackedWeight, x: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """The forward of a linear module: x [..., K] -> [..., N], nothing recorded for autograd.
 
-    A call for a few tokens is bound by the host (one projection 4096 x 4096 for one token: kernel 4.3 us, call
-    11.3 us), so nothing here is done that such a call does not need: a rank-two x is taken as it is, and grad mode is
-    only left where something would be recorded (as a decorator on forward no_grad costs about 2 us)."""
+    A call for a few tokens is bound by the host (one projection 4096 x 4096 for one token: the kernel takes 4.3 us, the
+    call 7.6, and 11.4 before it was shortened as follows), so nothing here is done that such a call does not need: a
+    rank-two x is taken as it is, and grad mode is only left where something would be recorded (as a decorator on forward
+    no_grad costs about 2 us)."""
     if (x.requires_grad or (bias is not None and bias.requires_grad)) and torch.is_grad_enabled():
         with torch.no_grad():
             return apply_linear(w, x, bias)
@@ -623,9 +624,10 @@ def linear_gate_up(
 ) -> torch.Tensor:
     """y[M, N/2] = act(x @ W[:, :N/2]) * (x @ W[:, N/2:]) for a weight that packs [gate | up].
 
-    One launch where a fused kernel covers the weight (GPTQ layout with contiguous groups);
-    otherwise the linear kernel followed by the elementwise act_mul kernel.  `fused`
-    forces one of the two (True raises if there is no fused kernel).
+    One launch where a fused kernel covers the weight and row count and measured faster (contiguous groups of
+    either layout: decode batches and prefill; act-order where the call regroups the rows); otherwise the linear
+    kernel followed by the elementwise act_mul kernel.  `fused` forces one of the two (True raises if there is no
+    fused kernel).
     """
     _require_cuda(x, "x")
     _require_cuda(w.qweight, "qweight")
@@ -884,7 +886,7 @@ def moe_linear(w: PackedMoeWeight, x: torch.Tensor, routing: MoeRouting, gather:
 def moe_linear_gate_up(w: PackedMoeWeight, x: torch.Tensor, routing: MoeRouting, act: str = "silu") -> torch.Tensor:
     """First projection of the experts with the gated-MLP tail: sorted row r becomes
     act(x[token(r)] @ gate_e) * (x[token(r)] @ up_e), [tokens*k, N/2].  One fused launch where
-    the decode kernel offers it (one token), else grouped linear + act_mul."""
+    the library offers it (GPTQ experts with up to 48 rows each on average), else grouped linear + act_mul."""
     _require_cuda(x, "x")
     if x.dtype not in _DTYPES:
         raise TypeError(f"x must be float16 or bfloat16, got {x.dtype}")
