@@ -529,22 +529,24 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
   // (uneven groups then cost what they always did)
   if (q4_select_path(w, M, dtype) != Q4_PATH_GEMM) return 0;
   // Sorting g_idx (3 us), the pass over the weights (8192 x 57344 131 us, 4096 x 4096 7), the gather of x and the
-  // launches that end at the flag (3-7 us) come back as rows and weights multiply; the kernels that read through g_idx
-  // hold row blocks of 128 and 256, in which they are flat in M.  Time through g_idx over time regrouped, MI355X, 23
-  // layer shapes, groups of 32 to 128, 17 row counts, both data types, plain and gated:
+  // launches that end at the flag (3-7 us) come back as rows and weights multiply; the kernels that read through g_idx hold
+  // row blocks of 128 and 256, in which they are flat in M.  Time through g_idx over time regrouped, MI355X, 19
+  // layer shapes, fp16, groups of 32 to 128, 26 row counts from 129 on, plain and gated (geometric mean; least, most of what is taken):
   //   33-64 rows    the batch decode kernel on the copy: 8192 x 57344 1.14-1.30; 4096 x 28672 0.94-1.06, 3584 x 37888
   //                 0.91-1.05, narrower ones down to 0.6
-  //   N >= 2 K      4096 x 22016 .. 8192 x 57344: 129-192 rows 1.02-1.66, from 320 on 1.06-1.70; 193-256 rows 0.95-1.08
-  //                 below 1.3e8 weights, 1.03-1.40 above; 4096 x 12288 from 320 rows on 0.99-1.46, below 0.89-1.08
-  //   other shapes  from 6e10 rows x weights on 1.00-1.77 (28672 x 8192 at 256 rows, 6e10, 0.89: from 320 on), below
-  //                 0.66-1.48 (13824 x 5120 at 768 0.94, 4096 x 4096 at 1024 0.91); 1536 rows and more 1.04-1.50 from 2.5e7
-  //                 weights on, 4096 x 4096 0.97-1.10
-  //   no table      (too many groups for LDS) 129 rows and more, 14336 x 4096 1.14-2.08, 28672 x 8192 0.99-2.15
+  //   no table      (too many groups for LDS) 1.53 (1.01, 2.39); 8192 x 1280 0.66-0.92 up to 512 rows
+  //   129-256 rows  1.28 (1.06, 1.64); 4096 x 12288 0.88-1.17, 8192 x 8192 0.89-1.03, 8192 x 10240 1.14 at 129, 0.94 at
+  //                 256; 4096 x 22016 and 28672 at 193-256 1.04-1.20, but bf16 layers 0.93-0.96 of their speed
+  //   257-512       1.31 (0.95, 1.68); 14336 x 4096 1.18-1.31 up to 320 and 0.92 at 512; 3584 x 8192 0.85-1.00
+  //   513 and more  1.26 (0.96, 1.71); 4096 x 6144 0.91-0.97 up to 640; 4096 x 4096 0.92-1.07 up to 1024, 1024 x 8192
+  //                 0.74-1.02
   const double weights = (double)w->K * w->N;
+  const bool wide = w->N / 2 >= w->K;
   if (M <= 128) return M >= Q4_REGROUP_MIN_ROWS && M <= 64 && w->N / 4 >= w->K && weights >= 2.6e8;
-  if (!gemm_act_order_table(w)) return weights >= 5e7;
-  if (w->N / 2 >= w->K && weights >= (M >= 320 ? 5e7 : (M <= 192 ? 8.5e7 : 1.3e8))) return 1;
-  return (M >= 320 && M * weights >= 6e10) || (M >= 1536 && weights >= 2.4e7);
+  if (!gemm_act_order_table(w)) return weights >= 4e7 || (M > 512 && weights >= 1e7);
+  if (M <= 256) return weights >= (M <= 192 ? 8e7 : 1.3e8) && (wide || (w->N >= w->K && M <= 160));
+  if (M <= 512) return weights >= 1e8 || (weights >= 4e7 && (wide || M <= 352));
+  return weights >= (M > 1024 ? 1.25e7 : (M > 640 ? 2.4e7 : 4e7));
 }
 
 int q4_linear_regroup(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
