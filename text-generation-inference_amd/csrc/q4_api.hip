@@ -538,7 +538,7 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
   //   129-256 rows  1.28 (1.06, 1.64); 4096 x 12288 0.88-1.17, 8192 x 8192 0.89-1.03, 8192 x 10240 1.14 at 129, 0.94 at
   //                 256; 4096 x 22016 and 28672 at 193-256 1.04-1.20, but bf16 layers 0.93-0.96 of their speed
   //   257-512       1.31 (0.95, 1.68); 14336 x 4096 1.18-1.31 up to 320 and 0.92 at 512; 3584 x 8192 0.85-1.00
-  //   513 and more  1.26 (0.96, 1.71); 4096 x 6144 0.91-0.97 up to 640; 4096 x 4096 0.92-1.07 up to 1024, 1024 x 8192
+  //   513 and more  1.26 (0.91: 3584 x 3584 at 1025, 1.71); 4096 x 6144 0.91-0.97 up to 640; 4096 x 4096 0.92-1.07 up to 1024, 1024 x 8192
   //                 0.74-1.02
   const double weights = (double)w->K * w->N;
   const bool wide = w->N / 2 >= w->K;
