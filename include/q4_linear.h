@@ -335,7 +335,7 @@ int q4_moe_route_grouped(const void* gating, int gating_dtype, int tokens, int e
 
 /* y[r, :] = x[x_rows ? x_rows[r] : r, :] @ W_e for every sorted row r of every expert e.
  * y is [tokens*topk, N] in sorted order.  GPTQ weights with contiguous groups run on the batch decode kernel while an
- * expert receives up to 48 rows on average; otherwise (AWQ, g_idx, groups it does not take) up to 16 tokens (64 when
+ * expert receives up to 48 rows on average (small experts: 5 or 16); otherwise (AWQ, g_idx, groups it does not take) up to 16 tokens (64 when
  * K <= 8192 and the groups are contiguous GPTQ) the decode kernel runs once per expert and 16 rows it received, above
  * the MFMA kernel.  Workspace as for q4_linear, sized by q4_moe_workspace_bytes, zero-initialised once. */
 int q4_moe_linear(const q4_moe_weight* w, const void* x, const int32_t* x_rows, const int32_t* expert_offsets,
@@ -355,6 +355,8 @@ int q4_moe_combine(const void* y_sorted, const float* topk_weights, const int32_
                    int tokens, int topk, int N, int dtype, void* stream);
 
 size_t q4_moe_workspace_bytes(const q4_moe_weight* w, int tokens, int topk);
+/* q4_linear_kernel for q4_moe_linear (gate_up = 0) and q4_moe_linear_gate_up (1); Q4_PATH_AUTO where none takes it. */
+int q4_moe_kernel(const q4_moe_weight* w, int tokens, int topk, int dtype, int gate_up);
 
 /* The Q4_PATH_* value q4_linear would take for this problem (negative on bad arguments). */
 int q4_select_path(const q4_weight* w, int M, int dtype);

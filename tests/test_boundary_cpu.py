@@ -241,6 +241,19 @@ def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, w
     assert pkg._lib.KERNEL_NAMES[rc] == want
 
 
+@pytest.mark.parametrize("E,topk,K,N,tokens,gate_up,want", [
+    (8, 2, 4096, 28672, 192, 1, "batch"), (8, 2, 14336, 4096, 192, 0, "batch"), (8, 2, 14336, 4096, 193, 0, "gemm"),
+    (64, 6, 1408, 2048, 48, 0, "batch"), (64, 6, 1408, 2048, 64, 0, "gemv"), (64, 6, 1408, 2048, 192, 0, "gemm"),
+    (64, 6, 2048, 2816, 170, 1, "batch"), (64, 6, 2048, 2816, 192, 1, "none"),
+    (16, 4, 4096, 2048, 64, 0, "batch"), (16, 4, 4096, 2048, 128, 0, "gemm"), (16, 4, 2048, 8192, 192, 1, "batch"),
+])
+def test_the_kernel_of_a_grouped_call(pkg, E, topk, K, N, tokens, gate_up, want):
+    lib, L = pkg._lib.load(), pkg._lib
+    w = L.Q4MoeWeight(_weight(pkg, K, N, 128), E, K * N // 8, K * N // 1024, K * N // 128, 0)
+    for dtype in (0, 1):
+        assert L.KERNEL_NAMES[lib.q4_moe_kernel(ctypes.byref(w), tokens, topk, dtype, gate_up)] == want
+
+
 def test_path_selection_and_workspace(pkg):
     lib = pkg._lib.load()
     L = pkg._lib

@@ -130,6 +130,7 @@ SIGNATURES = {
         [POINTER(Q4MoeWeight), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p],
     ),
     "q4_moe_combine": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    "q4_moe_kernel": (c_int, [POINTER(Q4MoeWeight), c_int, c_int, c_int, c_int]),
     "q4_moe_workspace_bytes": (c_size_t, [POINTER(Q4MoeWeight), c_int, c_int]),
 }
 

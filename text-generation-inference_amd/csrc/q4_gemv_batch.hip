@@ -198,6 +198,13 @@ static int batch_moe_blocks(int num_experts, int pairs) {
 // MFMA tiles, reduction and elementwise launch) / this one: first projection with its activation 1 token
 // 27.0 / 26.1, 16 tokens 111 / 82, 48 146 / 98, 64 194 / 101, 128 156 / 123, 256 (64 rows each) 232 / 229;
 // second 1 18.7 / 15.2, 16 76 / 40, 48 70 / 48, 64 73 / 47, 128 86 / 58, 256 112 / 111.
+// Small experts (2.5e6 weights and more; below not measured) end earlier: the workgroups of a split or of a further row block cost more than the weights they share.  Theirs
+// / this one, us, fp16: second projection of 64 experts, 1408 x 2048, top-6: 48 tokens 27.6 / 21.9, 64 29.1 / 31.8, 128 40 / 46,
+// 192 35 / 50; of 16 experts, 4096 x 2048, top-4: 64 tokens 36 / 32, 128 32 / 38, 192 35 / 46; first projection of the 64
+// experts, gated: 128 tokens 69 / 54, 192 59 / 60, 384 73 / 84.
+// Uneven routing (router logits rising by 3 over the experts, where the busiest expert meets two to three times the average): the
+// second projection above at 128 tokens 0.95 in fp16, 0.88 in bf16, at 192 0.91 and 0.83, with four experts at 48 and 64
+// tokens 0.70-0.87 (even 1.2-1.4); first projections 0.98 and more.
 static bool batch_moe_plan(const q4_moe_weight* w, int tokens, int pairs, bool gate_up, BatchPlan* plan) {
   const q4_weight* e0 = &w->expert0;
   return batch_plan(e0, pairs, batch_moe_blocks(w->num_experts, pairs), pairs < w->num_experts ? pairs : w->num_experts, gate_up,
@@ -208,6 +215,11 @@ bool batch_moe_default(const q4_moe_weight* w, int tokens, int topk, bool gate_u
   const long pairs = (long)tokens * topk;
   const q4_weight* e0 = &w->expert0;
   if (e0->layout != Q4_LAYOUT_GPTQ || tokens < 1 || pairs > 48L * w->num_experts || w->num_experts > 65535) return false;
+  const long weights = (long)e0->K * e0->N;
+  if (weights >= 2500000) {
+    if (!gate_up && weights < 10000000 && pairs > (e0->K < 2048 ? 5L : 16L) * w->num_experts) return false;
+    if (gate_up && weights < (1L << 23) && pairs > 16L * w->num_experts) return false;
+  }
   const long row_blocks = (tokens + 15) / 16;
   BatchPlan plan;
   return row_blocks * 8 <= 65535 && batch_supported(e0, (int)pairs, gate_up) && batch_moe_plan(w, tokens, (int)pairs, gate_up, &plan);

@@ -671,6 +671,20 @@ int q4_moe_combine(const void* y_sorted, const float* topk_weights, const int32_
   return Q4_OK;
 }
 
+int q4_moe_kernel(const q4_moe_weight* w, int tokens, int topk, int dtype, int gate_up) {
+  int rc = validate_moe_weight(w, "q4_moe_kernel");
+  if (rc != Q4_OK) return rc;
+  if ((dtype != Q4_DTYPE_F16 && dtype != Q4_DTYPE_BF16) || tokens < 1 || topk < 1 || topk > q4::kMoeMaxTopk ||
+      (long)tokens * topk > 0x7fffffffL) {
+    set_error("q4_moe_kernel: dtype=%d tokens=%d topk=%d", dtype, tokens, topk);
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
+  if (batch_moe_default(w, tokens, topk, gate_up != 0)) return Q4_KERNEL_BATCH;
+  if (moe_gemv_plan(w, tokens, topk, dtype, gate_up != 0).ok) return Q4_PATH_GEMV;
+  const bool gemm = moe_gemm_ok(&w->expert0, tokens, topk, dtype) || gemm_awq_supported(&w->expert0, tokens, dtype);
+  return !gate_up && gemm ? Q4_PATH_GEMM : Q4_PATH_AUTO;
+}
+
 size_t q4_moe_workspace_bytes(const q4_moe_weight* w, int tokens, int topk) {
   if (validate_moe_weight(w, "q4_moe_workspace_bytes") != Q4_OK || tokens < 0 || topk < 1) return 0;
   return moe_workspace_bytes(w, tokens, topk);
