@@ -204,7 +204,8 @@ static int batch_moe_blocks(int num_experts, int pairs) {
 // experts, gated: 128 tokens 69 / 54, 192 59 / 60, 384 73 / 84.
 // Uneven routing (router logits rising by 3 over the experts, where the busiest expert meets two to three times the average): the
 // second projection above at 128 tokens 0.95 in fp16, 0.88 in bf16, at 192 0.91 and 0.83, with four experts at 48 and 64
-// tokens 0.70-0.87 (even 1.2-1.4); first projections 0.98 and more.
+// tokens 0.70-0.87 (even 1.2-1.4), of eight experts 5632 x 2048 at 128 and 192 0.73-0.82 (even 1.07-1.23); first projections 0.96
+// and more, of small experts 0.89.  The host does not know the routing.
 static bool batch_moe_plan(const q4_moe_weight* w, int tokens, int pairs, bool gate_up, BatchPlan* plan) {
   const q4_weight* e0 = &w->expert0;
   return batch_plan(e0, pairs, batch_moe_blocks(w->num_experts, pairs), pairs < w->num_experts ? pairs : w->num_experts, gate_up,
