@@ -176,9 +176,9 @@ def test_weights_of_few_experts_are_not_rounded(pkg, oracle, gpu, T, E, dtype):
                                           ("gptq", 1024, 32768, 20), ("awq", 2048, 512, 4), ("awq", 4096, 512, 24)])
 @pytest.mark.parametrize("kind", ["dc_offset", "one_sign", "outliers", "small", "silu_product"])
 def test_bf16_off_distribution(pkg, oracle, gpu, layout, K, N, M, kind):
-    """bf16 sums with 128 + q, from which (128 + z) sum(x) is taken, on activations whose sum is far from zero.  Against 64-bit
-    sums with unrounded weights an output is off by its own rounding (8 significant bits: 2^-8 of it), and by fp32 sums of terms up to |x| 143 scale,
-    of which a group's 128 pass 4 MFMA of 32 and K / 128 groups follow: 4 + 32 + K / 128 roundings of 2^-24 of their sum."""
+    """bf16 sums of the exact integers q - z on activations whose sum is far from zero.  Against 64-bit sums with unrounded weights
+    an output is off by its own rounding (8 significant bits: 2^-8 of it), and by fp32 sums of the terms x (q - z) scale, of which a
+    stage's 64 pass two MFMA of 32 and K / 64 stages follow: 2 + 32 + K / 64 roundings of 2^-24 of the terms' sum."""
     from tests.test_offdist_gpu import make_activations
 
     gs = 128 if K % 256 == 0 else 64
@@ -192,9 +192,41 @@ def test_bf16_off_distribution(pkg, oracle, gpu, layout, K, N, M, kind):
     x = torch.from_numpy(make_activations(kind, M, K, M)).to(gpu).bfloat16()
     got = pkg.ops.linear(pk, x).double()
     scale = torch.from_numpy(np.repeat(sc.astype(np.float64), gs, axis=0)).to(gpu)
-    want = x.double() @ (torch.from_numpy(np.asarray(ints).astype(np.float64)).to(gpu) * scale)
-    terms = x.double().abs() @ (143.0 * scale.abs())
-    assert bool(((got - want).abs() <= 2.0**-8 * want.abs() + (36 + K // 128) * 2.0**-24 * terms).all())
+    w = torch.from_numpy(np.asarray(ints).astype(np.float64)).to(gpu) * scale
+    want, terms = x.double() @ w, x.double().abs() @ w.abs()
+    assert bool(((got - want).abs() <= 2.0**-8 * want.abs() + (34 + K // 64) * 2.0**-24 * terms).all())
+
+
+@pytest.mark.parametrize("layout", ["gptq", "awq"])
+@pytest.mark.parametrize("gs,M", [(128, 3), (128, 32), (64, 13), (32, 13)])
+@pytest.mark.parametrize("value", [2.0**30, 2.39e36])
+def test_bf16_sums_meet_x_times_weight_alone(pkg, oracle, gpu, layout, gs, M, value):
+    """A large activation under weights that are zero, but for one column: nothing of it may reach the other sums, and its product,
+    finite in fp32, stays finite.  Bound as above; the large row's term is zero where its weight is."""
+    K, N = 1024, 512
+    if layout == "awq":
+        qw, qz, sc = oracle.make_awq(K, N, gs, seed=M)
+        q, z = oracle.awq_unpack_cols(qw), oracle.awq_unpack_cols(qz)
+        z[300 // gs] = 8
+        q[300], q[300, 77] = 8, 15
+        qw, qz = oracle.awq_pack_cols(q), oracle.awq_pack_cols(z)
+        ints = oracle.dequant_awq(qw, qz, np.ones_like(sc), gs, "f16")
+    else:
+        qw, qz, sc, _ = oracle.make_gptq(K, N, gs, seed=M, sym=True)
+        q = oracle.unpack_rows(qw)
+        q[300], q[300, 77] = 8, 15
+        qw = oracle.pack_rows(q)
+        ints = oracle.dequant_gptq(qw, qz, np.ones_like(sc), None, gs, "f16")
+    pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), None, gs, 1 if layout == "awq" else 0)
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16) == "batch"
+    x = to_dev(oracle.make_x(M, K, seed=M, dtype="bf16"), gpu, bf16=True)
+    x[1, 300] = value
+    got = pkg.ops.linear(pk, x).double()
+    w = torch.from_numpy(np.asarray(ints).astype(np.float64) * np.repeat(sc.astype(np.float64), gs, axis=0)).to(gpu)
+    assert int((w[300] != 0).sum()) == 1
+    want, terms = x.double() @ w, x.double().abs() @ w.abs()
+    assert bool(torch.isfinite(got).all())
+    assert bool(((got - want).abs() <= 2.0**-8 * want.abs() + (34 + K // 32) * 2.0**-24 * terms).all())
 
 
 @pytest.mark.parametrize("layout,K,N,gs", [("gptq", 4096, 256, 128), ("gptq", 1152, 192, 64), ("gptq", 1024, 32768, 128), ("awq", 4096, 512, 128)])
@@ -220,9 +252,9 @@ def test_bf16_non_finite_rows_stay_alone(pkg, oracle, gpu, layout, K, N, gs, M):
 
 @pytest.mark.parametrize("K,N,M", [(8192, 8192, 1), (16384, 4096, 3), (8192, 8192, 2)])
 def test_bf16_few_rows_on_large_layers(pkg, oracle, gpu, K, N, M):
-    """One to three bf16 rows on 2^26 weights and more that are not wide, plain and with the gated epilogue."""
+    """One to three bf16 rows on 2^26 weights and more, plain and gated: the decode kernels'."""
     pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, 128, M, "bf16")
-    assert pkg.ops.kernel_of(pk, M, torch.bfloat16) == "batch" and pkg.ops.kernel_of(pk, M, torch.bfloat16, True) == "batch"
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16) == "gemv" and pkg.ops.kernel_of(pk, M, torch.bfloat16, True) == ("none" if M == 3 else "gemv")
     x = oracle.make_x(M, K, seed=M, dtype="bf16")
     y32, _ = oracle.linear_forward(x, w, None, "bf16")
     assert max_rel_err(to_f32(pkg.ops.linear(pk, to_dev(x, gpu, bf16=True))), y32) <= TOL["bf16"]
