@@ -344,6 +344,23 @@ def test_no_cpu_fallback(pkg, oracle):
         lin.dequantize()
 
 
+def test_nested_activations_raise(pkg, oracle):
+    """Tensors whose sizes throw come back as a Python error (in a process of their own: what a C++ exception ends is the process)."""
+    import subprocess
+    import sys
+
+    code = (
+        "import importlib, torch, warnings; warnings.simplefilter('ignore')\n"
+        "pkg = importlib.import_module('text-generation-inference_amd')\n"
+        "i = lambda *s: torch.zeros(s, dtype=torch.int32)\n"
+        "pk = pkg.ops.make_packed(i(32, 64), i(2, 8), torch.ones(2, 64, dtype=torch.float16), None, 128, 0)\n"
+        "x = torch.nested.nested_tensor([torch.zeros(2, 256), torch.zeros(3, 200)], dtype=torch.float16)\n"
+        "try:\n    pkg.ops.apply_linear(pk, x, None)\nexcept RuntimeError:\n    print('raised')\n"
+    )
+    got = subprocess.run([sys.executable, "-c", code], cwd=HEADER.parent.parent, capture_output=True, text=True, timeout=300)
+    assert got.returncode == 0 and got.stdout.strip() == "raised", got.stderr[-2000:]
+
+
 def test_make_packed_validation(pkg, oracle):
     qw, qz, sc, gi = _cpu_gptq_tensors(oracle, act_order=True)
     mk = pkg.ops.make_packed

@@ -58,12 +58,12 @@ bool watched() {
   return c10::impl::tls_local_dispatch_key_set().included_.has_any(kTransforms);
 }
 
-// a dense tensor of this GPU that operators would meet as it is
+// a dense tensor of this GPU that operators would meet as it is; asked before anything else of a tensor (sizes of a nested one throw)
 bool plain(const at::Tensor& t, int device) {
   const c10::DispatchKeySet odd({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                  c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
-                                 c10::DispatchKey::ZeroTensor});
-  return t.is_cuda() && t.layout() == c10::kStrided && t.get_device() == device && !t.key_set().has_any(odd) && t.is_contiguous();
+                                 c10::DispatchKey::ZeroTensor, c10::DispatchKey::NestedTensor, c10::DispatchKey::AutogradNestedTensor});
+  return t.is_cuda() && t.layout() == c10::kStrided && !t.key_set().has_any(odd) && t.get_device() == device && t.is_contiguous();
 }
 
 // An integer of a tuple.
@@ -88,13 +88,13 @@ PyObject* call(Call* self, PyObject* x_obj, PyObject* bias_obj, PyObject* owner)
   const at::Tensor& x = THPVariable_Unpack(x_obj);
   const q4_weight& w = self->weight;
   const auto type = x.scalar_type();
-  if ((type != at::kHalf && type != at::kBFloat16) || x.dim() < 2 || x.size(-1) != w.K || !plain(x, self->device)) Py_RETURN_NONE;
+  if ((type != at::kHalf && type != at::kBFloat16) || !plain(x, self->device) || x.dim() < 2 || x.size(-1) != w.K) Py_RETURN_NONE;
   if (x.requires_grad() && c10::GradMode::is_enabled()) Py_RETURN_NONE;
   const void* bias = nullptr;
   if (bias_obj != Py_None) {
     if (!THPVariable_Check(bias_obj)) Py_RETURN_NONE;
     const at::Tensor& b = THPVariable_Unpack(bias_obj);
-    if (b.scalar_type() != type || b.numel() != w.N || !plain(b, self->device) || (b.requires_grad() && c10::GradMode::is_enabled()))
+    if (b.scalar_type() != type || !plain(b, self->device) || b.numel() != w.N || (b.requires_grad() && c10::GradMode::is_enabled()))
       Py_RETURN_NONE;
     bias = b.const_data_ptr();
   }
@@ -132,15 +132,10 @@ PyObject* call(Call* self, PyObject* x_obj, PyObject* bias_obj, PyObject* owner)
   const at::Tensor workspace = THPVariable_Unpack(ws_obj);  // (its own reference: the dict may change while the lock is released)
   if (workspace.numel() < need) Py_RETURN_NONE;
 
-  at::Tensor y;
+  c10::SmallVector<int64_t, 4> sizes(x.sizes().begin(), x.sizes().end());
+  sizes.back() = w.N;
+  at::Tensor y = at::empty(sizes, x.options());
   int rc;
-  try {
-    c10::SmallVector<int64_t, 4> sizes(x.sizes().begin(), x.sizes().end());
-    sizes.back() = w.N;
-    y = at::empty(sizes, x.options());
-  } catch (...) {
-    Py_RETURN_NONE;  // out of memory, say: the Python code meets it again and raises
-  }
   void* ws = workspace.data_ptr();
   void* yp = y.data_ptr();
   const size_t ws_bytes = (size_t)workspace.numel();
@@ -170,7 +165,12 @@ PyObject* call_vector(PyObject* self, PyObject* const* args, size_t nargsf, PyOb
     return nullptr;
   }
   Py_INCREF(self);  // (the lock is released during the launch)
-  PyObject* y = call((Call*)self, args[0], args[1], count == 3 ? args[2] : nullptr);
+  PyObject* y;
+  try {
+    y = call((Call*)self, args[0], args[1], count == 3 ? args[2] : nullptr);
+  } catch (...) {  // out of memory, say: no exception may leave a C function, and the Python code meets the cause again and raises
+    y = PyErr_Occurred() ? nullptr : Py_NewRef(Py_None);
+  }
   Py_DECREF(self);
   return y;
 }
