@@ -344,6 +344,20 @@ def test_no_cpu_fallback(pkg, oracle):
         lin.dequantize()
 
 
+@pytest.mark.parametrize("layout,g_idx", [(0, False), (0, True), (1, False)])
+def test_weights_on_another_gpu_are_refused(pkg, monkeypatch, layout, g_idx):
+    """Nothing is launched with the addresses of two GPUs (stand-ins for the tensors: there are no two here)."""
+    from types import SimpleNamespace
+
+    at = lambda i, **kw: SimpleNamespace(is_cuda=True, device=torch.device("cuda", i), data_ptr=lambda: 0x1000, **kw)  # noqa: E731
+    x = at(1, dtype=torch.float16, shape=(4, 4096), dim=lambda: 2, is_contiguous=lambda: True)
+    w = pkg.ops.PackedWeight(at(0), at(0), at(0), at(0) if g_idx else None, 4096, 8192, 128, 32, layout)
+    monkeypatch.setattr(pkg.ops, "_launch_linear", lambda *a: pytest.fail("launched"))
+    for call in (pkg.ops.linear, pkg.ops.linear_gate_up):
+        with pytest.raises(RuntimeError, match="weights on cuda:0"):
+            call(w, x)
+
+
 def test_nested_activations_raise(pkg, oracle):
     """Tensors whose sizes throw come back as a Python error (in a process of their own: what a C++ exception ends is the process)."""
     import subprocess

@@ -649,6 +649,8 @@ def linear_gate_up(
     """
     _require_cuda(x, "x")
     _require_cuda(w.qweight, "qweight")
+    if x.device != w.qweight.device:
+        raise RuntimeError(f"x is on {x.device}, weights on {w.qweight.device}")
     if x.dtype not in _DTYPES:
         raise TypeError(f"x must be float16 or bfloat16, got {x.dtype}")
     if x.dim() != 2 or x.shape[1] != w.K:
