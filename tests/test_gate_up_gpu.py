@@ -163,6 +163,24 @@ def test_unfused_fallback(pkg, oracle, gpu, layout, act_order, M):
         _case(pkg, oracle, gpu, 2048, 1024, 128, M, layout=layout, act_order=act_order, fused=True, seed=M + 20)
 
 
+@pytest.mark.parametrize("layout,act_order,K,N,gs,dtype", [("gptq", True, 1024, 512, 128, "f16"), ("awq", False, 8192, 4352, 128, "bf16"),
+                                                           ("gptq", False, 1024, 512, 32, "f16"), ("gptq", False, 1024, 512, 128, "bf16")])
+def test_output_at_any_address(pkg, oracle, gpu, layout, act_order, K, N, gs, dtype):
+    """An `out` off a 16-byte boundary holds what a fresh one does, in one launch or two."""
+    if layout == "awq":
+        qw, qz, sc = oracle.make_awq(K, N, gs, seed=3)
+        gi = None
+    else:
+        qw, qz, sc, gi = oracle.make_gptq(K, N, gs, seed=3, sym=False, act_order=act_order)
+    pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), to_dev(gi, gpu), gs, 1 if layout == "awq" else 0)
+    x = to_dev(oracle.make_x(3, K, seed=3, dtype=dtype), gpu, bf16=dtype == "bf16")
+    want = pkg.ops.linear_gate_up(pk, x)
+    room = torch.zeros(want.numel() + 3, dtype=x.dtype, device=gpu)
+    out = room[1:-2].view(want.shape)
+    assert pkg.ops.linear_gate_up(pk, x, out=out) is out
+    assert torch.equal(out, want) and not room[0].any() and not room[-2:].any()
+
+
 def test_fused_equals_unfused_bitwise_at_decode(pkg, oracle, gpu):
     """Same kernel, same summation order, same roundings: the two routes agree bit for bit."""
     K, N, gs, M = 4096, 28672, 128, 2

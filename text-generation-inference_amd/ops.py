@@ -666,6 +666,8 @@ def linear_gate_up(
         raise ValueError(f"out must be a contiguous [{M}, {inter}] {x.dtype} tensor on {x.device}")
     if M == 0 or inter == 0:
         return y
+    if fused is None and y.data_ptr() % 16:  # an `out` where the fused launches do not write: whichever call it is, it is served
+        return y.copy_(linear_gate_up(w, x, act, bias))
     fusable_bias = bias is None or (bias.dtype == x.dtype and bias.is_cuda and bias.numel() == w.N)
     need, scratch = w.regroup(M, _DTYPES[x.dtype], True) if fused is None and fusable_bias else (0, 0)
     if scratch:
