@@ -36,14 +36,18 @@ def test_rows_and_shapes(pkg, oracle, gpu, K, N, gs, sym, M, dtype):
     bias = oracle.f32_to_bf16_bits(b32) if bf else b32.astype(np.float16)
     xt, bt = to_dev(x, gpu, bf16=bf), to_dev(bias, gpu, bf16=bf)
     y32, _ = oracle.linear_forward(x, w, bias, dtype)
+    assert pkg.ops.kernel_of(pk, M, xt.dtype) == "batch"
     got = pkg.ops.linear(pk, xt, bt)
     assert torch.equal(got, pkg.ops.linear(pk, xt, bt))  # the exchange cells are left at zero
     assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
     if N % 128 == 0:
-        assert pkg.ops._gate_up_fused_preferred(pk, M, 1 if bf else 0, True)
+        assert pkg.ops.kernel_of(pk, M, xt.dtype, True) == "batch"
         _, want = oracle.gate_up_forward(x, w, "silu", bias, dtype)
         gated = pkg.ops.linear_gate_up(pk, xt, "silu", bt)
         assert max_rel_err(to_f32(gated), oracle.to_f32(want, dtype)) <= TOL_GATED[dtype]
+        assert torch.equal(gated, pkg.ops.linear_gate_up(pk, xt, "silu", bt, fused=True))
+        two = pkg.ops.linear_gate_up(pk, xt, "silu", bt, fused=False)
+        assert max_rel_err(to_f32(gated), to_f32(two)) <= TOL_GATED[dtype]
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
@@ -81,7 +85,7 @@ def test_without_a_workspace(pkg, oracle, gpu):
 
     K, N, M = 27264, 128, 64  # 426 groups: their table and the groups of all rows are more than a workgroup's LDS
     pk, w = _weight(pkg, oracle, gpu, K, N, 64, 11, "f16")
-    assert pkg.ops._gate_up_fused_preferred(pk, M, 0, True)  # (with the cells it is this kernel's)
+    assert pkg.ops.kernel_of(pk, M) == "batch"  # (with the cells it is this kernel's)
     x = oracle.make_x(M, K, seed=12)
     xt, y = to_dev(x, gpu), torch.empty((M, N), dtype=torch.float16, device=gpu)
     lib = pkg._lib

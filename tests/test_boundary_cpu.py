@@ -215,7 +215,13 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     (14336, 4096, 128, 0, False, 49, "f16", 0, "batch"), (14336, 8192, 128, 0, False, 49, "f16", 0, "gemm"),
     (4096, 28672, 128, 1, False, 1, "f16", 0, "gemv"), (4096, 28672, 128, 1, False, 16, "f16", 1, "batch"),
     (4096, 4096, 128, 1, False, 1, "f16", 0, "batch"), (14336, 4096, 128, 1, False, 33, "f16", 0, "gemm"),
-    (8192, 10240, 128, 0, True, 4, "f16", 0, "gemv"), (8192, 10240, 128, 0, True, 33, "f16", 0, "gemm"),
+    (8192, 10240, 128, 0, True, 4, "f16", 0, "gemv"), (8192, 10240, 128, 0, True, 33, "f16", 0, "batch"),
+    (8192, 10240, 128, 0, True, 4, "f16", 1, "batch"), (8192, 10240, 128, 0, True, 6, "f16", 0, "batch"),
+    (18944, 3584, 128, 0, True, 2, "bf16", 0, "gemv"), (18944, 3584, 128, 0, True, 3, "bf16", 0, "batch"),
+    (8192, 57344, 32, 0, True, 2, "f16", 1, "batch"), (8192, 57344, 32, 0, True, 3, "f16", 1, "none"),
+    (8192, 57344, 32, 0, True, 16, "bf16", 0, "gemv"), (8192, 57344, 32, 0, True, 17, "bf16", 0, "batch"),
+    (4096, 4096, 128, 0, True, 64, "f16", 1, "batch"), (4096, 4096, 128, 0, True, 65, "f16", 1, "none"),
+    (4096, 4096, 128, 0, True, 65, "f16", 0, "gemm"), (4096, 4160, 128, 0, True, 1, "f16", 1, "none"),
     (8192, 57344, 128, 1, False, 5, "f16", 0, "gemv"), (8192, 57344, 128, 1, False, 5, "bf16", 1, "none"),
     (8192, 57344, 128, 1, False, 7, "f16", 0, "batch"), (8192, 57344, 128, 1, False, 7, "f16", 1, "batch"),
     (3584, 37888, 128, 1, False, 32, "f16", 0, "batch"), (3584, 37888, 128, 1, False, 33, "f16", 0, "gemm"),

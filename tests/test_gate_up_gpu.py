@@ -154,10 +154,9 @@ def test_prefill_fused_equals_two_kernels_bitwise(pkg, oracle, gpu, act, dtype, 
             assert max_rel_err(to_f32(one), to_f32(two)) <= (TOL_BF16 if bf else TOL)
 
 
-@pytest.mark.parametrize("layout,act_order", [("awq", False), ("gptq", True)])
-@pytest.mark.parametrize("M", [1, 200])
+@pytest.mark.parametrize("layout,act_order,M", [("awq", False, 1), ("awq", False, 200), ("gptq", True, 65), ("gptq", True, 200)])
 def test_unfused_fallback(pkg, oracle, gpu, layout, act_order, M):
-    """AWQ and act-order weights have no fused kernel: linear + elementwise kernel, same result."""
+    """Small AWQ layers, and act-order ones beyond the decode batches, have no fused kernel: linear + elementwise kernel, same result."""
     _case(pkg, oracle, gpu, 2048, 1024, 128, M, layout=layout, act_order=act_order, seed=M + 20)
     with pytest.raises(pkg._lib.Q4Error):
         _case(pkg, oracle, gpu, 2048, 1024, 128, M, layout=layout, act_order=act_order, fused=True, seed=M + 20)

@@ -253,7 +253,8 @@ int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up) {
   if (gate_up && (w->N & 1)) return Q4_PATH_AUTO;
   const int path = q4_select_path(w, M, dtype);
   BatchPlan batch;
-  if ((gate_up || path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) && batch_default(w, M, dtype, gate_up != 0, &batch))
+  if ((gate_up || path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) &&
+      (batch_default(w, M, dtype, gate_up != 0, &batch) || batch_act_default(w, M, dtype, gate_up != 0, &batch)))
     return Q4_KERNEL_BATCH;
   TallPlan tall;
   if (path == Q4_PATH_GEMM && gemm_tall_default(w, M, dtype, gate_up != 0, &tall))

@@ -681,7 +681,7 @@ def linear_gate_up(
                     y.data_ptr(), M, _DTYPES[x.dtype], _lib.ACTIVATIONS[act], ws.data_ptr(), ws.numel(), mem.data_ptr(),
                     mem.numel(), stream))
                 return y
-    if fused is None and fusable_bias and w.g_idx is not None and _gate_up_fused_preferred(w, M, _DTYPES[x.dtype], True):
+    if fused is not False and fusable_bias and w.g_idx is not None and _gate_up_fused_preferred(w, M, _DTYPES[x.dtype], True):
         with _on_device(x.device):
             stream = _stream_handle(x.device)
             ws = _workspace_for_call(x.device, w.plan(M, _DTYPES[x.dtype])[1], stream)
