@@ -263,7 +263,7 @@ def test_bf16_few_rows_on_large_layers(pkg, oracle, gpu, K, N, M):
     assert max_rel_err(to_f32(got), oracle.to_f32(want, "bf16")) <= TOL_GATED["bf16"]
 
 
-@pytest.mark.parametrize("layout,K,N", [("gptq", 512, 64), ("gptq", 1152, 384), ("gptq", 1024, 16384), ("awq", 512, 256), ("awq", 4096, 1024),
+@pytest.mark.parametrize("layout,K,N", [("gptq", 512, 64), ("gptq", 1152, 384), ("gptq", 1024, 16384), ("gptq", 2048, 16384), ("awq", 512, 256), ("awq", 4096, 1024),
                                         ("awq", 9216, 512)])
 @pytest.mark.parametrize("M,dtype", [(1, "f16"), (3, "bf16"), (16, "f16"), (17, "bf16"), (32, "f16"), (33, "bf16"), (48, "f16"), (64, "bf16")])
 def test_groups_of_32_rows(pkg, oracle, gpu, layout, K, N, M, dtype):

@@ -210,7 +210,7 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     (4096, 6144, 128, 0, False, 1, "f16", 0, "gemv"), (4096, 6144, 128, 0, False, 5, "f16", 0, "batch"),
     (4096, 28672, 128, 0, False, 1, "f16", 1, "batch"), (3584, 37888, 128, 0, False, 13, "bf16", 0, "batch"),
     (4096, 28672, 128, 0, False, 3, "bf16", 0, "gemv"), (8192, 57344, 128, 0, False, 16, "f16", 1, "none"),
-    (14336, 4096, 64, 0, False, 1, "f16", 0, "batch"), (4096, 14336, 32, 0, False, 37, "f16", 0, "gemm"),
+    (14336, 4096, 64, 0, False, 1, "f16", 0, "batch"), (4096, 14336, 32, 0, False, 37, "f16", 0, "batch"),
     (4608, 28672, 384, 0, False, 1, "f16", 1, "gemv"), (4096, 6144, 128, 0, False, 64, "f16", 0, "batch"),
     (14336, 4096, 128, 0, False, 49, "f16", 0, "batch"), (14336, 8192, 128, 0, False, 49, "f16", 0, "gemm"),
     (4096, 28672, 128, 1, False, 1, "f16", 0, "gemv"), (4096, 28672, 128, 1, False, 16, "f16", 1, "batch"),
