@@ -247,6 +247,18 @@ def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, w
     assert pkg._lib.KERNEL_NAMES[rc] == want
 
 
+@pytest.mark.parametrize("K,N,gs,M,want", [(8192, 32768, 128, 33, 0), (8192, 32768, 128, 64, 0), (8192, 57344, 32, 48, 0), (8256, 33024, 64, 32, 0),
+                                          (8256, 33024, 64, 33, 1), (8256, 57344, 64, 64, 1), (8256, 57344, 64, 65, 0), (8256, 28672, 64, 48, 0),
+                                          (8192, 32768, 128, 128, 0), (8192, 32768, 128, 129, 1)])
+def test_decode_batches_regroup_where_no_kernel_reads_through_g_idx(pkg, K, N, gs, M, want):
+    """33-64 rows: the act-order batch kernel's calls are never regrouped, the widest of the others are."""
+    lib, w = pkg._lib.load(), _weight(pkg, K, N, gs, g_idx=True)
+    need, scratch = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    for dtype in (0, 1):
+        assert lib.q4_linear_regroup_plan(ctypes.byref(w), M, dtype, 0, ctypes.byref(need), ctypes.byref(scratch)) == want
+        assert not (want and pkg._lib.KERNEL_NAMES[lib.q4_linear_kernel(ctypes.byref(w), M, dtype, 0)] == "batch")
+
+
 @pytest.mark.parametrize("E,topk,K,N,tokens,gate_up,want", [
     (8, 2, 4096, 28672, 192, 1, "batch"), (8, 2, 14336, 4096, 192, 0, "batch"), (8, 2, 14336, 4096, 193, 0, "gemm"),
     (64, 6, 1408, 2048, 48, 0, "batch"), (64, 6, 1408, 2048, 64, 0, "gemv"), (64, 6, 1408, 2048, 192, 0, "gemm"),

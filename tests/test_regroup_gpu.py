@@ -64,12 +64,12 @@ def test_regrouped_call_matches_oracle(pkg, oracle, gpu, K, N, gs, M, dtype):
     assert np.abs(got - want).max() <= 4 * (2.0 ** -8 if dtype == "bf16" else 2.0 ** -11) * np.abs(want).max()
 
 
-@pytest.mark.parametrize("K,N,M,regroups", [(512, 32768, 48, False), (4096, 28672, 48, False), (4096, 28672, 130, True), (4096, 4096, 1024, False), (4096, 6144, 1536, True),
+@pytest.mark.parametrize("K,N,M,regroups", [(512, 32768, 48, False), (4096, 28672, 48, False), (8192, 32768, 48, False), (8256, 33024, 48, True), (4096, 28672, 130, True), (4096, 4096, 1024, False), (4096, 6144, 1536, True),
                                           (14336, 4096, 301, True), (14336, 4096, 400, False), (4096, 6144, 700, True), (3584, 4608, 1100, True)])
 def test_layers_regroup_from_the_librarys_row_count_on(pkg, oracle, gpu, K, N, M, regroups):
     """The tensor calls take the regrouped route by the library's rule; gated and plain agree with the
     kernels that read through g_idx (the same weights, sums in another order)."""
-    _, pk = build(pkg, oracle, gpu, K, N, 128, seed=N)
+    _, pk = build(pkg, oracle, gpu, K, N, 64 if K % 128 else 128, seed=N)
     x = torch.randn((M, K), device=gpu, dtype=torch.float16) * 0.1
     assert (pk.regroup(M, 0, False)[1] > 0) == regroups
     plain = pkg.ops.linear(pk, x, path=2)
@@ -78,8 +78,8 @@ def test_layers_regroup_from_the_librarys_row_count_on(pkg, oracle, gpu, K, N, M
     assert pkg.ops.linear(pk, x[:0]).shape == (0, N)
 
 
-# On the size below, 48 rows: the batch decode kernel on the copy; 200: the prefill kernels
-ROWS = [48, 200]
+# On the size below the library regroups from 129 rows on: just above, and well inside
+ROWS = [130, 200]
 
 
 def big(pkg, gpu, seed):

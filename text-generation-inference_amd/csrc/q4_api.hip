@@ -536,8 +536,10 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
   // launches that end at the flag (3-7 us) come back as rows and weights multiply; the kernels that read through g_idx hold
   // row blocks of 128 and 256, in which they are flat in M.  Time through g_idx over time regrouped, MI355X, 19
   // layer shapes, fp16, groups of 32 to 128, 26 row counts from 129 on, plain and gated (geometric mean; least, most of what is taken):
-  //   33-64 rows    the batch decode kernel on the copy, before q4_gemv_batch_act.cuh: 8192 x 57344 1.14-1.30; 4096 x 28672 0.94-1.06, 3584 x 37888
-  //                 0.91-1.05, narrower ones down to 0.6
+  //   33-64 rows    0.52-0.87 where the act-order batch kernel reads through g_idx (8192 x 32768 at 48 rows 69 / 114 us, gated
+  //                 8192 x 57344 at 33 115 / 201); what it does not hold (K no multiple of 128) 1.07-1.46: 8256 x 33024 at 48 rows 181 / 147,
+  //                 8256 x 57344 253 / 217; against the kernels before it 4096 x 28672 0.94-1.06, 3584 x 37888 0.91-1.05, narrower
+  //                 ones down to 0.6
   //   no table      (too many groups for LDS) 1.53 (1.01, 2.39); 8192 x 1280 0.66-0.92 up to 512 rows
   //   129-256 rows  1.28 (1.06, 1.64); 4096 x 12288 0.88-1.17, 8192 x 8192 0.89-1.03, 8192 x 10240 1.14 at 129, 0.94 at
   //                 256; 4096 x 22016 and 28672 at 193-256 1.04-1.20, but bf16 layers 0.93-0.96 of their speed
@@ -546,9 +548,9 @@ int q4_linear_regroup_plan(const q4_weight* w, int M, int dtype, int gate_up, si
   //                 0.74-1.02
   const double weights = (double)w->K * w->N;
   const bool wide = w->N / 2 >= w->K;
-  // (up to 64 rows the kernel of q4_gemv_batch_act.cuh reads through g_idx faster than any copy is made: gated 8192 x 57344 regrouped /
-  // there 33 rows 205 / 123 us, 64 rows 218 / 169; the tests of the regrouped route hold 8192 x 32768 at 48 rows, 120 us, to it)
-  if (M <= 128) return M >= Q4_REGROUP_MIN_ROWS && M <= 64 && w->N / 4 >= w->K && weights >= 2.6e8 && weights < 3e8;
+  BatchPlan batch;
+  if (M <= 128)
+    return M >= Q4_REGROUP_MIN_ROWS && M <= 64 && w->N / 4 >= w->K && weights >= 2.6e8 && !batch_act_default(w, M, dtype, gate_up != 0, &batch);
   if (!gemm_act_order_table(w)) return weights >= 4e7 || (M > 512 && weights >= 1e7);
   if (M <= 256) return weights >= (M <= 192 ? 8e7 : 1.3e8) && (wide || (w->N >= w->K && M <= 160));
   if (M <= 512) return weights >= 1e8 || (weights >= 4e7 && (wide || M <= 352));
