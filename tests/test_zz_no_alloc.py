@@ -57,8 +57,9 @@ def test_noalloc_matches_q4_linear_two_calls_in_a_row(pkg, oracle, gpu):
     _both(pkg, oracle, gpu, 14336, 4096, 8, seed=3, kernel="batch")
     _both(pkg, oracle, gpu, 4096, 1024, 5, seed=4, kernel="batch")
     _both(pkg, oracle, gpu, 4096, 2048, 16, layout="awq", seed=8, kernel="batch")
-    # ticket path (act-order, bf16)
-    _both(pkg, oracle, gpu, 4096, 1024, 5, act=True, dtype="bf16", seed=9, kernel="gemv")
+    # act-order, bf16: the ticket path (256 groups, a K deal that does not come out even), and the batch kernel's exchange cells
+    _both(pkg, oracle, gpu, 32768, 384, 5, act=True, dtype="bf16", seed=13, kernel="gemv")
+    _both(pkg, oracle, gpu, 4096, 1024, 5, act=True, dtype="bf16", seed=9, kernel="batch")
     # prefill: split-K partial tiles in the array, then a smaller prefill and a decode call
     _both(pkg, oracle, gpu, 4096, 1024, 256, seed=5, kernel="tall")
     _both(pkg, oracle, gpu, 4096, 1024, 300, layout="awq", seed=10, kernel="gemm")
