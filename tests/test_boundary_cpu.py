@@ -376,6 +376,29 @@ def test_weights_on_another_gpu_are_refused(pkg, monkeypatch, layout, g_idx):
             call(w, x)
 
 
+@pytest.mark.parametrize("why", ["missing", "built against torch"])
+def test_calls_without_the_extension_module(pkg, oracle, monkeypatch, tmp_path, why):
+    """The Python code answers where the eager call's module cannot be used; without the library nothing does."""
+    qw, qz, sc, _ = _cpu_gptq_tensors(oracle)
+    pk = pkg.ops.make_packed(qw, qz, sc, None, 128, 0)
+    monkeypatch.setattr(pkg._lib, "_call", None)
+    if why == "missing":
+        monkeypatch.setattr(pkg._lib, "CALL_PATH", tmp_path / "_q4call.so")
+    else:
+        monkeypatch.setattr(torch, "__version__", "2.0.0")
+    with pytest.warns(RuntimeWarning, match=why):
+        call = pk.call()
+    x = torch.zeros(1, 256, dtype=torch.float16)
+    assert call(x, None) is None and call(x, None, pk) is None
+    with pytest.raises(RuntimeError, match="GPU only"):  # linear's own answer to a tensor on the CPU
+        pkg.ops.apply_linear(pk, x, None)
+    monkeypatch.setattr(pkg._lib, "_lib", None)
+    monkeypatch.setattr(pkg._lib, "LIB_PATH", tmp_path / "libq4linear.so")
+    monkeypatch.setattr(pkg._lib, "_call", None)
+    with pytest.raises(ImportError, match="no fallback"):
+        pkg.ops.make_packed(qw, qz, sc, None, 128, 0).call()
+
+
 def test_nested_activations_raise(pkg, oracle):
     """Tensors whose sizes throw come back as a Python error (in a process of their own: what a C++ exception ends is the process)."""
     import subprocess

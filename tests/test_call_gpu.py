@@ -77,6 +77,15 @@ def test_other_forms_are_left_to_the_python_code(pkg, oracle, gpu):
     side.synchronize()
 
 
+def test_without_the_extension_module(pkg, oracle, gpu, monkeypatch):
+    """The same bytes from the steps in Python."""
+    pk, x = _weight(pkg, oracle, gpu, "gptq"), torch.randn((2, 3, 512), device=gpu).half()
+    want = pkg.ops.apply_linear(pk, x, None)
+    monkeypatch.setattr(pkg._lib, "_call", False)
+    bare = _weight(pkg, oracle, gpu, "gptq")
+    assert bare.call()(x, None) is None and torch.equal(pkg.ops.apply_linear(bare, x, None), want)
+
+
 def test_captured_call(pkg, oracle, gpu):
     pk = _weight(pkg, oracle, gpu, "gptq", K=4096)
     pk.prepare()

@@ -2,11 +2,13 @@
 
 The library is the only compute path of this package: if it is missing, loading fails
 with an error that says how to build it; nothing falls back to PyTorch or the CPU.
+(The host path of the eager call, _q4call.so, is another matter: the Python code launches the same kernels.)
 """
 
 from __future__ import annotations
 
 import ctypes
+import warnings
 from ctypes import POINTER, Structure, c_char_p, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -141,7 +143,7 @@ SIGNATURES = {
 }
 
 _lib = None
-_call = None
+_call = None  # the module, or False where there is none for this torch
 
 
 class Q4Error(RuntimeError):
@@ -173,18 +175,28 @@ def load() -> ctypes.CDLL:
 
 def load_call(workspaces: dict):
     """The extension module of the eager call (csrc/bindings/q4_call.cpp), bound to the library's entry points and to the
-    dict of workspaces; raises if it has not been built."""
+    dict of workspaces.  None, with a warning, where it is not built or was built against another torch, whose classes it
+    reads: the Python code then makes every call, about 2 us slower on the host."""
     global _call
     if _call is None:
-        if not CALL_PATH.exists():
-            raise ImportError(f"{CALL_PATH} is missing: build it with `python {HERE / 'build.py'}`; there is no fallback path")
-        from . import _q4call
-
         lib = load()
-        addresses = [ctypes.cast(fn, c_void_p).value for fn in (lib.q4_linear_ex, lib.q4_gemv_tuned)]
-        _q4call.bind(*addresses, workspaces, check)
-        _call = _q4call
-    return _call
+        try:
+            if not CALL_PATH.exists():
+                raise ImportError(f"{CALL_PATH} is missing")
+            import torch
+
+            from . import _q4call
+
+            if _q4call.torch_version != str(torch.__version__):
+                raise ImportError(f"{CALL_PATH} was built against torch {_q4call.torch_version}, this is {torch.__version__}")
+        except ImportError as e:
+            warnings.warn(f"eager calls take their host path in Python: {e}; build it with `python {HERE / 'build.py'}`", RuntimeWarning)
+            _call = False
+        else:
+            addresses = [ctypes.cast(fn, c_void_p).value for fn in (lib.q4_linear_ex, lib.q4_gemv_tuned)]
+            _q4call.bind(*addresses, workspaces, check)
+            _call = _q4call
+    return _call or None
 
 
 def check(code: int) -> None:

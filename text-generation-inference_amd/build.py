@@ -4,7 +4,7 @@ libq4linear.so           the product: every kernel and the C ABI of include/q4_l
 libq4probe.so            read-only / LDS probe kernels of bench.py (csrc/bench/q4_probe.hip)
 libq4linear_stamps.so    the product's sources with -DQ4_PHASE_STAMPS: the decode kernels also leave
                          clock readings per wave and phase (bench.py --phase-breakdown)
-_q4call.so               the host path of the eager call (csrc/bindings, g++ against torch's headers)
+_q4call.so               the host path of the eager call (csrc/bindings, g++ or amdclang++ against torch's headers); optional
 All are built in-tree next to this file so that they travel with the source tree.
 Run as a script (`python build.py`) or call build_all().
 """
@@ -134,14 +134,16 @@ def build_bench_libraries(verbose: bool = False) -> list[Path]:
 
 def build_call_module(verbose: bool = False) -> Path:
     """The extension module of the eager call: host code only, no kernel in it."""
+    import shutil
     import sysconfig
 
     import torch
 
     base = Path(torch.__file__).parent
     tmp = CALL_LIB_PATH.with_suffix(".so.tmp")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}", f"-I{base / 'include'}",
+    compiler = shutil.which("g++") or str(Path(HIPCC).parent / "amdclang++")
+    cmd = [compiler, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f'-DQ4_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}", f"-I{base / 'include'}",
            f"-I{base / 'include/torch/csrc/api/include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
            str(CSRC / "bindings" / "q4_call.cpp"), "-o", str(tmp), f"-L{base / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip"]
     if verbose:
@@ -152,7 +154,14 @@ def build_call_module(verbose: bool = False) -> Path:
 
 
 def build_all(verbose: bool = False) -> list[Path]:
-    return [build_library(verbose=verbose), build_call_module(verbose=verbose)] + build_bench_libraries(verbose=verbose)
+    """Everything; where Python's or torch's headers are missing, without the extension module, which no call needs."""
+    built = [build_library(verbose=verbose)]
+    try:
+        built.append(build_call_module(verbose=verbose))
+    except (subprocess.CalledProcessError, OSError, ImportError) as e:
+        CALL_LIB_PATH.unlink(missing_ok=True)  # (one of an earlier build knows an earlier library)
+        print(f"[build] {CALL_LIB_PATH.name} FAILED, eager calls take their host path in Python: {e}", file=sys.stderr)
+    return built + build_bench_libraries(verbose=verbose)
 
 
 if __name__ == "__main__":

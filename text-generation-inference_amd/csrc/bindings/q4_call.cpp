@@ -224,5 +224,8 @@ PyMODINIT_FUNC PyInit__q4call(void) {
   CallType.tp_call = PyVectorcall_Call;
   CallType.tp_dealloc = call_dealloc;
   if (PyType_Ready(&CallType) < 0) return nullptr;
-  return PyModule_Create(&kModule);
+  PyObject* module = PyModule_Create(&kModule);
+  // the torch whose classes are compiled in
+  if (module != nullptr && PyModule_AddStringConstant(module, "torch_version", Q4_TORCH_VERSION) < 0) Py_CLEAR(module);
+  return module;
 }

@@ -59,6 +59,10 @@ def _dense16(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _left_to_python(x, bias, weight=None) -> None:
+    """PackedWeight.call where there is no extension module."""
+
+
 @dataclass
 class PackedWeight:
     """Validated view of one quantized weight, ready to be passed through the C ABI."""
@@ -102,8 +106,9 @@ class PackedWeight:
         if self._call is None:
             first = 0 if self.perm is not None else (_lib.REGROUP_MIN_ROWS if self.g_idx is not None else 1 << 40)
             device = self.qweight.device.index if self.qweight.is_cuda else None
-            handle = _lib.load_call(_workspaces).handle
-            self._call = handle(bytes(self.struct()), self._plans, -1 if device is None else device, first)
+            module = _lib.load_call(_workspaces)
+            self._call = _left_to_python if module is None else module.handle(
+                bytes(self.struct()), self._plans, -1 if device is None else device, first)
         return self._call
 
     def plan(self, M: int, dtype_code: int) -> tuple:
