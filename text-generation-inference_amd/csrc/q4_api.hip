@@ -134,7 +134,8 @@ int q4_select_path(const q4_weight* w, int M, int dtype) {
   }
   // AWQ and act-order: the decode kernels take any M in row chunks of 16; the MFMA kernel
   // that unpacks the weights into LDS (split-K when its tile grid is small) takes over where
-  // it measured faster on MI355X.
+  // it measured faster on MI355X.  (Up to 64 rows this is the answer for forced paths and for what
+  // the batch decode kernels leave: batch_default, batch_act_default.)
   // Act-order: from M = 33 on when its parameter table fits in LDS (two 16-row blocks of the
   // decode kernel, which is flat in M within a block, against the MFMA kernel, flat in M up to
   // 128 rows, us at M = 32: 4096 x 4096 14.2 / 20.3, 14336 x 4096 27.0 / 43.4, 8192 x 10240
@@ -671,16 +672,20 @@ int q4_linear_gate_up_act_order_plan(const q4_weight* w, int M, int dtype, int* 
 
 int q4_linear_gate_up_act_order(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int act,
                                 void* workspace, size_t workspace_bytes, void* stream) {
-  int fused = 0;
-  int rc = q4_linear_gate_up_act_order_plan(w, M, dtype, &fused);
+  int rc = validate_weight(w, "q4_linear_gate_up_act_order");
+  if (rc == Q4_OK) rc = validate_dtype(dtype, "q4_linear_gate_up_act_order");
   if (rc != Q4_OK) return rc;
+  if (M < 0) {
+    set_error("q4_linear_gate_up_act_order: negative M=%d", M);
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
   if (act != Q4_ACT_SILU && act != Q4_ACT_GELU_TANH && act != Q4_ACT_GELU) {
     set_error("q4_linear_gate_up_act_order: unknown activation %d", act);
     return Q4_ERR_INVALID_ARGUMENT;
   }
   if (M == 0 || w->N == 0) return Q4_OK;
   BatchPlan plan;
-  if (!fused || !batch_act_default(w, M, dtype, true, &plan)) {
+  if (!batch_act_default(w, M, dtype, true, &plan)) {
     set_error("q4_linear_gate_up_act_order: no fused kernel for this problem (layout=%d g_idx=%p M=%d K=%d N=%d groupsize=%d)",
               w->layout, (const void*)w->g_idx, M, w->K, w->N, w->groupsize);
     return Q4_ERR_UNSUPPORTED;

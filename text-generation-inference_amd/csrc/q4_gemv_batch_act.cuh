@@ -1,9 +1,9 @@
-// Batch decode kernel for act-order weights (GPTQ layout with g_idx): y[M, N] = x @ dequant(W) for blocks of 16 to 64
-// activation rows, optionally with the gated-MLP epilogue.
+// Batch decode kernel for act-order weights (GPTQ layout with g_idx): y[M, N] = x @ dequant(W) for up to 64 activation rows,
+// optionally with the gated-MLP epilogue.
 //
 // Every K row has its own group, so every weight looks its scale and zero point up: about four vector instructions a weight, which
 // bound the launch (8192 x 57344 in fp16: the vector pipes issue two thirds of the time).  So:
-//   * A weight is unpacked once for all rows of a block of up to 64; a further 16 rows cost four matrix instructions,
+//   * A weight is unpacked once for all rows; a further 16 rows cost four matrix instructions,
 //     the fetch of their activations and four permutes per 32 x 64 weights.
 //   * The table of scale | -(1024 + zero), one row of 64 columns per group, lies at the start of LDS and a row is 256 bytes: the
 //     address of a lane's four columns is one byte permute of the group number and the lane's offset.
@@ -34,9 +34,7 @@ __global__ __launch_bounds__(64 * WK, MT <= 2 ? 4 : (MT == 3 ? 3 : 2)) void gemv
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, kq = lane >> 4;
   const int N = bp.N, half = N >> 1, tile = blockIdx.x;
-  const int split = blockIdx.y % (unsigned)bp.splits;
-  const int rb = blockIdx.y / (unsigned)bp.splits * (16 * MT);
-  const int M = min(bp.M - rb, 16 * MT);
+  const int split = blockIdx.y, M = bp.M;
   const int col = FUSE ? tile * 32 + 4 * (j & 7) + (j >> 3) * half : tile * 64 + 4 * j;
 
   const int slot0 = split * WK, slot = slot0 + wave;
@@ -50,7 +48,7 @@ __global__ __launch_bounds__(64 * WK, MT <= 2 ? 4 : (MT == 3 ? 3 : 2)) void gemv
   const uint32_t w_lane = ((uint32_t)kq * (uint32_t)N + (uint32_t)col) * 4u;
   uint32_t x_lane[MT];  // rows past the end lie past the end of x: zeros, no memory touched
 #pragma unroll
-  for (int m = 0; m < MT; ++m) x_lane[m] = ((uint32_t)(rb + 16 * m + j) * (uint32_t)bp.K + (uint32_t)kq * 8u) * 2u;
+  for (int m = 0; m < MT; ++m) x_lane[m] = ((uint32_t)(16 * m + j) * (uint32_t)bp.K + (uint32_t)kq * 8u) * 2u;
   struct Step {
     uint4_t x[MT], w;
   };
@@ -193,7 +191,7 @@ __global__ __launch_bounds__(64 * WK, MT <= 2 ? 4 : (MT == 3 ? 3 : 2)) void gemv
 
   __syncthreads();  // everybody is done with the table
   auto sums = [&](int w, int m, int r) { return (float*)(act_lds + (size_t)(w * MT + m) * 4096 + r * 256); };
-  batch_finish<DTYPE, false, MT, 1, 1, WK, FUSE, false>(bp, acc, sums, lane, wave, tile, split, 0, rb, M);
+  batch_finish<DTYPE, false, MT, 1, 1, WK, FUSE, false>(bp, acc, sums, lane, wave, tile, split, 0, 0, M);
 }
 
 }  // namespace q4

@@ -22,7 +22,7 @@ static bool act_supported(const q4_weight* w, int M, bool gate_up) {
 // the levels of the exchange and its traffic.  Its picks are 0.4 % above the best measured ones on average, 4.7 % at worst.
 // uneven: the chunks that the busiest CU's waves walk over an even share.
 static bool act_plan(const q4_weight* w, int M, int mt, BatchPlan* plan, double* uneven) {
-  const int chunks = w->K / 128, tiles = w->N / 64, row_blocks = (M + 16 * mt - 1) / (16 * mt);
+  const int chunks = w->K / 128, tiles = w->N / 64;
   double best = -1.0;
   for (int wk = 8; wk >= 4; wk -= 4)
     for (int sp = 1; sp <= 16; sp *= 2) {
@@ -33,7 +33,7 @@ static bool act_plan(const q4_weight* w, int M, int mt, BatchPlan* plan, double*
       int resident = (int)(160 * 1024 / lds);
       const int by_registers = (mt <= 2 ? 16 : (mt == 3 ? 12 : 8)) / wk;
       if (resident > by_registers) resident = by_registers;
-      const long wgs = (long)tiles * row_blocks * sp;
+      const long wgs = (long)tiles * sp;
       const double per_wave = (double)((chunks + wk * sp - 1) / (wk * sp));
       const double per_cu = (double)((wgs + 255) / 256), rounds = (double)((wgs + 256L * resident - 1) / (256L * resident));
       double t = (0.653 + 0.229 * mt) * per_wave * (0.724 * rounds + 1.027 * per_cu * wk / 4.0) + 2.263 * (rounds - 1.0);
@@ -42,7 +42,7 @@ static bool act_plan(const q4_weight* w, int M, int mt, BatchPlan* plan, double*
       if (best < 0.0 || t < best) {
         best = t;
         *plan = BatchPlan{1, wk, sp};
-        *uneven = per_cu * wk * per_wave * 256.0 / ((double)chunks * tiles * row_blocks);
+        *uneven = per_cu * wk * per_wave * 256.0 / ((double)chunks * tiles);
       }
     }
   return best >= 0.0;
@@ -101,7 +101,7 @@ int launch_batch_act(const q4_weight* w, const void* x, const void* bias, void* 
                      size_t workspace_bytes, const BatchPlan& plan_in, hipStream_t stream) {
   BatchPlan plan = plan_in;
   const bool fuse = gate_up_act != 0;
-  const int mt = M > 64 ? 4 : (M + 15) / 16;
+  const int mt = (M + 15) / 16;
   if (plan.splits > 1 && !act_cells(workspace, workspace_bytes)) plan.splits = 1;
   const size_t lds = q4::batch_act_lds(w->num_groups, act_k_rows(w, plan.wk, plan.splits), plan.wk, mt);
   if (lds > 160 * 1024 - 1024) {
@@ -128,7 +128,7 @@ int launch_batch_act(const q4_weight* w, const void* x, const void* bias, void* 
   bp.splits = plan.splits;
   bp.units = (M + 1) / 2;
   bp.act = fuse ? gate_up_act - 1 : 0;
-  const dim3 grid((unsigned)(w->N / 64), (unsigned)(plan.splits * ((M + 16 * mt - 1) / (16 * mt))));
+  const dim3 grid((unsigned)(w->N / 64), (unsigned)plan.splits);
   if (dtype == Q4_DTYPE_F16) act_rows<Q4_DTYPE_F16>(bp, mt, plan.wk, fuse, grid, lds, stream);
   else act_rows<Q4_DTYPE_BF16>(bp, mt, plan.wk, fuse, grid, lds, stream);
   const hipError_t err = hipGetLastError();
