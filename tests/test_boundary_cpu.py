@@ -227,6 +227,14 @@ def test_noalloc_entry_point_validation_without_gpu(pkg):
     (3584, 37888, 128, 1, False, 32, "f16", 0, "batch"), (3584, 37888, 128, 1, False, 33, "f16", 0, "gemm"),
     (3584, 37888, 128, 0, False, 49, "bf16", 0, "gemm"), (3584, 37888, 128, 0, False, 49, "bf16", 1, "batch"),
     (3584, 37888, 128, 0, False, 49, "f16", 0, "batch"),
+    # deals of K over power-of-two splits that come out uneven are left to the older kernels
+    (4608, 4608, 32, 0, False, 3, "f16", 0, "gemv"), (4608, 4608, 32, 0, False, 4, "f16", 0, "batch"), (4608, 4608, 32, 0, False, 1, "bf16", 0, "batch"),
+    (5760, 8704, 32, 0, False, 48, "f16", 0, "batch"), (5760, 8704, 32, 0, False, 49, "f16", 0, "gemm"), (5760, 8704, 32, 0, False, 49, "f16", 1, "batch"),
+    (3584, 37888, 32, 0, False, 64, "bf16", 1, "none"), (2432, 1024, 32, 0, False, 49, "f16", 0, "gemv"),
+    (3584, 8192, 128, 1, False, 1, "bf16", 1, "none"), (3584, 8192, 32, 1, False, 1, "bf16", 1, "batch"), (4096, 6144, 128, 1, False, 1, "bf16", 1, "batch"),
+    (8192, 10240, 128, 1, False, 4, "bf16", 1, "none"), (4096, 22016, 128, 1, False, 4, "bf16", 1, "batch"), (8192, 10240, 32, 1, False, 4, "f16", 1, "none"),
+    (5760, 8704, 128, 1, False, 2, "bf16", 0, "gemv"), (5760, 8704, 128, 1, False, 3, "bf16", 0, "batch"),
+    (8192, 10240, 32, 0, True, 16, "f16", 1, "none"), (8192, 10240, 32, 0, True, 17, "f16", 1, "batch"), (8192, 10240, 32, 0, True, 3, "bf16", 1, "batch"),
     # prefill
     (4096, 6144, 128, 0, False, 2048, "bf16", 0, "gemm"), (4096, 28672, 128, 0, False, 2048, "bf16", 1, "gemm"),
     (4096, 28672, 128, 0, False, 301, "f16", 1, "tall"), (14336, 4096, 128, 0, False, 301, "f16", 0, "tall"),

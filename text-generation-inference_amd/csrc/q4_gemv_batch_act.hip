@@ -56,12 +56,15 @@ static bool act_plan(const q4_weight* w, int M, int mt, BatchPlan* plan, double*
 // Its K splits are powers of two, which deal some layers out unevenly; up to a few rows the older kernel, whose splits are
 // any number, is as fast or faster there: fp16 3584 x 4608 1 row 7.9 / 8.8, 5 rows 8.6 / 9.0, 8192 x 10240 18.0 / 18.9,
 // 18944 x 3584 16.7 / 17.4, 3584 x 3584 7.6 / 7.9 (3584 x 4608 in bf16 10.7 / 9.3); groups of 32, whose tables leave room for fewer
-// workgroups, 8192 x 10240 1 row 19.6 / 22.2, 16 rows 22.4 / 23.3, and 8192 x 57344 from 3 rows on, gated 5 rows 91.7 / 99.0.
+// workgroups, 8192 x 10240 1 row 19.6 / 22.2, 16 rows 22.4 / 23.3 (gated fp16 21.5 / 24.0 and 24.5 / 25.5, bf16 up to 2 rows; gated 9344 x
+// 18560 is faster here, 1.1 and more), and 8192 x 57344 from 3 rows on, gated 5 rows 91.7 / 99.0.
 bool batch_act_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan) {
   double uneven = 1.0;
   if (M > 64 || !act_supported(w, M, gate_up) || !act_plan(w, M, (M + 15) / 16, plan, &uneven)) return false;
   const double weights = (double)w->K * w->N;
-  if (w->num_groups >= 256 && M <= 16 && (weights >= 2.6e8 ? M > 2 : !gate_up && uneven >= 1.19)) return false;
+  if (w->num_groups >= 256 && M <= 16 && weights >= 2.6e8 && M > 2) return false;
+  if (w->num_groups >= 256 && M <= 16 && weights < 2.6e8 && uneven >= 1.19 && (!gate_up || (weights < 1.2e8 && (dtype == Q4_DTYPE_F16 || M <= 2))))
+    return false;
   if (gate_up || weights < 1.2e7) return true;
   if (w->groupsize < 64) return !(dtype == Q4_DTYPE_F16 && M <= 2 && uneven >= 1.9);
   return !(dtype == Q4_DTYPE_F16 ? M <= 5 && uneven >= 1.11 : M <= 2 && uneven >= 1.19 && w->K >= 8192);
