@@ -118,10 +118,10 @@ int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);
  * (server/text_generation_server/models/custom_modeling/flash_llama_modeling.py:400-404;
  * the reference fuses this only for unquantized ROCm decode, `ops.LLMM_Silu`, :378-397).
  * Runs for contiguous groups, either layout, in the kernels that q4_linear_kernel(w, M, dtype, 1) names: up to 64
- * rows the batch decode kernel (AWQ from five rows on; groups it does not take: the GPTQ decode kernel, one or
- * two rows), above the prefill kernels.  Returns Q4_ERR_UNSUPPORTED where that answer is Q4_PATH_AUTO (g_idx, few
- * AWQ rows, odd shapes, some sizes where the two launches measured faster): the caller then runs q4_linear into an
- * [M, N] buffer and q4_act_mul.
+ * rows the batch decode kernel (what it does not take: the GPTQ decode kernel, one or two rows), above the prefill
+ * kernels.  Returns Q4_ERR_UNSUPPORTED where that answer is Q4_PATH_AUTO (odd shapes, sizes where the two launches measured
+ * faster) and for every act-order weight (g_idx set; q4_linear_gate_up_act_order below): the caller then runs q4_linear into
+ * an [M, N] buffer and q4_act_mul.
  */
 #define Q4_ACT_SILU 0       /* x * sigmoid(x) */
 #define Q4_ACT_GELU_TANH 1  /* gelu(approximate="tanh"): "gelu_fast", "gelu_pytorch_tanh" */

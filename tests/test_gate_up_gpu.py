@@ -54,7 +54,7 @@ def _case(pkg, oracle, gpu, K, N, gs, M, act="silu", dtype="f16", layout="gptq",
 
 @pytest.mark.parametrize("M", [1, 2, 3, 8, 16])
 def test_decode_llama3_8b_gate_up(pkg, oracle, gpu, M):
-    # the fused kernel is offered for one and two rows; more rows take the two-kernel route
+    # one and two rows by force, more by the library's own choice
     _case(pkg, oracle, gpu, 4096, 28672, 128, M, fused=True if M <= 2 else None, seed=M)
 
 

@@ -1,5 +1,5 @@
 // Unfused tail of a gated MLP: y[M, I] = act(gate_up[:, :I]) * gate_up[:, I:], for the
-// weights whose linear kernels have no fused epilogue (AWQ layout, act-order).  HBM-bound
+// calls that no gated launch takes or that are faster in two.  HBM-bound
 // elementwise pass: 16-byte loads of both halves, one 16-byte store.
 #include "q4_common.cuh"
 
