@@ -288,3 +288,32 @@ def test_groups_of_32_rows(pkg, oracle, gpu, layout, K, N, M, dtype):
     want = torch.where(ref == ref, ref, torch.full_like(ref, float("nan")))  # (an infinity times zero)
     assert torch.equal(torch.isnan(bad[M - 1].float().cpu()), torch.isnan(want))
     assert torch.equal(torch.isposinf(bad[M - 1].float().cpu()), torch.isposinf(want)) and torch.equal(bad[:-1], got[:-1])
+
+
+@pytest.mark.parametrize("layout,N", [("gptq", 192), ("gptq", 16640), ("awq", 512)])
+@pytest.mark.parametrize("K,gs", [(640, 64), (640, 128), (1408, 128), (1280, 256), (1152, -1)])
+@pytest.mark.parametrize("M,dtype", [(6, "f16"), (16, "bf16"), (31, "f16"), (40, "bf16")])
+def test_group_lengths_over_ragged_deals(pkg, oracle, gpu, layout, N, K, gs, M, dtype):
+    """Groups that end inside, with and beyond a 128-row chunk, K waves that walk one chunk and several."""
+    pk, w = _weight(pkg, oracle, gpu, layout, K, N, gs, K + M, dtype)
+    bf = dtype == "bf16"
+    x = oracle.make_x(M, K, seed=M, dtype=dtype)
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16) == "batch"
+    y32, _ = oracle.linear_forward(x, w, None, dtype)
+    assert max_rel_err(to_f32(pkg.ops.linear(pk, to_dev(x, gpu, bf16=bf))), y32) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("T,dtype", [(9, "f16"), (40, "bf16")])
+def test_experts_in_groups_of_64(pkg, oracle, gpu, T, dtype):
+    K, N, E, gs, topk = 640, 768, 4, 64, 2
+    parts = [oracle.make_gptq(K, N, gs, seed=e, sym=False)[:3] for e in range(E)]
+    packed = pkg.ops.make_packed_moe(*[torch.stack([to_dev(p[i], gpu) for p in parts]) for i in range(3)], gs)
+    xs = oracle.make_x(T, K, seed=T, dtype=dtype)
+    routing = pkg.ops.moe_route(torch.randn((T, E), device=gpu, generator=torch.Generator(device=gpu).manual_seed(T)), topk)
+    got = to_f32(pkg.ops.moe_linear(packed, to_dev(xs, gpu, bf16=dtype == "bf16"), routing, gather=True))
+    rows, offsets = routing.sorted_tokens.cpu().numpy(), routing.expert_offsets.cpu().numpy()
+    for e, (qw, qz, sc) in enumerate(parts):
+        own = slice(offsets[e], offsets[e + 1])
+        if own.start < own.stop:
+            want, _ = oracle.linear_forward(xs[rows[own]], oracle.dequant_gptq(qw, qz, sc, None, gs, dtype), None, dtype)
+            assert max_rel_err(got[own], want) <= TOL[dtype]

@@ -4,8 +4,8 @@
 namespace q4host {
 
 void launch_batch_awq_g32(const BatchParams& bp, int dtype, int mt, int wk, bool fuse, dim3 grid, hipStream_t stream) {
-  if (dtype == Q4_DTYPE_F16) batch_rows_awq<Q4_DTYPE_F16, true>(bp, mt, wk, fuse, grid, stream);
-  else batch_rows_awq<Q4_DTYPE_BF16, true>(bp, mt, wk, fuse, grid, stream);
+  if (dtype == Q4_DTYPE_F16) batch_rows_awq<Q4_DTYPE_F16, 32>(bp, mt, wk, fuse, grid, stream);
+  else batch_rows_awq<Q4_DTYPE_BF16, 32>(bp, mt, wk, fuse, grid, stream);
 }
 
 }  // namespace q4host

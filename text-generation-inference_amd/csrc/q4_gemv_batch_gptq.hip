@@ -1,11 +1,11 @@
-// Batch decode kernel, dense launches over GPTQ weights (instantiations).
+// Batch decode kernel, dense launches over GPTQ weights in groups of 128 rows and more (instantiations).
 #include "q4_gemv_batch_launch.cuh"
 
 namespace q4host {
 
 void launch_batch_gptq(const BatchParams& bp, int dtype, int mt, int nq, int wk, bool fuse, dim3 grid, hipStream_t stream) {
-  if (dtype == Q4_DTYPE_F16) batch_rows_gptq<Q4_DTYPE_F16, false>(bp, mt, nq, wk, fuse, grid, stream);
-  else batch_rows_gptq<Q4_DTYPE_BF16, false>(bp, mt, nq, wk, fuse, grid, stream);
+  if (dtype == Q4_DTYPE_F16) batch_rows_gptq<Q4_DTYPE_F16, 128>(bp, mt, nq, wk, fuse, grid, stream);
+  else batch_rows_gptq<Q4_DTYPE_BF16, 128>(bp, mt, nq, wk, fuse, grid, stream);
 }
 
 }  // namespace q4host

@@ -1,36 +1,11 @@
-// Batch decode kernel, grouped launches over stacked GPTQ experts (instantiations).
-#include "q4_gemv_batch.cuh"
+// Batch decode kernel, grouped launches over stacked GPTQ experts in groups of 128 rows and more (instantiations).
+#include "q4_gemv_batch_launch.cuh"
 
 namespace q4host {
 
-using q4::BatchParams;
-
-template <int DTYPE, int MT, int NQ, int WK>
-static void launch_one(const BatchParams& bp, bool fuse, dim3 grid, hipStream_t stream) {
-  using namespace q4;
-  if (fuse) hipLaunchKernelGGL((gemv_batch_kernel<DTYPE, kBatchGptq, MT, NQ, 1, WK, true, true>), grid, dim3(64 * WK), 0, stream, bp);
-  else hipLaunchKernelGGL((gemv_batch_kernel<DTYPE, kBatchGptq, MT, NQ, 1, WK, false, true>), grid, dim3(64 * WK), 0, stream, bp);
-}
-
-template <int DTYPE, int MT>
-static void launch_tile(const BatchParams& bp, int nq, int wk, bool fuse, dim3 grid, hipStream_t stream) {
-  if (nq == 1 && wk == 8) launch_one<DTYPE, MT, 1, 8>(bp, fuse, grid, stream);
-  else if (nq == 1) launch_one<DTYPE, MT, 1, 4>(bp, fuse, grid, stream);
-  else if (wk == 8) launch_one<DTYPE, MT, 2, 8>(bp, fuse, grid, stream);
-  else launch_one<DTYPE, MT, 2, 4>(bp, fuse, grid, stream);
-}
-
-template <int DTYPE>
-static void launch_rows(const BatchParams& bp, int mt, int nq, int wk, bool fuse, dim3 grid, hipStream_t stream) {
-  if (mt == 1) launch_tile<DTYPE, 1>(bp, nq, wk, fuse, grid, stream);
-  else if (mt == 2) launch_tile<DTYPE, 2>(bp, nq, wk, fuse, grid, stream);
-  else if (mt == 3) launch_tile<DTYPE, 3>(bp, nq, wk, fuse, grid, stream);
-  else launch_tile<DTYPE, 4>(bp, nq, wk, fuse, grid, stream);
-}
-
 void launch_batch_moe(const BatchParams& bp, int dtype, int mt, int nq, int wk, bool fuse, dim3 grid, hipStream_t stream) {
-  if (dtype == Q4_DTYPE_F16) launch_rows<Q4_DTYPE_F16>(bp, mt, nq, wk, fuse, grid, stream);
-  else launch_rows<Q4_DTYPE_BF16>(bp, mt, nq, wk, fuse, grid, stream);
+  if (dtype == Q4_DTYPE_F16) batch_rows_moe<Q4_DTYPE_F16, 128>(bp, mt, nq, wk, fuse, grid, stream);
+  else batch_rows_moe<Q4_DTYPE_BF16, 128>(bp, mt, nq, wk, fuse, grid, stream);
 }
 
 }  // namespace q4host
