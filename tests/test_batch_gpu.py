@@ -317,3 +317,20 @@ def test_experts_in_groups_of_64(pkg, oracle, gpu, T, dtype):
         if own.start < own.stop:
             want, _ = oracle.linear_forward(xs[rows[own]], oracle.dequant_gptq(qw, qz, sc, None, gs, dtype), None, dtype)
             assert max_rel_err(got[own], want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("K,N,M,dtype", [(16640, 192, 13, "bf16"), (16640, 192, 37, "f16"), (2176, 16384, 37, "f16"), (2176, 16384, 5, "f16"),
+                                         (2176, 32768, 20, "bf16"), (3200, 8192, 16, "f16")])
+def test_unequal_ranges_of_eight_waves(pkg, oracle, gpu, K, N, M, dtype):
+    """Two chunks a wave and more, with and without left-over ones: the older waves of a workgroup take the longer ranges.  Each row of x meets
+    one row of the weights, so that a range left out or met twice shows in every column."""
+    pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, 128, K + M, dtype)
+    bf = dtype == "bf16"
+    w = torch.from_numpy(oracle.to_f32(w, dtype) if bf else w.astype(np.float32)).to(gpu)
+    for k0 in range(0, K, M * 61):
+        ks = torch.arange(M, device=gpu) * 61 % K + k0
+        ks = ks[ks < K]
+        x = torch.zeros((M, K), dtype=torch.bfloat16 if bf else torch.float16, device=gpu)
+        x[torch.arange(len(ks), device=gpu), ks] = 1
+        got = pkg.ops.linear(pk, x).float()[: len(ks)]
+        assert bool(((got - w[ks]).abs() <= 2.0 ** (-7 if bf else -10) * w[ks].abs()).all())  # (one weight, rounded once or twice)
