@@ -104,7 +104,7 @@ int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, i
  * q4_linear_gate_up_act_order) run for this problem with a workspace: a Q4_PATH_* or one of the Q4_KERNEL_* below (an
  * answer only, no path to ask for); Q4_PATH_AUTO when no gated kernel takes it.  A pure function of (w's geometry, M, dtype).
  */
-#define Q4_KERNEL_BATCH 4 /* up to 64 rows: GPTQ, act-order (its own variant) and AWQ */
+#define Q4_KERNEL_BATCH 4 /* up to 64 rows: GPTQ, act-order (its own variant) and AWQ (one to four rows: its own variant) */
 #define Q4_KERNEL_TALL 5  /* prefill, tiles of 96 to 256 rows, one wave per SIMD */
 #define Q4_KERNEL_BLOCK 6 /* prefill, tiles of 256 x 256, fp16 */
 int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);

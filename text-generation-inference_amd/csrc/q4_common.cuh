@@ -234,11 +234,21 @@ size_t gemv_direct_workspace_bytes(const q4_weight* w, int M, int dtype, int spl
 bool gemv_direct_default(const q4_weight* w, int M, int dtype, int* wk, int* splits);
 int launch_gemv_direct(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, void* workspace,
                        size_t workspace_bytes, int wk, int splits, hipStream_t stream);
+// AWQ, one to four rows (q4_gemv_awq_few.cuh)
+struct AwqFewPlan {
+  int wn;      // column waves of a workgroup; 0: no plan
+  int wk;      // K waves
+  int splits;  // workgroups along K, up to 16
+};
+bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan);
+int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act, void* workspace,
+                   size_t workspace_bytes, const AwqFewPlan& plan, hipStream_t stream);
 // the batch decode kernel (q4_gemv_batch.cuh): up to 64 rows, GPTQ (contiguous groups) and AWQ
 struct BatchPlan {
   int nq;      // wave tile: 1 = 64 columns, 2 = 128
   int wk;      // K waves per workgroup
   int splits;  // workgroups along K: 1, 2, 4 or 8
+  AwqFewPlan few = {0, 0, 0};  // wn > 0: launch_batch runs the AWQ kernel for few rows in its place
 };
 bool batch_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan);
 int launch_batch(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act,
