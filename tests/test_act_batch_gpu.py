@@ -111,3 +111,34 @@ def test_replays(pkg, oracle, gpu):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(outs, want))
         assert torch.equal(pkg.ops.linear(pk, x), want[0])
+
+
+@pytest.mark.parametrize("K,N,gs", [(4096, 28672, 128), (2048, 24576, 64), (2176, 49152, 128), (5504, 192, 128), (4608, 4608, 128), (18944, 256, 256)])
+@pytest.mark.parametrize("M,dtype", [(1, "f16"), (3, "bf16"), (4, "f16"), (5, "f16"), (16, "f16"), (37, "bf16")])
+@pytest.mark.parametrize("sym", [False, True])
+def test_tiles_and_splits(pkg, oracle, gpu, K, N, gs, M, dtype, sym):
+    """128-column tiles of the gated epilogue in one round and in workgroups along K, x of a few rows through LDS over long ranges, splits
+    that are no power of two; one zero point and several."""
+    if K * N * M > 2.5e9:
+        M = 5 if M == 37 else M
+    bf = dtype == "bf16"
+    qw, qz, sc, gi = oracle.make_gptq(K, N, gs, seed=K + M, sym=sym, act_order=True)
+    w = oracle.dequant_gptq(qw, qz, sc, gi, gs, dtype)
+    pk = pkg.ops.make_packed(to_dev(qw, gpu), to_dev(qz, gpu), to_dev(sc, gpu), to_dev(gi, gpu), gs, 0)
+    x = oracle.make_x(M, K, seed=M, dtype=dtype)
+    xt = to_dev(x, gpu, bf16=bf)
+    y32, _ = oracle.linear_forward(x, w, None, dtype)
+    got = pkg.ops.linear(pk, xt)
+    assert torch.equal(got, pkg.ops.linear(pk, xt))
+    assert max_rel_err(to_f32(got), y32) <= (8e-3 if bf else 2e-3)
+    if N % 128 == 0:
+        _, want = oracle.gate_up_forward(x, w, "silu", None, dtype)
+        gated = pkg.ops.linear_gate_up(pk, xt, "silu")
+        assert torch.equal(gated, pkg.ops.linear_gate_up(pk, xt, "silu"))
+        assert max_rel_err(to_f32(gated), oracle.to_f32(want, dtype)) <= (1.2e-2 if bf else 2e-3)
+    # one-hot rows read the rounded weights back bit for bit
+    hot = torch.zeros_like(xt)
+    ks = (torch.arange(M) * 997 + 13) % K
+    hot[torch.arange(M), ks] = 1
+    back = pkg.ops.linear(pk, hot).cpu().view(torch.int16).numpy().view(np.uint16)
+    assert np.array_equal(back & 0x7FFF, w[ks.numpy()].view(np.uint16) & 0x7FFF)  # (a zero may have lost its sign)
