@@ -22,7 +22,7 @@ CSRC = HERE / "csrc"
 LIB_NAME = "libq4linear.so"
 LIB_PATH = HERE / LIB_NAME
 
-SOURCES = ["q4_api.hip", "q4_dequant.hip", "q4_generic.hip", "q4_gemv.hip", "q4_gemv_lean.hip", "q4_gemv_direct.hip", "q4_gemv_awq.hip", "q4_gemv_awq_few.hip", "q4_gemv_gate_up.hip", "q4_gemv_batch.hip", "q4_gemv_batch_gptq.hip", "q4_gemv_batch_awq.hip", "q4_gemv_batch_gptq_g64.hip", "q4_gemv_batch_awq_g64.hip", "q4_gemv_batch_moe_g64.hip", "q4_gemv_batch_gptq_g32.hip", "q4_gemv_batch_awq_g32.hip", "q4_gemv_batch_moe.hip", "q4_gemv_batch_act.hip", "q4_gemm.hip", "q4_gemm_awq.hip", "q4_gemm_awq_direct.hip", "q4_gemm_tall.hip", "q4_gemm_tall_gptq_f16.hip", "q4_gemm_tall_gptq_bf16.hip", "q4_gemm_tall_awq_f16.hip", "q4_gemm_tall_awq_bf16.hip", "q4_act_mul.hip", "q4_moe.hip", "q4_sequential.hip", "q4_gptq_solve.hip"]
+SOURCES = ["q4_api.hip", "q4_dequant.hip", "q4_generic.hip", "q4_gemv.hip", "q4_gemv_lean.hip", "q4_gemv_direct.hip", "q4_gemv_awq.hip", "q4_gemv_awq_few.hip", "q4_gemv_awq_wide.hip", "q4_gemv_gate_up.hip", "q4_gemv_batch.hip", "q4_gemv_batch_gptq.hip", "q4_gemv_batch_awq.hip", "q4_gemv_batch_gptq_g64.hip", "q4_gemv_batch_awq_g64.hip", "q4_gemv_batch_moe_g64.hip", "q4_gemv_batch_gptq_g32.hip", "q4_gemv_batch_awq_g32.hip", "q4_gemv_batch_moe.hip", "q4_gemv_batch_act.hip", "q4_gemm.hip", "q4_gemm_awq.hip", "q4_gemm_awq_direct.hip", "q4_gemm_tall.hip", "q4_gemm_tall_gptq_f16.hip", "q4_gemm_tall_gptq_bf16.hip", "q4_gemm_tall_awq_f16.hip", "q4_gemm_tall_awq_bf16.hip", "q4_act_mul.hip", "q4_moe.hip", "q4_sequential.hip", "q4_gptq_solve.hip"]
 # translation units that see the decode kernels' parameter block (recompiled for the stamps build)
 STAMP_SOURCES = ["q4_gemv.hip", "q4_gemv_lean.hip", "q4_gemv_direct.hip", "q4_gemv_direct.hip", "q4_gemv_awq.hip", "q4_gemv_gate_up.hip", "q4_moe.hip"]
 PROBE_LIB_PATH = HERE / "libq4probe.so"

@@ -240,7 +240,10 @@ struct AwqFewPlan {
   int wk;      // K waves
   int splits;  // workgroups along K, up to 16
 };
+bool awq_few_supported(const q4_weight* w, int M, bool gate_up);
 bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan);
+// five to sixteen rows (q4_gemv_awq_wide.cuh); launched by launch_awq_few
+bool awq_wide_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan);
 int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act, void* workspace,
                    size_t workspace_bytes, const AwqFewPlan& plan, hipStream_t stream);
 // the batch decode kernel (q4_gemv_batch.cuh): up to 64 rows, GPTQ (contiguous groups) and AWQ

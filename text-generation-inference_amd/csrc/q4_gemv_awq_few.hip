@@ -1,14 +1,17 @@
-// AWQ decode kernel for one to four rows (q4_gemv_awq_few.cuh): what it takes, its decomposition, and the launches.
+// AWQ decode kernel for one to four rows (q4_gemv_awq_few.cuh): what it takes, its decomposition, and the launches (those of
+// q4_gemv_awq_wide.cuh, which takes the same weights at more rows, go through here).
 #include "q4_gemv_awq_few.cuh"
 
 namespace q4host {
 
 using q4::AwqFewParams;
 
+void launch_awq_wide(const AwqFewParams& p, int dtype, const AwqFewPlan& plan, bool fuse, hipStream_t stream);
+
 // Groups of 128 << s rows (or one group), K in whole 128-row chunks, N in whole wave tiles of 256 columns (gated epilogue: gate and
 // up half each), tensors below 2 GB (32-bit offsets).
-static bool awq_few_supported(const q4_weight* w, int M, bool gate_up) {
-  if (w->layout != Q4_LAYOUT_AWQ || M < 1 || M > q4::kAwqFewRows) return false;
+bool awq_few_supported(const q4_weight* w, int M, bool gate_up) {
+  if (w->layout != Q4_LAYOUT_AWQ || M < 1) return false;
   if (w->K % 128 != 0 || w->K < 128 || w->N % (gate_up ? 512 : 256) != 0) return false;
   if (w->num_groups > 1) {
     const int per = w->groupsize / 128;
@@ -57,7 +60,7 @@ static bool awq_few_plan(const q4_weight* w, int M, bool gate_up, AwqFewPlan* pl
 // 57344 0.95-1.03).
 bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan) {
   if (gate_up ? w->K <= (dtype == Q4_DTYPE_BF16 ? 2048 : 1024) : w->K < 2048 || (long)w->K * w->N >= (1L << 28)) return false;
-  return awq_few_supported(w, M, gate_up) && awq_few_plan(w, M, gate_up, plan);
+  return M <= q4::kAwqFewRows && awq_few_supported(w, M, gate_up) && awq_few_plan(w, M, gate_up, plan);
 }
 
 template <int DTYPE>
@@ -73,6 +76,10 @@ int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y,
                    size_t workspace_bytes, const AwqFewPlan& plan, hipStream_t stream) {
   const bool cells = workspace != nullptr && workspace_bytes >= Q4_WORKSPACE_COUNTER_BYTES;
   const int splits = cells ? plan.splits : 1;
+  if (M > q4::kAwqFewRows && !cells) {
+    set_error("q4_linear(AWQ, five to sixteen rows): a workspace of Q4_WORKSPACE_COUNTER_BYTES is needed");
+    return Q4_ERR_WORKSPACE;
+  }
   AwqFewParams p;
   p.qweight = w->qweight;
   p.qzeros = w->qzeros;
@@ -80,7 +87,7 @@ int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y,
   p.x = x;
   p.bias = bias;
   p.y = y;
-  p.cells = splits > 1 ? (unsigned long long*)((char*)workspace + Q4_WORKSPACE_TICKET_BYTES) : nullptr;
+  p.cells = cells ? (unsigned long long*)((char*)workspace + Q4_WORKSPACE_TICKET_BYTES) : nullptr;
   p.N = w->N;
   p.K = w->K;
   p.M = M;
@@ -95,7 +102,8 @@ int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y,
   p.splits = splits;
   p.act = gate_up_act != 0 ? gate_up_act - 1 : 0;
   const dim3 grid((unsigned)(w->N / (256 * plan.wn)), (unsigned)splits);
-  if (dtype == Q4_DTYPE_F16) launch_dtype<Q4_DTYPE_F16>(p, plan.wn, plan.wk, gate_up_act != 0, grid, stream);
+  if (M > q4::kAwqFewRows) launch_awq_wide(p, dtype, plan, gate_up_act != 0, stream);
+  else if (dtype == Q4_DTYPE_F16) launch_dtype<Q4_DTYPE_F16>(p, plan.wn, plan.wk, gate_up_act != 0, grid, stream);
   else launch_dtype<Q4_DTYPE_BF16>(p, plan.wn, plan.wk, gate_up_act != 0, grid, stream);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
