@@ -334,3 +334,22 @@ def test_unequal_ranges_of_eight_waves(pkg, oracle, gpu, K, N, M, dtype):
         x[torch.arange(len(ks), device=gpu), ks] = 1
         got = pkg.ops.linear(pk, x).float()[: len(ks)]
         assert bool(((got - w[ks]).abs() <= 2.0 ** (-7 if bf else -10) * w[ks].abs()).all())  # (one weight, rounded once or twice)
+
+
+# (decompositions that are no power of two, or another tile than the plan of powers of two: three workgroups along K of 128- and of 64-column
+# tiles, whole K ranges of four waves, an odd one out with ragged chunks)
+@pytest.mark.parametrize("K,N,M,dtype,gated", [(8192, 10240, 16, "f16", False), (3584, 4608, 13, "bf16", False), (4096, 22016, 8, "f16", True), (3584, 37888, 13, "bf16", True),
+                                               (9088, 6400, 10, "f16", False), (8192, 10240, 40, "bf16", False), (5504, 4736, 24, "f16", True)])
+def test_any_number_of_splits(pkg, oracle, gpu, K, N, M, dtype, gated):
+    pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, 128, M, dtype)
+    x = oracle.make_x(M, K, seed=M, dtype=dtype)
+    xt = to_dev(x, gpu, bf16=dtype == "bf16")
+    if gated:
+        _, want = oracle.gate_up_forward(x, w, "silu", None, dtype)
+        got, again = (pkg.ops.linear_gate_up(pk, xt, "silu") for _ in range(2))
+        assert max_rel_err(to_f32(got), oracle.to_f32(want, dtype)) <= TOL_GATED[dtype]
+    else:
+        y32, _ = oracle.linear_forward(x, w, None, dtype)
+        got, again = (pkg.ops.linear(pk, xt) for _ in range(2))
+        assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
+    assert torch.equal(got, again)

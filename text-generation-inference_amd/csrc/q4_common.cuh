@@ -250,7 +250,7 @@ int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y,
 struct BatchPlan {
   int nq;      // wave tile: 1 = 64 columns, 2 = 128
   int wk;      // K waves per workgroup
-  int splits;  // workgroups along K: 1, 2, 4 or 8
+  int splits;  // workgroups along K, up to 16
   AwqFewPlan few = {0, 0, 0};  // wn > 0: launch_batch runs the AWQ kernel for few rows in its place
 };
 bool batch_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan);
