@@ -339,7 +339,8 @@ def test_unequal_ranges_of_eight_waves(pkg, oracle, gpu, K, N, M, dtype):
 # (decompositions that are no power of two, or another tile than the plan of powers of two: three workgroups along K of 128- and of 64-column
 # tiles, whole K ranges of four waves, an odd one out with ragged chunks)
 @pytest.mark.parametrize("K,N,M,dtype,gated", [(8192, 10240, 16, "f16", False), (3584, 4608, 13, "bf16", False), (4096, 22016, 8, "f16", True), (3584, 37888, 13, "bf16", True),
-                                               (9088, 6400, 10, "f16", False), (8192, 10240, 40, "bf16", False), (5504, 4736, 24, "f16", True)])
+                                               (9088, 6400, 10, "f16", False), (3584, 37888, 1, "f16", True), (4096, 22016, 2, "f16", True), (8960, 2304, 1, "bf16", True),
+                                               (3584, 4608, 1, "bf16", False), (8192, 10240, 40, "bf16", False), (5504, 4736, 24, "f16", True)])
 def test_any_number_of_splits(pkg, oracle, gpu, K, N, M, dtype, gated):
     pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, 128, M, dtype)
     x = oracle.make_x(M, K, seed=M, dtype=dtype)
