@@ -81,6 +81,29 @@ def test_splits_of_the_picked_kernels(pkg, oracle, gpu, layout, M, K, N, gs, dty
     assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
 
 
+# GPTQ, two halves of K in a workgroup: 96-, 128- and 160-row tiles, ragged and full, with and without splits, four K tiles a half
+# (1024 x 8192) and more, groups of 64 and one group
+@pytest.mark.parametrize("M,K,N,gs,dtype", [(100, 4096, 4096, 128, "f16"), (96, 3584, 8192, 64, "f16"), (301, 1024, 8192, 1024, "f16"), (301, 1024, 8192, 64, "bf16"),
+                                            (420, 1024, 8192, 128, "f16"), (160, 14336, 4096, 128, "bf16"), (161, 8192, 8192, 128, "f16"), (640, 3584, 8192, 128, "f16")])
+def test_two_halves_of_k(pkg, oracle, gpu, M, K, N, gs, dtype):
+    pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, gs, K + M, dtype)
+    bf = dtype == "bf16"
+    assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16) == "tall"
+    x = oracle.make_x(M, K, seed=M, dtype=dtype)
+    b32 = np.random.default_rng(M).standard_normal(N).astype(np.float32)
+    bias = oracle.f32_to_bf16_bits(b32) if bf else b32.astype(np.float16)
+    y32, _ = oracle.linear_forward(x, w, bias, dtype)
+    xt, bt = to_dev(x, gpu, bf16=bf), to_dev(bias, gpu, bf16=bf)
+    got = pkg.ops.linear(pk, xt, bt)
+    assert torch.equal(got, pkg.ops.linear(pk, xt, bt))
+    assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
+    clean = got.clone()
+    xt[3, K // 2], xt[M - 1, 5] = float("inf"), float("nan")
+    got = pkg.ops.linear(pk, xt, bt)
+    keep = [r for r in range(M) if r not in (3, M - 1)]
+    assert torch.equal(got[keep], clean[keep]) and bool(torch.isnan(got[M - 1]).all()) and not bool(torch.isfinite(got[3]).any())
+
+
 @pytest.mark.parametrize("layout", ["gptq", "awq"])
 def test_non_finite_rows_stay_alone(pkg, oracle, gpu, layout):
     """An infinite or undefined activation changes its own row only, the last row of a ragged tile included."""

@@ -306,6 +306,7 @@ struct TallPlan {
   int r;       // tile height in blocks of 32 rows: 3 .. 6 or 8
   bool block;  // 8 blocks, fp16: the 256 x 256 kernel of eight waves
   int splits;  // workgroups along K
+  int kw = 1;  // 2: two halves of K and 128 columns a workgroup
 };
 double gemm_round_us(long wgs, int slots, double kt, double alone, double full);
 double gemm_estimate_us(const q4_weight* w, int M, bool gate_up);

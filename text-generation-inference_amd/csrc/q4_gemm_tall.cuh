@@ -15,6 +15,9 @@
 //   * The activations stay in their own K order, so GPTQ words are unpacked byte by byte (16 operations per word of eight).
 // Measured on MI355X, us, 128 x 256 tiles (two workgroups per CU, 384 rows padded) / this kernel with 160-row
 // tiles: 4096 x 28672 gated at 301 rows 109 / 78, 14336 x 4096 57 / 49.
+// GPTQ tiles of up to 160 rows may split K inside the workgroup (KW = 2): two column waves times two halves of K, each half with its own ring of
+// activation tiles (160 KB of LDS at 160 rows), whose sums meet in LDS.  Half the partial sums that go through memory for as many
+// workgroups: 3584 x 8192 at 301 rows 34.4 us / 28.9; the rule is tall_plan's.
 // Quantisation groups are multiples of 64 rows (one group per K tile).
 #pragma once
 
@@ -98,20 +101,25 @@ __device__ __forceinline__ void awq_unpack_half(uint32_t w0, uint32_t w1, uint32
   hi = o[1];
 }
 
-template <int DTYPE, int LAYOUT, int R, bool FUSE>
+// KW = 2: the workgroup's waves are two column waves times two halves of its K range, which meet in LDS; its tile is 128 columns.
+template <int DTYPE, int LAYOUT, int R, bool FUSE, int KW = 1>
 __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
+  static_assert(KW == 1 || (!FUSE && R <= 5), "two K halves: plain launches, whose rings fit LDS");
   constexpr bool AWQ = LAYOUT == kTileAwq;
   constexpr int BM = 32 * R;
   constexpr int WAVES = 4;
   constexpr int A_BLOCKS = BM / 8;                // 8 rows x 128 bytes of the activation tile: one load of a wave
-  constexpr int A_LOADS = A_BLOCKS / WAVES;            // of a wave
+  constexpr int CW = WAVES / KW;                       // column waves, which load their K half's tile
+  constexpr int BN = kTallBN / KW;
+  constexpr int A_LOADS = A_BLOCKS / CW;               // of a wave
   constexpr int FR = kKSteps * R;                  // A fragments of a wave per K tile
   // four arrays: the compiler then knows which outstanding load a fragment read has to wait for
-  __shared__ uint4_t ring0[BM * 8], ring1[BM * 8], ring2[BM * 8], ring3[BM * 8];
+  __shared__ uint4_t ring0[KW * BM * 8], ring1[KW * BM * 8], ring2[KW * BM * 8], ring3[KW * BM * 8];
   const Problem& p = gp.p;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & (WAVES - 1);  // (known range: LDS addresses fold into offsets)
+  const int cw = wave % CW, kh = wave / CW;  // column wave, K half
   const int j = lane & 31;
   const int kq = lane >> 5;
   const int N = p.N, K = p.K, M = p.M;
@@ -120,7 +128,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
   // M tiles (activations in its L2) and walks the column blocks; otherwise it takes a few column blocks and
   // all their M tiles.
   const int tiles_m = (M + BM - 1) / BM;
-  const int tiles_n = N / kTallBN;
+  const int tiles_n = N / BN;
   const int total = tiles_m * tiles_n;
   const int split = blockIdx.x / total;
   int tm, tn;
@@ -142,14 +150,15 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
   const int m0 = tm * BM;
   const int half = N >> 1;
   // first column of this wave (gated epilogue: waves wave = 0, 1 the gate columns, 2, 3 the up columns that go with them)
-  const int nw = FUSE ? tn * (kTallBN / 2) + (wave & 1) * 64 + (wave >> 1) * half : tn * kTallBN + wave * 64;
+  const int nw = FUSE ? tn * (kTallBN / 2) + (wave & 1) * 64 + (wave >> 1) * half : tn * BN + cw * 64;
   // the two columns this lane finishes start here; AWQ: lane j unpacks byte j % 4 of word j / 4, columns acol and acol + 2
   const int ncol = AWQ ? nw + 8 * (j >> 2) + ((j & 1) << 2) + (j & 2) : nw + 2 * j;
   const int acol = nw + 8 * (j >> 2) + ((j & 1) << 2) + ((j >> 1) & 1);
 
   const int KT_all = K / kBK;
-  const int kt0 = (int)((long)split * KT_all / gp.splits);
-  const int KT = (int)((long)(split + 1) * KT_all / gp.splits) - kt0;
+  // (KW = 2: the host sees to whole halves)
+  const int kt_first = (int)((long)split * KT_all / gp.splits), kt_count = (int)((long)(split + 1) * KT_all / gp.splits) - kt_first;
+  const int KT = kt_count / KW, kt0 = kt_first + kh * KT;
   const int last_tile = KT - 1;
 
   // ---- packed words of a 16-row step.  GPTQ: row 8 kt + 2 s + kq, columns ncol, ncol + 1.  AWQ: rows
@@ -210,19 +219,19 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
     }
   };
 
-  // ---- activation tile: global -> LDS.  Load i of a wave covers rows 8 (wave + 4 i) .. + 7, the LDS unit lane % 8 of a
+  // ---- activation tile: global -> LDS.  Load i of a wave covers rows 8 (cw + CW i) .. + 7, the LDS unit lane % 8 of a
   // row receives its unit (lane % 8) ^ (row / 2 % 8).
   const buffer_rsrc_t xrsrc = make_rsrc(p.x, (uint32_t)M * (uint32_t)K * 2u);  // host: below 2 GB
   // Rows past M lie past the end of x: such a load touches no memory.
-  const int a_row0 = 8 * wave + (lane >> 3);
+  const int a_row0 = 8 * cw + (lane >> 3);
   const uint32_t a_off0 = ((uint32_t)(m0 + a_row0) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((a_row0 >> 1) & 7)) * 8u) * 2u;
-  const uint32_t a_step = (uint32_t)K * (16u * WAVES);  // 8 WAVES rows
+  const uint32_t a_step = (uint32_t)K * (16u * CW);  // 8 CW rows
   auto load_a = [&](int kt, uint4_t* ring) {
     const uint32_t tile_off = uniform_u32((uint32_t)(kt0 + min(kt, last_tile)) * (kBK * 2));
     uint32_t off = a_off0;
     asm volatile("" : "+v"(off));  // (added up for every tile: as loop invariants the sums cost a register each)
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) load_to_lds(xrsrc, ring + (wave + WAVES * i) * 64, off + (uint32_t)i * a_step, tile_off);
+    for (int i = 0; i < A_LOADS; ++i) load_to_lds(xrsrc, ring + kh * (BM * 8) + (cw + CW * i) * 64, off + (uint32_t)i * a_step, tile_off);
   };
 
   float16_t acc[R][2];
@@ -235,7 +244,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
 
   // A fragment g of a tile (g = s * R + mt): the wave's rows 32 mt + j, K unit 2 s + kq (swizzled)
   const int a_swz = (j >> 1) & 7;
-  const int a_row = (j) * 8;
+  const int a_row = kh * (BM * 8) + j * 8;
   int a_lane[kKSteps];
 #pragma unroll
   for (int s = 0; s < kKSteps; ++s) a_lane[s] = a_row + ((2 * s + kq) ^ a_swz);
@@ -338,6 +347,36 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the tiles asked for past the end still write the ring)
 
+  if constexpr (KW == 2) {
+    // The K halves hand each other half of their sums through LDS (a column wave's in one array, 8 R KB): half 0 finishes registers 0 .. 7 of
+    // every fragment, half 1 the others.
+    __syncthreads();
+    float4_t* xch = (float4_t*)(cw ? ring1 : ring0) + lane;
+#pragma unroll
+    for (int mt = 0; mt < R; ++mt)
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float4_t v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = kh ? acc[mt][f][4 * q + i] : acc[mt][f][8 + 4 * q + i];
+          xch[(((kh * R + mt) * 2 + f) * 2 + q) * 64] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < R; ++mt)
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const float4_t v = xch[((((1 - kh) * R + mt) * 2 + f) * 2 + q) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[mt][f][4 * q + i] = (kh ? acc[mt][f][8 + 4 * q + i] : acc[mt][f][4 * q + i]) + v[i];
+        }
+  }
+  constexpr int REGS = 16 / KW;  // of a fragment that the wave finishes, from 8 kh on
+
   // ---- epilogue.  C layout of the 32x32 MFMA: register r of lane (j, kq) is row 8 (r / 4) + 4 kq + r % 4, column j of
   // the fragment.  GPTQ: fragment f is column ncol + f.  AWQ: columns acol, acol + 2; lanes j and j ^ 2 swap one of
   // their two sums, then each owns ncol and ncol + 1 as well.
@@ -351,14 +390,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
       return float2_t{a, b};
     }
   };
-  auto row_of = [&](int mt, int r) { return m0 + mt * 32 + 8 * (r >> 2) + 4 * kq + (r & 3); };
+  auto row_of = [&](int mt, int r) { return m0 + mt * 32 + (KW == 2 ? 16 * kh : 0) + 8 * (r >> 2) + 4 * kq + (r & 3); };
   if (gp.splits > 1) {
     // fp32 partial tile; bias, rounding and the store to y happen in the reduction kernel
     float* part = gp.partials + (size_t)split * gp.partial_rows * N;
 #pragma unroll
     for (int mt = 0; mt < R; ++mt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
+      for (int r = 0; r < REGS; ++r) {
         const int m = row_of(mt, r);
         const float2_t v = sums(mt, r);
         if (m < M) *(float2_t*)(part + (size_t)m * N + ncol) = v;
@@ -428,7 +467,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmParams gp) {
 #pragma unroll
   for (int mt = 0; mt < R; ++mt)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < REGS; ++r) {
       const int m = row_of(mt, r);
       const uint32_t o = finish2(mt, r);
       if (m < M) *(uint32_t*)(y + (size_t)m * N + ncol) = o;

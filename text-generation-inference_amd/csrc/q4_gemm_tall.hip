@@ -7,10 +7,10 @@ namespace q4host {
 using q4::GemmParams;
 using q4::Problem;
 
-void launch_tall_gptq_f16(const GemmParams& gp, int r, bool fuse, dim3 grid, hipStream_t stream);
-void launch_tall_gptq_bf16(const GemmParams& gp, int r, bool fuse, dim3 grid, hipStream_t stream);
-void launch_tall_awq_f16(const GemmParams& gp, int r, bool fuse, dim3 grid, hipStream_t stream);
-void launch_tall_awq_bf16(const GemmParams& gp, int r, bool fuse, dim3 grid, hipStream_t stream);
+void launch_tall_gptq_f16(const GemmParams& gp, int r, int kw, bool fuse, dim3 grid, hipStream_t stream);
+void launch_tall_gptq_bf16(const GemmParams& gp, int r, int kw, bool fuse, dim3 grid, hipStream_t stream);
+void launch_tall_awq_f16(const GemmParams& gp, int r, int kw, bool fuse, dim3 grid, hipStream_t stream);
+void launch_tall_awq_bf16(const GemmParams& gp, int r, int kw, bool fuse, dim3 grid, hipStream_t stream);
 void launch_block_gptq(const GemmParams& gp, bool fuse, dim3 grid, hipStream_t stream);
 void launch_block_awq(const GemmParams& gp, bool fuse, dim3 grid, hipStream_t stream);
 
@@ -37,8 +37,8 @@ static double tall_estimate_us(bool awq, int dtype, int M, int K, int N, int r, 
 }
 
 // The plan with the smallest estimate.  K is split while the tiles alone leave CUs idle, at least four K tiles a
-// workgroup, two rounds at most.
-static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, TallPlan* plan) {
+// workgroup, two rounds at most.  halves: K halves inside a workgroup too.
+static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, bool halves, TallPlan* plan) {
   static const int kSplits[] = {1, 2, 3, 4, 6, 8};
   double best = -1.0;
   for (int r = 3; r <= 9; ++r) {
@@ -55,6 +55,27 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
       }
     }
   }
+  if (!halves || gate_up || awq || M > 768) return best;
+  // Two halves of K in a workgroup, 128 columns: as many CUs at work with half the splits, whose fp32 partial sums (8 M N bytes each, out and in)
+  // otherwise cost up to a third of a call; every fragment of x then serves half as many columns, which is why they end where two
+  // splits and less would do.  Fitted to 15 layer shapes x 100-640 rows x all heights and splits, within 7 %; where it puts them 2 % ahead they
+  // are, 28 calls: 1.10 in geometric mean (0.99-1.37); us, before / so: 3584 x 8192 301 rows 34.4 / 28.9, 14336 x 4096 160 rows 36.3 / 33.3, bf16
+  // 38.9 / 33.3, 8192 x 8192 160 rows 39.6 / 35.9, 1024 x 8192 301 rows 18.0 / 13.1.  Over 176
+  // calls of 37 shapes at 65-768 rows, changed or not, 1.05 in geometric mean (0.98).  (AWQ, whose words are loaded row by row, 0.75-1.1: not built in.)
+  static const double kHalves[3][2] = {{0.54, 0.81}, {0.69, 1.00}, {0.85, 1.23}};  // (bf16: 0.065 more)
+  const int KT = K / q4::kBK;
+  for (int r = 3; r <= 5; ++r)
+    for (int sp : kSplits) {
+      const long wgs = (long)((M + 32 * r - 1) / (32 * r)) * (N / (q4::kTallBN / 2)) * sp;
+      if (KT % (2 * sp) != 0 || KT / (2 * sp) < 4 || wgs < 96 || wgs > 1024) continue;
+      const double more = dtype == Q4_DTYPE_BF16 ? 0.065 : 0.0;
+      const double t = 1.02 * (gemm_round_us(wgs, 256, KT / (2 * sp), kHalves[r - 3][0] + more, kHalves[r - 3][1] + more) + 7.7 +
+                               (sp > 1 ? 0.55 + 1.69e-6 * sp * M * N : 0.0));
+      if (t < best) {
+        best = t;
+        *plan = TallPlan{r, false, sp, 2};
+      }
+    }
   return best;
 }
 
@@ -89,7 +110,7 @@ bool gemm_tall_default(const q4_weight* w, int M, int dtype, bool gate_up, TallP
   const bool awq = w->layout == Q4_LAYOUT_AWQ;
   auto others = [&](bool fused) { return awq ? gemm_awq_direct_estimate_us(w, M, dtype) : gemm_estimate_us(w, M, fused); };
   auto taken = [&](double other) {
-    return tall_plan(awq, dtype, M, w->K, w->N, gate_up, plan) * 1.08 < other && !tall_outdone(awq, dtype, M, w->K, w->N, gate_up, *plan);
+    return tall_plan(awq, dtype, M, w->K, w->N, gate_up, true, plan) * 1.08 < other && !tall_outdone(awq, dtype, M, w->K, w->N, gate_up, *plan);
   };
   if (!gate_up) return taken(others(false));
   const bool old_fused = gemm_gate_up_supported(w, M, dtype);
@@ -98,7 +119,7 @@ bool gemm_tall_default(const q4_weight* w, int M, int dtype, bool gate_up, TallP
   if (!old_fused) {
     // two launches: the faster plain kernel, the elementwise one
     TallPlan plain;
-    const double t = tall_plan(awq, dtype, M, w->K, w->N, false, &plain);
+    const double t = tall_plan(awq, dtype, M, w->K, w->N, false, false, &plain);
     other = others(false);
     other = (t < other ? t : other) + 4.0 + (double)M * w->N * 3e-6 / 5.0;
   }
@@ -112,8 +133,10 @@ size_t gemm_tall_workspace_bytes(int M, int K, int N) {
   for (int awq = 0; awq < 2; ++awq)
     for (int dtype : {Q4_DTYPE_F16, Q4_DTYPE_BF16}) {
       TallPlan plan;
-      tall_plan(awq != 0, dtype, M, K, N, false, &plan);
-      if (plan.splits > splits) splits = plan.splits;
+      for (bool halves : {false, true}) {
+        tall_plan(awq != 0, dtype, M, K, N, false, halves, &plan);
+        if (plan.splits > splits) splits = plan.splits;
+      }
     }
   return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
@@ -132,7 +155,7 @@ int launch_gemm_tall(const q4_weight* w, const void* x, const void* bias, void* 
   gp.splits = plan.splits;
   gp.partials = plan.splits > 1 ? (float*)((char*)workspace + Q4_WORKSPACE_COUNTER_BYTES) : nullptr;
   const int bm = 32 * plan.r;
-  const long total = (long)((M + bm - 1) / bm) * (w->N / q4::kTallBN) * plan.splits;
+  const long total = (long)((M + bm - 1) / bm) * (w->N / (q4::kTallBN / plan.kw)) * plan.splits;
   if (total > 0x7fffffffL) {
     set_error("q4_linear(gemm): grid too large");
     return Q4_ERR_UNSUPPORTED;
@@ -140,8 +163,8 @@ int launch_gemm_tall(const q4_weight* w, const void* x, const void* bias, void* 
   const dim3 grid((unsigned)total);
   const bool fuse = gate_up_act != 0, awq = w->layout == Q4_LAYOUT_AWQ;
   if (plan.block) (awq ? launch_block_awq : launch_block_gptq)(gp, fuse, grid, stream);
-  else if (dtype == Q4_DTYPE_F16) (awq ? launch_tall_awq_f16 : launch_tall_gptq_f16)(gp, plan.r, fuse, grid, stream);
-  else (awq ? launch_tall_awq_bf16 : launch_tall_gptq_bf16)(gp, plan.r, fuse, grid, stream);
+  else if (dtype == Q4_DTYPE_F16) (awq ? launch_tall_awq_f16 : launch_tall_gptq_f16)(gp, plan.r, plan.kw, fuse, grid, stream);
+  else (awq ? launch_tall_awq_bf16 : launch_tall_gptq_bf16)(gp, plan.r, plan.kw, fuse, grid, stream);
   if (plan.splits > 1) launch_gemm_reduce(gp.partials, bias, y, M, w->N, plan.splits, dtype, stream);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) {

@@ -4,8 +4,8 @@
 
 namespace q4host {
 
-void launch_tall_awq_bf16(const q4::GemmParams& gp, int r, bool fuse, dim3 grid, hipStream_t stream) {
-  launch_tall<Q4_DTYPE_BF16, q4::kTileAwq>(gp, r, fuse, grid, stream);
+void launch_tall_awq_bf16(const q4::GemmParams& gp, int r, int kw, bool fuse, dim3 grid, hipStream_t stream) {
+  launch_tall<Q4_DTYPE_BF16, q4::kTileAwq>(gp, r, kw, fuse, grid, stream);
 }
 
 }  // namespace q4host
