@@ -82,6 +82,20 @@ def test_gated(pkg, oracle, gpu, K, N, gs):
         assert err <= {"f16": 2e-3, "bf16": 1.2e-2}[dtype]
 
 
+def test_the_decode_path_runs_it_on_the_largest_layers(pkg, gpu):
+    """Five and six rows of 2^28 weights and more stay the decode path's calls; their sums are those of seven rows' batch."""
+    K, N, g = 8192, 32768, torch.Generator(device=gpu).manual_seed(1)
+    words = lambda *s: torch.randint(-(2**31), 2**31 - 1, s, dtype=torch.int32, device=gpu, generator=g)  # noqa: E731
+    pk = pkg.ops.make_packed(words(K, N // 8), words(K // 128, N // 8), (torch.rand((K // 128, N), device=gpu, generator=g) * 0.02).half(), None, 128, 1)
+    x = _rand(gpu, "f16", 1, 7, K)
+    seven = pkg.ops.linear(pk, x)
+    for M in (5, 6):
+        assert pkg.ops.kernel_of(pk, M) == "gemv"
+        got = pkg.ops.linear(pk, x[:M])
+        # (other K deals: fp32 sums in another order, so neighbouring outputs)
+        assert float((got.double() - seven[:M].double()).abs().max() / seven.double().abs().max()) <= 2.0**-10
+
+
 def test_without_a_workspace_the_batch_kernel_answers(pkg, oracle, gpu):
     """The C entry, no workspace: gate and up tiles could not meet."""
     import ctypes
