@@ -178,6 +178,22 @@ def test_workspace_sizing_other_group_sizes_and_70b_shapes(pkg):
                             assert rc != L.ERR_WORKSPACE, ("gate_up", K, N, gs, M, dt, lib.q4_last_error())
 
 
+@pytest.mark.parametrize("K,N,gs,without", [(65536, 24576, 1024, True), (65536, 28672, 1024, True), (65536, 32768, 1024, True), (65536, 57344, 1024, True),
+                                            (61440, 49152, 640, True), (81920, 24576, 81920, False), (131072, 28672, 131072, False), (8192, 57344, 128, True)])
+def test_gated_act_order_plan_and_launch_agree(pkg, K, N, gs, without):
+    """A gated act-order call that the plan says is one launch is not refused for its LDS: with a full workspace never, without one where
+    the groups of all K rows fit beside the table of 64 columns."""
+    lib, L, fused = pkg._lib.load(), pkg._lib, ctypes.c_int(0)
+    for M in (1, 4, 5, 16, 17):
+        for dt in (0, 1):
+            w = _weight(pkg, K, N, gs, g_idx=True)
+            assert lib.q4_linear_gate_up_act_order_plan(ctypes.byref(w), M, dt, ctypes.byref(fused)) == 0 and fused.value == 1
+            rc = lib.q4_linear_gate_up_act_order(ctypes.byref(w), 0x10, None, 0x20, M, dt, 0, 0x40, lib.q4_workspace_bytes(M, K, N), None)
+            assert rc != L.ERR_WORKSPACE, (M, dt, lib.q4_last_error())
+            rc = lib.q4_linear_gate_up_act_order(ctypes.byref(w), 0x10, None, 0x20, M, dt, 0, None, 0, None)
+            assert (rc != L.ERR_WORKSPACE) == without, (M, dt, lib.q4_last_error())
+
+
 def test_linear_plan_matches_its_parts(pkg):
     lib = pkg._lib.load()
     L = pkg._lib

@@ -5,6 +5,8 @@ namespace q4host {
 
 using q4::BatchParams;
 
+constexpr size_t kActLds = 160 * 1024 - 1024;  // of a workgroup
+
 static int act_k_rows(const q4_weight* w, int wk, int splits) {  // largest K range of a workgroup
   const int chunks = w->K / 128, slots = wk * splits, cpw = chunks / slots, rem = chunks % slots;
   return (cpw * wk + (rem < wk ? rem : wk)) * 128;
@@ -16,7 +18,7 @@ static bool act_few(const q4_weight* w, int M, int nq, int wk, int splits) {
   if (M > 4 || nq != 1 || w->K / 128 / (wk * splits) < 4) return false;
   // (not where the chunk's LDS costs a resident workgroup: 8192 x 57344 in groups of 32, whose two workgroups then just fill LDS, 72 us
   // without and 87 with)
-  const size_t lds = 160 * 1024 - 1024, rows = act_k_rows(w, wk, splits);
+  const size_t lds = kActLds, rows = act_k_rows(w, wk, splits);
   size_t resident = lds / q4::batch_act_lds(w->num_groups, (int)rows, wk, 1, 1, false);
   if (resident > (size_t)(16 / wk)) resident = 16 / wk;
   return lds / q4::batch_act_lds(w->num_groups, (int)rows, wk, 1, 1, true) >= resident;
@@ -45,7 +47,7 @@ static double act_plan(const q4_weight* w, int M, int mt, bool pow2, BatchPlan* 
       if (wk * sp > chunks) break;
       if (sp > 1 && (long)(sp - 1) * act_units(1, M) * tiles * 512 > Q4_WORKSPACE_CELL_BYTES) break;
       const size_t lds = q4::batch_act_lds(w->num_groups, act_k_rows(w, wk, sp), wk, mt, 1, act_few(w, M, 1, wk, sp));
-      if (lds > 160 * 1024 - 1024) continue;
+      if (lds > kActLds) continue;
       int resident = (int)(160 * 1024 / lds);
       const int by_registers = (mt <= 2 ? 16 : (mt == 3 ? 12 : 8)) / wk;
       if (resident > by_registers) resident = by_registers;
@@ -73,7 +75,10 @@ static void act_wide(const q4_weight* w, int M, BatchPlan* plan) {
   if (w->N % 128 != 0 || tiles < 192 || (tiles > 256 && tiles < 384) || w->num_groups > 96 || chunks < 16) return;
   int splits = 1;
   while (tiles > 256 && splits < 4 && (2L * splits - 1) * act_units(2, M) * tiles * 512 <= Q4_WORKSPACE_CELL_BYTES) splits *= 2;
-  *plan = BatchPlan{2, tiles <= 256 ? 8 : 4, splits};
+  const int wk = tiles <= 256 ? 8 : 4;
+  // (the table's rows are twice those that act_plan has seen to, and one workgroup along K holds the groups of all rows: K = 65536 stays on 64 columns)
+  if (q4::batch_act_lds(w->num_groups, act_k_rows(w, wk, splits), wk, 1, 2, false) > kActLds) return;
+  *plan = BatchPlan{2, wk, splits};
 }
 
 // Where this kernel runs, measured on MI355X against the kernels it takes over from (gemv_gptq_act_kernel in blocks of 16 rows
@@ -120,7 +125,7 @@ static bool act_cells(const void* workspace, size_t workspace_bytes) {
 
 // Without a workspace a workgroup walks all of K: the groups of all rows then have to lie in LDS beside the table.
 bool batch_act_fits(const q4_weight* w, int M, const BatchPlan& plan, const void* workspace, size_t workspace_bytes) {
-  return act_cells(workspace, workspace_bytes) || q4::batch_act_lds(w->num_groups, w->K, plan.wk, (M + 15) / 16, plan.nq, act_few(w, M, plan.nq, plan.wk, 1)) <= 160 * 1024 - 1024;
+  return act_cells(workspace, workspace_bytes) || q4::batch_act_lds(w->num_groups, w->K, plan.wk, (M + 15) / 16, plan.nq, act_few(w, M, plan.nq, plan.wk, 1)) <= kActLds;
 }
 
 template <int DTYPE, int MT, int WK, bool FUSE, int NQ = 1, bool FEW = false>
@@ -157,9 +162,11 @@ int launch_batch_act(const q4_weight* w, const void* x, const void* bias, void* 
   const bool fuse = gate_up_act != 0;
   const int mt = (M + 15) / 16;
   if (plan.splits > 1 && !act_cells(workspace, workspace_bytes)) plan.splits = 1;
+  // (a workgroup that walks all of K for want of a workspace holds the groups of all rows: on 64 columns where only that fits)
+  if (plan.nq == 2 && q4::batch_act_lds(w->num_groups, act_k_rows(w, plan.wk, plan.splits), plan.wk, mt, 2, false) > kActLds) plan.nq = 1;
   const bool few = act_few(w, M, plan.nq, plan.wk, plan.splits);
   const size_t lds = q4::batch_act_lds(w->num_groups, act_k_rows(w, plan.wk, plan.splits), plan.wk, mt, plan.nq, few);
-  if (lds > 160 * 1024 - 1024) {
+  if (lds > kActLds) {
     set_error("q4_linear(act-order batch kernel): %zu bytes of LDS needed without a workspace", lds);
     return Q4_ERR_WORKSPACE;
   }
