@@ -108,6 +108,12 @@ int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, i
 #define Q4_KERNEL_TALL 5  /* prefill, tiles of 96 to 256 rows, one wave per SIMD */
 #define Q4_KERNEL_BLOCK 6 /* prefill, tiles of 256 x 256, fp16 */
 int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);
+/*
+ * The tiles of a call that q4_linear_kernel answers Q4_KERNEL_TALL or Q4_KERNEL_BLOCK for: *rows of a tile, workgroups along K
+ * (*splits), and *k_halves = 2 where the waves of a workgroup halve its K range once more, else 1.  *rows = 0 for every other
+ * call.  For tests and benchmarks.
+ */
+int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int* rows, int* splits, int* k_halves);
 
 /*
  * First half of a gated MLP in one launch: W packs [gate | up] along N and

@@ -271,6 +271,25 @@ def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, w
     assert pkg._lib.KERNEL_NAMES[rc] == want
 
 
+def _tiles(pkg, M, K, N, gs, dtype, layout=0, gate_up=0):
+    out = [ctypes.c_int(-1) for _ in range(3)]
+    w = _weight(pkg, K, N, gs, layout)
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), M, 1 if dtype == "bf16" else 0, gate_up, *map(ctypes.byref, out)) == 0
+    return tuple(v.value for v in out)
+
+
+def test_the_tiles_of_a_prefill_call(pkg):
+    """The calls that the GPU test of two K halves means run on two K halves; calls of other kernels have no tiles."""
+    from tests.test_tall_gpu import HALVES
+
+    for M, K, N, gs, dtype, rows, splits in HALVES:
+        assert _tiles(pkg, M, K, N, gs, dtype) == (rows, splits, 2), (M, K, N)
+    assert _tiles(pkg, 161, 8192, 8192, 128, "f16") == (96, 4, 1) and _tiles(pkg, 1000, 4096, 28672, 128, "f16", gate_up=1) == (256, 1, 1)
+    assert _tiles(pkg, 64, 4096, 4096, 128, "f16") == (0, 0, 0) and _tiles(pkg, 301, 4104, 4104, 8, "f16") == (0, 0, 0)
+    w = _weight(pkg, 4096, 4096, 128)
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), 301, 0, 0, None, None, None) == pkg._lib.ERR_INVALID_ARGUMENT
+
+
 @pytest.mark.parametrize("K,N,gs,M,want", [(8192, 32768, 128, 33, 0), (8192, 32768, 128, 64, 0), (8192, 57344, 32, 48, 0), (8256, 33024, 64, 32, 0),
                                           (8256, 33024, 64, 33, 1), (8256, 57344, 64, 64, 1), (8256, 57344, 64, 65, 0), (8256, 28672, 64, 48, 0),
                                           (8192, 32768, 128, 128, 0), (8192, 32768, 128, 129, 1)])

@@ -6,6 +6,8 @@ the fp32 accumulation), 8e-3 in bf16 (output rounding 2^-8); the gated epilogue 
 that size and the same bars, as in test_gate_up_gpu.py.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -81,14 +83,20 @@ def test_splits_of_the_picked_kernels(pkg, oracle, gpu, layout, M, K, N, gs, dty
     assert max_rel_err(to_f32(got), y32) <= TOL[dtype]
 
 
-# GPTQ, two halves of K in a workgroup: 96-, 128- and 160-row tiles, ragged and full, with and without splits, four K tiles a half
-# (1024 x 8192) and more, groups of 64 and one group
-@pytest.mark.parametrize("M,K,N,gs,dtype", [(100, 4096, 4096, 128, "f16"), (96, 3584, 8192, 64, "f16"), (301, 1024, 8192, 1024, "f16"), (301, 1024, 8192, 64, "bf16"),
-                                            (420, 1024, 8192, 128, "f16"), (160, 14336, 4096, 128, "bf16"), (161, 8192, 8192, 128, "f16"), (640, 3584, 8192, 128, "f16")])
+# GPTQ, two halves of K in a workgroup: 96-, 128- and 160-row tiles, ragged and full, without and with splits in both data types, four K tiles
+# a half (1024 x 8192) and more, groups of 64 and one group.  (M, K, N, groupsize, dtype, rows of a tile, splits)
+HALVES = [(77, 14336, 4096, 128, "f16", 96, 8), (96, 3584, 8192, 64, "f16", 96, 4), (301, 1024, 8192, 1024, "f16", 96, 1), (301, 1024, 8192, 64, "bf16", 96, 1),
+          (420, 1024, 8192, 128, "f16", 128, 1), (85, 4096, 4096, 128, "bf16", 96, 8), (300, 2048, 2048, 64, "f16", 96, 4), (640, 3584, 8192, 128, "f16", 160, 1),
+          (96, 4096, 4096, 128, "bf16", 96, 4), (147, 4608, 5632, 128, "f16", 160, 4), (120, 2688, 7168, 128, "bf16", 128, 3)]
+
+
+@pytest.mark.parametrize("M,K,N,gs,dtype", [case[:5] for case in HALVES])
 def test_two_halves_of_k(pkg, oracle, gpu, M, K, N, gs, dtype):
     pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, gs, K + M, dtype)
     bf = dtype == "bf16"
     assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16) == "tall"
+    tiles = [ctypes.c_int(0) for _ in range(3)]
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(pk.struct()), M, int(bf), 0, *map(ctypes.byref, tiles)) == 0 and tiles[2].value == 2
     x = oracle.make_x(M, K, seed=M, dtype=dtype)
     b32 = np.random.default_rng(M).standard_normal(N).astype(np.float32)
     bias = oracle.f32_to_bf16_bits(b32) if bf else b32.astype(np.float16)

@@ -265,6 +265,23 @@ int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up) {
   return path == Q4_PATH_GEMM && gemm_gate_up_supported(w, M, dtype) ? path : Q4_PATH_AUTO;
 }
 
+int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int* rows, int* splits, int* k_halves) {
+  if (rows == nullptr || splits == nullptr || k_halves == nullptr) {
+    set_error("q4_linear_tiles: null output");
+    return Q4_ERR_INVALID_ARGUMENT;
+  }
+  *rows = *splits = *k_halves = 0;
+  const int kernel = q4_linear_kernel(w, M, dtype, gate_up);
+  if (kernel < 0) return kernel;
+  TallPlan tall;
+  if ((kernel == Q4_KERNEL_TALL || kernel == Q4_KERNEL_BLOCK) && gemm_tall_default(w, M, dtype, gate_up != 0, &tall)) {
+    *rows = 32 * tall.r;
+    *splits = tall.splits;
+    *k_halves = tall.kw;
+  }
+  return Q4_OK;
+}
+
 int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
                  void* workspace, size_t workspace_bytes, int path, void* stream) {
   int rc = validate_weight(w, "q4_linear");
