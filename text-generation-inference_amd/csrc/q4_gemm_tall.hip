@@ -68,6 +68,11 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
     for (int sp : kSplits) {
       const long wgs = (long)((M + 32 * r - 1) / (32 * r)) * (N / (q4::kTallBN / 2)) * sp;
       if (KT % (2 * sp) != 0 || KT / (2 * sp) < 4 || wgs < 96 || wgs > 1024) continue;
+      // A second round of workgroups starts and ends anew, which costs 4-6 us that the estimate does not know: below 4096 rows of K halves only
+      // where all workgroups run at once (us, whole K ranges / halves in two rounds and more: 1024 x 16640 167 rows 18.1 / 23.4, 896 x 18944
+      // 638 rows 30.3 / 42.9, 1152 x 17664 794 rows 48.7 / 57.6, 1792 x 43264 296 rows 68.0 / 74.3; 4096 x 45056 300 rows 140.9 / 142.2, 5632 x
+      // 45056 258 rows 183.3 / 178.4, bf16 229.9 on 128-row workgroups / 180.9)
+      if (wgs > 256 && K < 4096) continue;
       const double more = dtype == Q4_DTYPE_BF16 ? 0.065 : 0.0;
       // (padded rows draw power for nothing, more than the fit's card showed: 4096 x 6144 301 rows in 384, 30.2 / 29.5 us on one card, slower on another)
       const double padded = (double)((M + 32 * r - 1) / (32 * r) * (32 * r)) / M - 1.1;
