@@ -287,6 +287,8 @@ def test_the_tiles_of_a_prefill_call(pkg):
     # (halves that would go out in two rounds of workgroups over a short K)
     assert _tiles(pkg, 167, 1024, 16640, 128, "f16") == (96, 1, 1) and _tiles(pkg, 794, 1152, 17664, 128, "f16")[2] == 1
     assert _tiles(pkg, 638, 896, 18944, 128, "f16") == (256, 1, 1) and _tiles(pkg, 258, 5632, 45056, 128, "bf16")[2] == 2
+    # (160-row tiles whose halves are four or five K tiles)
+    assert _tiles(pkg, 825, 640, 4864, 128, "f16") == (96, 1, 1) and _tiles(pkg, 679, 512, 6144, 128, "f16") == (96, 1, 1)
     assert _tiles(pkg, 161, 8192, 8192, 128, "f16") == (96, 4, 1) and _tiles(pkg, 1000, 4096, 28672, 128, "f16", gate_up=1) == (256, 1, 1)
     assert _tiles(pkg, 64, 4096, 4096, 128, "f16") == (0, 0, 0) and _tiles(pkg, 301, 4104, 4104, 8, "f16") == (0, 0, 0)
     w = _weight(pkg, 4096, 4096, 128)

@@ -73,6 +73,9 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
       // 638 rows 30.3 / 42.9, 1152 x 17664 794 rows 48.7 / 57.6, 1792 x 43264 296 rows 68.0 / 74.3; 4096 x 45056 300 rows 140.9 / 142.2, 5632 x
       // 45056 258 rows 183.3 / 178.4, bf16 229.9 on 128-row workgroups / 180.9)
       if (wgs > 256 && K < 4096) continue;
+      // (160-row tiles fill LDS and start late, which four or five K tiles a half don't make up for against 96-row tiles over whole K ranges: 640 x
+      // 4864 825 rows 13.8 / 14.8, 640 x 10752 434 rows 14.4 / 15.3, 512 x 6144 679 rows 12.7 / 13.1; beyond 1024 rows those are left out below)
+      if (r == 5 && K < 768 && M <= 1024) continue;
       const double more = dtype == Q4_DTYPE_BF16 ? 0.065 : 0.0;
       // (padded rows draw power for nothing, more than the fit's card showed: 4096 x 6144 301 rows in 384, 30.2 / 29.5 us on one card, slower on another)
       const double padded = (double)((M + 32 * r - 1) / (32 * r) * (32 * r)) / M - 1.1;
