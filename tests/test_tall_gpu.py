@@ -87,7 +87,7 @@ def test_splits_of_the_picked_kernels(pkg, oracle, gpu, layout, M, K, N, gs, dty
 # a half (1024 x 8192) and more, groups of 64 and one group.  (M, K, N, groupsize, dtype, rows of a tile, splits)
 HALVES = [(77, 14336, 4096, 128, "f16", 96, 8), (96, 3584, 8192, 64, "f16", 96, 4), (301, 1024, 8192, 1024, "f16", 96, 1), (301, 1024, 8192, 64, "bf16", 96, 1),
           (420, 1024, 8192, 128, "f16", 128, 1), (85, 4096, 4096, 128, "bf16", 96, 8), (300, 2048, 2048, 64, "f16", 96, 4), (640, 3584, 8192, 128, "f16", 160, 1),
-          (96, 4096, 4096, 128, "bf16", 96, 4), (147, 4608, 5632, 128, "f16", 160, 4), (120, 2688, 7168, 128, "bf16", 128, 3)]
+          (96, 4096, 4096, 128, "bf16", 96, 4), (147, 4608, 5632, 128, "f16", 160, 4), (120, 2688, 7168, 128, "bf16", 128, 3), (1245, 4096, 2048, 128, "bf16", 96, 1)]
 
 
 @pytest.mark.parametrize("M,K,N,gs,dtype", [case[:5] for case in HALVES])

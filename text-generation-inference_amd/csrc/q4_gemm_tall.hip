@@ -104,13 +104,16 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
 //   GPTQ, tiles below 256 rows, three rounds of the chip and more: every CU is at work, and these tiles unpack a weight as
 //     often as two 128-row workgroups: 4096 x 28672 at 1400 and 2048 rows 0.93-0.96, 4096 x 12288 at 2048 0.92, gated 0.95,
 //     8192 x 57344 at 1400 0.96; 256-row tiles in 3.5-7 rounds 0.97-1.06
-//   GPTQ, 96-row tiles for more than 1024 rows: 4096 x 4096 and 3584 x 3584 at 1400 0.93-0.94; at 700 0.97-1.07
+//   GPTQ, 96-row tiles over whole K ranges for more than 1024 rows: 4096 x 4096 and 3584 x 3584 at 1400 0.93-0.94; at 700 0.97-1.07.  In K
+//     halves, 128 columns wide, they are the faster ones, 30 calls 1.35 in geometric mean (1.00): 5120 x 2304 1040 rows 40.8 us on 128-row
+//     workgroups, 38.9 so (42.5 on 160-row tiles in four splits), 6400 x 2048 1312 rows 54.6 / 46.4, 4096 x 2048 1245 bf16 rows 37.8 / 33.8
 //   AWQ, K of 9 to 16 K tiles (shorter ones not measured), where start and epilogue count as much as the tiles in between: 1024 x 8192 at 1000
 //     rows 0.90, gated bf16 at 512 to 1400 rows 0.86-1.02; up to 129 rows, in splits, 1.13-1.28, 256 x 256 tiles 1.20-1.34,
 //     gated fp16 0.97-1.08
 static bool tall_outdone(bool awq, int dtype, int M, int K, int N, bool gate_up, const TallPlan& plan) {
   if (plan.block) return false;
   if (awq) return K > 512 && K <= 1024 && M > 384 && (!gate_up || dtype == Q4_DTYPE_BF16);
+  if (plan.kw == 2) return false;  // (128 columns: at most 512 tiles of 256, and 96 rows are no fault)
   const long tiles = (long)((M + 32 * plan.r - 1) / (32 * plan.r)) * (N / q4::kTallBN);
   return (plan.r < 8 && tiles >= 3 * 256) || (plan.r == 3 && !gate_up && M > 1024);
 }
