@@ -292,6 +292,8 @@ def test_the_tiles_of_a_prefill_call(pkg):
     # (halves on 96-row tiles beyond 1024 rows, where whole K ranges on such tiles are left out)
     for K, N, M in ((5120, 2304, 1025), (5504, 2304, 1025), (4864, 2304, 1099), (4864, 2048, 1173), (4864, 1792, 1432), (4096, 2048, 1245)):
         assert _tiles(pkg, M, K, N, 128, "f16") == (96, 1, 2)
+    # (tiles that are a third padding)
+    assert _tiles(pkg, 104, 4096, 4096, 128, "f16") == (96, 4, 2) and _tiles(pkg, 203, 4096, 12288, 128, "f16") == (128, 1, 2)
     assert _tiles(pkg, 161, 8192, 8192, 128, "f16") == (96, 4, 1) and _tiles(pkg, 1000, 4096, 28672, 128, "f16", gate_up=1) == (256, 1, 1)
     assert _tiles(pkg, 64, 4096, 4096, 128, "f16") == (0, 0, 0) and _tiles(pkg, 301, 4104, 4104, 8, "f16") == (0, 0, 0)
     w = _weight(pkg, 4096, 4096, 128)

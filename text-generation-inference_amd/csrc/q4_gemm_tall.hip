@@ -58,10 +58,11 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
   if (!halves || gate_up || awq || M > 1536) return best;
   // Two halves of K in a workgroup, 128 columns: as many CUs at work with half the splits, whose fp32 partial sums (8 M N bytes each, out and in)
   // otherwise cost up to a third of a call; every fragment of x then serves half as many columns, which is why they end where two
-  // splits and less would do.  Fitted to 15 layer shapes x 100-640 rows x all heights and splits, within 7 %; where it puts them 2 % ahead they
-  // are, 23 calls: 1.12 in geometric mean (1.00-1.37); us, before / so: 3584 x 8192 301 rows 34.4 / 28.9, 14336 x 4096 160 rows 36.3 / 33.3, bf16
-  // 38.9 / 33.3, 8192 x 8192 160 rows 39.6 / 35.9, 1024 x 8192 301 rows 18.0 / 13.1.  Over 176
-  // calls of 37 shapes at 65-768 rows, changed or not, 1.05 in geometric mean (0.98), over 126 of 29 shapes at 769-1536 1.01 (0.99; 3584 x 3584 1000 rows 40.0 / 34.4).  (AWQ, whose words are loaded row by row, 0.75-1.1: not built in.)
+  // splits and less would do.  Fitted to 15 layer shapes x 100-640 rows x all heights and splits, within 7 % where the workgroups are one round;
+  // where it puts them 2 % ahead they run.  188 such calls of 24 layer shapes at 65-1536 rows 1.17 in geometric mean (0.96-1.71), 150 of
+  // any shape 1.20 (0.99); us, before / so: 3584 x 8192 301 rows 35.7 / 30.2, bf16 35.1 / 30.9, 1024 x 8192 301 rows 17.4 / 12.8, 14336 x 4096 89
+  // rows 30.7 / 25.0, 3584 x 3584 1000 rows 40.3 / 35.5, 4096 x 6144 301 rows 29.9 / 30.0.  (A price on padded rows, which left the last one
+  // out, cost 90 calls that it changed 1.09 in geometric mean.  AWQ, whose words are loaded row by row, 0.75-1.1: not built in.)
   static const double kHalves[3][2] = {{0.54, 0.81}, {0.69, 1.00}, {0.85, 1.23}};  // (bf16: 0.065 more)
   const int KT = K / q4::kBK;
   for (int r = 3; r <= 5; ++r)
@@ -77,9 +78,7 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
       // 4864 825 rows 13.8 / 14.8, 640 x 10752 434 rows 14.4 / 15.3, 512 x 6144 679 rows 12.7 / 13.1; beyond 1024 rows those are left out below)
       if (r == 5 && K < 768 && M <= 1024) continue;
       const double more = dtype == Q4_DTYPE_BF16 ? 0.065 : 0.0;
-      // (padded rows draw power for nothing, more than the fit's card showed: 4096 x 6144 301 rows in 384, 30.2 / 29.5 us on one card, slower on another)
-      const double padded = (double)((M + 32 * r - 1) / (32 * r) * (32 * r)) / M - 1.1;
-      const double t = (padded > 0.0 ? 1.02 + 0.1 * padded : 1.02) * (gemm_round_us(wgs, 256, KT / (2 * sp), kHalves[r - 3][0] + more, kHalves[r - 3][1] + more) + 7.7 +
+      const double t = 1.02 * (gemm_round_us(wgs, 256, KT / (2 * sp), kHalves[r - 3][0] + more, kHalves[r - 3][1] + more) + 7.7 +
                                (sp > 1 ? 0.55 + 1.69e-6 * sp * M * N : 0.0));
       if (t < best) {
         best = t;
