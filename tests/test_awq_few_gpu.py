@@ -28,7 +28,7 @@ def _case(pkg, oracle, gpu, K, N, gs, seed):
 
 # K: one chunk a wave, ragged deals (17, 43, 67 chunks), an odd number of workgroups along K; N: one tile, an odd number, pairs of tiles
 @pytest.mark.parametrize("K,N,gs", [(2048, 256, 128), (2176, 768, 128), (5504, 512, 256), (8576, 1280, 128), (4096, 28672, 128), (14336, 4096, -1),
-                                    (8192, 10240, 512)])
+                                    (8192, 10240, 512), (2176, 16640, 128), (5504, 6400, 128)])
 @pytest.mark.parametrize("M,dtype", [(1, "f16"), (1, "bf16"), (2, "f16"), (3, "bf16"), (4, "f16"), (4, "bf16")])
 def test_plain(pkg, oracle, gpu, K, N, gs, M, dtype):
     gs = gs if gs == -1 or K % gs == 0 else 128
@@ -83,11 +83,29 @@ def test_gated(pkg, oracle, gpu, K, N, gs, M, dtype, act):
     assert max_rel_err(to_f32(got), oracle.to_f32(want, dtype)) <= {"f16": 2e-3, "bf16": 1.2e-2}[dtype]
 
 
+# ragged deals of K (17 and 67 chunks) over as many tiles as this kernel takes them for
+@pytest.mark.parametrize("K,N", [(2176, 20480), (8576, 5120)])
+@pytest.mark.parametrize("M,dtype", [(1, "f16"), (3, "bf16"), (4, "f16")])
+def test_gated_against_64_bits(pkg, oracle, gpu, K, N, M, dtype):
+    """Bar: the roundings of both sums, of the activation (whose slope is at most 1.1) and of the product, one unit each, and the fp32 sums'
+    36 + K / 128; 1 % for their products."""
+    pk, w = _case(pkg, oracle, gpu, K, N, 128, K + N)
+    x = (torch.randn((M, K), device=gpu, generator=torch.Generator(device=gpu).manual_seed(M)) / 8).to(DT[dtype])
+    got, u = pkg.ops.linear_gate_up(pk, x, "silu"), U[dtype]
+    sums, terms = x.double() @ w, (x.double().abs() @ w.abs()) * (36 + K // 128) * 2.0**-24
+    gate, up = sums.chunk(2, dim=1)
+    eg, eu = (u * sums.abs() + terms).chunk(2, dim=1)
+    act = torch.nn.functional.silu(gate)
+    bar = 1.1 * eg * up.abs() + act.abs() * eu + 2 * u * (act * up).abs()
+    assert bool(((got.double() - act * up).abs() <= 1.01 * bar + 2.0**-24).all())
+
+
 def test_replays_and_captures(pkg, oracle, gpu):
     """Several replays of a graph with eager calls between them, and a stream of their own."""
     pk, w = _case(pkg, oracle, gpu, 4096, 4096, 128, 9)
     x = torch.randn((3, 4096), device=gpu).half()
     want = pkg.ops.linear(pk, x)
+    pkg.ops.reserve_workspace(gpu, 16 << 20, pkg.ops.SHARED)
     graph, out = torch.cuda.CUDAGraph(), None
     with torch.cuda.graph(graph):
         out = pkg.ops.linear(pk, x)

@@ -300,6 +300,27 @@ def test_the_tiles_of_a_prefill_call(pkg):
     assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), 301, 0, 0, None, None, None) == pkg._lib.ERR_INVALID_ARGUMENT
 
 
+def _launched(pkg, w, M, dtype, gate_up=0, path=0):
+    """The launch that a call with a full workspace ends at (it fails for want of a GPU, and says its name), or the error code."""
+    lib = pkg._lib.load()
+    ws = lib.q4_workspace_bytes(M, w.K, w.N)
+    if gate_up:
+        rc = lib.q4_linear_gate_up(ctypes.byref(w), 0x10, None, 0x20, M, dtype, 0, 0x40, ws, None)
+    else:
+        rc = lib.q4_linear_ex(ctypes.byref(w), 0x10, None, 0x20, M, dtype, 0x40, ws, path, None)
+    return lib.q4_last_error().decode().split(":")[0] if rc == pkg._lib.ERR_LAUNCH else rc
+
+
+# (K in whole 128-row chunks, one and more a wave; fewer and more units of 128 x 256 weights than the chip has SIMDs)
+@pytest.mark.parametrize("K,N,gate_up,dtype,few", [(2176, 4096, 0, 0, False), (2176, 16384, 0, 0, True), (3968, 8192, 0, 1, False), (2048, 512, 0, 0, True), (8320, 1024, 0, 1, True),
+                                                   (2176, 4096, 1, 0, False), (2176, 20480, 1, 0, True), (11008, 2048, 1, 0, False), (11008, 3072, 1, 0, True),
+                                                   (2048, 4096, 1, 0, True), (4096, 4096, 1, 1, False), (4096, 8192, 1, 1, True)])
+def test_awq_rows_of_small_ragged_layers(pkg, K, N, gate_up, dtype, few):
+    for M in (1, 4):
+        got = _launched(pkg, _weight(pkg, K, N, 128, layout=1), M, dtype, gate_up)
+        assert (got == "q4_linear(AWQ, up to four rows)") == few, (M, got)
+
+
 @pytest.mark.parametrize("K,N,gs,M,want", [(8192, 32768, 128, 33, 0), (8192, 32768, 128, 64, 0), (8192, 57344, 32, 48, 0), (8256, 33024, 64, 32, 0),
                                           (8256, 33024, 64, 33, 1), (8256, 57344, 64, 64, 1), (8256, 57344, 64, 65, 0), (8256, 28672, 64, 48, 0),
                                           (8192, 32768, 128, 128, 0), (8192, 32768, 128, 129, 1)])
