@@ -103,17 +103,19 @@ int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, i
  * Which kernels q4_linear (gate_up = 0) or the gated launch (gate_up = 1: q4_linear_gate_up, for act-order weights
  * q4_linear_gate_up_act_order) run for this problem with a workspace: a Q4_PATH_* or one of the Q4_KERNEL_* below (an
  * answer only, no path to ask for); Q4_PATH_AUTO when no gated kernel takes it.  A pure function of (w's geometry, M, dtype).
+ * Q4_PATH_GEMV stands for the decode path's row range: its plain AWQ calls of one to six rows and act-order calls of one to five
+ * may run on the variants that Q4_KERNEL_BATCH has for them; q4_linear_tiles tells.  A forced Q4_PATH_GEMV never does.
  */
-#define Q4_KERNEL_BATCH 4 /* up to 64 rows: GPTQ, act-order (its own variant) and AWQ (one to four rows: its own variant) */
+#define Q4_KERNEL_BATCH 4 /* up to 64 rows: GPTQ, act-order (its own variant) and AWQ (variants of their own for one to four and for five to sixteen rows) */
 #define Q4_KERNEL_TALL 5  /* prefill, tiles of 96 to 256 rows, one wave per SIMD */
 #define Q4_KERNEL_BLOCK 6 /* prefill, tiles of 256 x 256, fp16 */
 int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up);
 /*
- * The tiles of a call that q4_linear_kernel answers Q4_KERNEL_TALL or Q4_KERNEL_BLOCK for: *rows of a tile, workgroups along K
- * (*splits), and *k_halves = 2 where the waves of a workgroup halve its K range once more, else 1.  *rows = 0 for every other
- * call.  For tests and benchmarks.
+ * The workgroups of a call that runs on the batch decode kernels or the prefill kernels whose tiles follow the row count
+ * (Q4_KERNEL_BATCH, Q4_KERNEL_TALL, Q4_KERNEL_BLOCK and the decode calls named above): rows and columns of a tile, the parts in which a
+ * workgroup's waves walk its K range, and the workgroups along K.  tiles[0] = 0 for every other call.  For tests and benchmarks.
  */
-int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int* rows, int* splits, int* k_halves);
+int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int tiles[4]);
 
 /*
  * First half of a gated MLP in one launch: W packs [gate | up] along N and

@@ -271,11 +271,18 @@ def test_the_kernel_of_a_call(pkg, K, N, gs, layout, g_idx, M, dtype, gate_up, w
     assert pkg._lib.KERNEL_NAMES[rc] == want
 
 
-def _tiles(pkg, M, K, N, gs, dtype, layout=0, gate_up=0):
-    out = [ctypes.c_int(-1) for _ in range(3)]
-    w = _weight(pkg, K, N, gs, layout)
-    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), M, 1 if dtype == "bf16" else 0, gate_up, *map(ctypes.byref, out)) == 0
-    return tuple(v.value for v in out)
+def _all_tiles(pkg, M, K, N, gs, dtype, layout=0, gate_up=0, g_idx=False):
+    """(rows, columns, K parts inside a workgroup, workgroups along K)"""
+    out, w = (ctypes.c_int * 4)(-1, -1, -1, -1), _weight(pkg, K, N, gs, layout, g_idx)
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), M, 1 if dtype == "bf16" else 0, gate_up, out) == 0
+    return tuple(out)
+
+
+def _tiles(pkg, M, K, N, gs, dtype, **kw):
+    """Of a prefill call: (rows, workgroups along K, K halves)"""
+    rows, columns, halves, splits = _all_tiles(pkg, M, K, N, gs, dtype, **kw)
+    assert columns * halves == (256 if rows else 0)
+    return rows, splits, halves
 
 
 def test_the_tiles_of_a_prefill_call(pkg):
@@ -295,9 +302,9 @@ def test_the_tiles_of_a_prefill_call(pkg):
     # (tiles that are a third padding)
     assert _tiles(pkg, 104, 4096, 4096, 128, "f16") == (96, 4, 2) and _tiles(pkg, 203, 4096, 12288, 128, "f16") == (128, 1, 2)
     assert _tiles(pkg, 161, 8192, 8192, 128, "f16") == (96, 4, 1) and _tiles(pkg, 1000, 4096, 28672, 128, "f16", gate_up=1) == (256, 1, 1)
-    assert _tiles(pkg, 64, 4096, 4096, 128, "f16") == (0, 0, 0) and _tiles(pkg, 301, 4104, 4104, 8, "f16") == (0, 0, 0)
+    assert _tiles(pkg, 2048, 4096, 28672, 128, "bf16") == (0, 0, 0) and _tiles(pkg, 301, 4104, 4104, 8, "f16") == (0, 0, 0)
     w = _weight(pkg, 4096, 4096, 128)
-    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), 301, 0, 0, None, None, None) == pkg._lib.ERR_INVALID_ARGUMENT
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(w), 301, 0, 0, None) == pkg._lib.ERR_INVALID_ARGUMENT
 
 
 def _launched(pkg, w, M, dtype, gate_up=0, path=0):
@@ -311,6 +318,25 @@ def _launched(pkg, w, M, dtype, gate_up=0, path=0):
     return lib.q4_last_error().decode().split(":")[0] if rc == pkg._lib.ERR_LAUNCH else rc
 
 
+FEW = "q4_linear(AWQ, up to four rows)"
+
+
+@pytest.mark.parametrize("K,N,layout,g_idx,M,dtype,kernel,tiles", [
+    (4096, 28672, 1, False, 1, "f16", FEW, (4, 256, 8, 2)), (14336, 4096, 1, False, 4, "bf16", FEW, (4, 256, 8, 14)),
+    (8192, 57344, 1, False, 5, "f16", "q4_linear(AWQ, five to sixteen rows)", (16, 256, 8, 1)),
+    (8192, 10240, 0, True, 4, "f16", "q4_linear(act-order batch kernel)", (16, 64, 8, 3))])
+def test_a_forced_decode_path_runs_its_own_kernels(pkg, K, N, layout, g_idx, M, dtype, kernel, tiles):
+    """Decode calls that are named for their path and run on a batch kernel's variant: only where the caller leaves the choice, and only with
+    the workspace that the path asks for."""
+    lib, L, dt = pkg._lib.load(), pkg._lib, 1 if dtype == "bf16" else 0
+    w = _weight(pkg, K, N, 128, layout, g_idx)
+    assert _launched(pkg, w, M, dt) == kernel and _all_tiles(pkg, M, K, N, 128, dtype, layout=layout, g_idx=g_idx) == tiles
+    assert _launched(pkg, w, M, dt, path=L.PATH_GEMV) == "q4_linear(gemv)"
+    if L.KERNEL_NAMES[lib.q4_linear_kernel(ctypes.byref(w), M, dt, 0)] == "gemv":
+        lib.q4_linear_ex(ctypes.byref(w), 0x10, None, 0x20, M, dt, 0x40, L.WORKSPACE_COUNTER_BYTES - 16, L.PATH_AUTO, None)
+        assert kernel.encode() not in lib.q4_last_error()
+
+
 # (K in whole 128-row chunks, one and more a wave; fewer and more units of 128 x 256 weights than the chip has SIMDs)
 @pytest.mark.parametrize("K,N,gate_up,dtype,few", [(2176, 4096, 0, 0, False), (2176, 16384, 0, 0, True), (3968, 8192, 0, 1, False), (2048, 512, 0, 0, True), (8320, 1024, 0, 1, True),
                                                    (2176, 4096, 1, 0, False), (2176, 20480, 1, 0, True), (11008, 2048, 1, 0, False), (11008, 3072, 1, 0, True),
@@ -318,7 +344,7 @@ def _launched(pkg, w, M, dtype, gate_up=0, path=0):
 def test_awq_rows_of_small_ragged_layers(pkg, K, N, gate_up, dtype, few):
     for M in (1, 4):
         got = _launched(pkg, _weight(pkg, K, N, 128, layout=1), M, dtype, gate_up)
-        assert (got == "q4_linear(AWQ, up to four rows)") == few, (M, got)
+        assert (got == FEW) == few, (M, got)
 
 
 @pytest.mark.parametrize("K,N,gs,M,want", [(8192, 32768, 128, 33, 0), (8192, 32768, 128, 64, 0), (8192, 57344, 32, 48, 0), (8256, 33024, 64, 32, 0),

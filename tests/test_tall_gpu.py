@@ -95,8 +95,8 @@ def test_two_halves_of_k(pkg, oracle, gpu, M, K, N, gs, dtype):
     pk, w = _weight(pkg, oracle, gpu, "gptq", K, N, gs, K + M, dtype)
     bf = dtype == "bf16"
     assert pkg.ops.kernel_of(pk, M, torch.bfloat16 if bf else torch.float16) == "tall"
-    tiles = [ctypes.c_int(0) for _ in range(3)]
-    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(pk.struct()), M, int(bf), 0, *map(ctypes.byref, tiles)) == 0 and tiles[2].value == 2
+    tiles = (ctypes.c_int * 4)()
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(pk.struct()), M, int(bf), 0, tiles) == 0 and tiles[2] == 2
     x = oracle.make_x(M, K, seed=M, dtype=dtype)
     b32 = np.random.default_rng(M).standard_normal(N).astype(np.float32)
     bias = oracle.f32_to_bf16_bits(b32) if bf else b32.astype(np.float16)

@@ -86,7 +86,7 @@ SIGNATURES = {
         [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_size_t, c_int, c_void_p],
     ),
     "q4_linear_kernel": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int]),
-    "q4_linear_tiles": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int, POINTER(c_int), POINTER(c_int), POINTER(c_int)]),
+    "q4_linear_tiles": (c_int, [POINTER(Q4Weight), c_int, c_int, c_int, POINTER(c_int)]),
     "q4_gemv_tuned": (
         c_int,
         [POINTER(Q4Weight), c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_size_t, c_int, c_int, c_int, c_int, c_void_p],

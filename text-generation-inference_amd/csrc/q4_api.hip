@@ -265,21 +265,29 @@ int q4_linear_kernel(const q4_weight* w, int M, int dtype, int gate_up) {
   return path == Q4_PATH_GEMM && gemm_gate_up_supported(w, M, dtype) ? path : Q4_PATH_AUTO;
 }
 
-int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int* rows, int* splits, int* k_halves) {
-  if (rows == nullptr || splits == nullptr || k_halves == nullptr) {
+int q4_linear_tiles(const q4_weight* w, int M, int dtype, int gate_up, int tiles[4]) {
+  if (tiles == nullptr) {
     set_error("q4_linear_tiles: null output");
     return Q4_ERR_INVALID_ARGUMENT;
   }
-  *rows = *splits = *k_halves = 0;
+  auto answer = [tiles](int rows, int columns, int k_parts, int splits) {
+    tiles[0] = rows;
+    tiles[1] = columns;
+    tiles[2] = k_parts;
+    tiles[3] = splits;
+    return Q4_OK;
+  };
   const int kernel = q4_linear_kernel(w, M, dtype, gate_up);
   if (kernel < 0) return kernel;
   TallPlan tall;
-  if ((kernel == Q4_KERNEL_TALL || kernel == Q4_KERNEL_BLOCK) && gemm_tall_default(w, M, dtype, gate_up != 0, &tall)) {
-    *rows = 32 * tall.r;
-    *splits = tall.splits;
-    *k_halves = tall.kw;
-  }
-  return Q4_OK;
+  if ((kernel == Q4_KERNEL_TALL || kernel == Q4_KERNEL_BLOCK) && gemm_tall_default(w, M, dtype, gate_up != 0, &tall))
+    return answer(32 * tall.r, 256 / tall.kw, tall.kw, tall.splits);
+  BatchPlan batch;
+  const bool named = kernel == Q4_KERNEL_BATCH && (batch_default(w, M, dtype, gate_up != 0, &batch) || batch_act_default(w, M, dtype, gate_up != 0, &batch));
+  if (!named && !(kernel == Q4_PATH_GEMV && !gate_up && decode_few_default(w, M, dtype, &batch))) return answer(0, 0, 0, 0);
+  if (batch.few.wn > 0) return answer(M <= 4 ? 4 : 16, 256 * batch.few.wn, batch.few.wk, batch.few.splits);
+  // (AWQ, gated: a gate and an up tile)
+  return answer((M + 15) / 16 * 16, 64 * batch.nq * (gate_up && w->layout == Q4_LAYOUT_AWQ ? 2 : 1), batch.wk, batch.splits);
 }
 
 int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype,
@@ -310,6 +318,13 @@ int q4_linear_ex(const q4_weight* w, const void* x, const void* bias, void* y, i
     if ((path == Q4_PATH_GEMV || path == Q4_PATH_GEMM) && batch_act_default(w, M, dtype, false, &batch) &&
         batch_act_fits(w, M, batch, workspace, workspace_bytes))
       return launch_batch_act(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, batch, (hipStream_t)stream);
+    if (path == Q4_PATH_GEMV && decode_few_default(w, M, dtype, &batch)) {
+      // (with the workspace that the decode path asks for; without, its own kernels answer or refuse)
+      const int splits = gemv_pick_config(w, M).splits;
+      const size_t need = (size_t)Q4_WORKSPACE_COUNTER_BYTES + (splits > 1 ? (size_t)splits * M * w->N * sizeof(float) : 0);
+      if (workspace != nullptr && workspace_bytes >= need)
+        return (w->g_idx != nullptr ? launch_batch_act : launch_batch)(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, batch, (hipStream_t)stream);
+    }
     TallPlan tall;
     if (path == Q4_PATH_GEMM && gemm_tall_default(w, M, dtype, false, &tall))
       return launch_gemm_tall(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, tall, (hipStream_t)stream);

@@ -259,6 +259,8 @@ int launch_batch(const q4_weight* w, const void* x, const void* bias, void* y, i
 // the same for act-order weights (q4_gemv_batch_act.cuh)
 bool batch_act_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan);
 bool batch_act_few_default(const q4_weight* w, int M, int dtype, BatchPlan* plan);
+// either, for plain calls on the decode path
+bool decode_few_default(const q4_weight* w, int M, int dtype, BatchPlan* plan);
 bool batch_act_fits(const q4_weight* w, int M, const BatchPlan& plan, const void* workspace, size_t workspace_bytes);
 int launch_batch_act(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act,
                      void* workspace, size_t workspace_bytes, const BatchPlan& plan, hipStream_t stream);

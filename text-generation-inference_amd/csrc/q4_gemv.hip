@@ -652,20 +652,6 @@ int launch_gemv(const q4_weight* w, const void* x, const void* bias, void* y, in
   const bool awq = w->layout == Q4_LAYOUT_AWQ;
   const bool act = !awq && w->g_idx != nullptr;
   GemvConfig cfg = cfg_in ? *cfg_in : (gate_up_act != 0 ? gemv_pick_config(w, M, true) : gemv_pick_config(w, M));
-  // AWQ, one to four rows, plain call: the kernel of q4_gemv_awq_few.cuh, with the workspace that the kernels below ask for (five and six
-  // rows of 2^28 weights and more, which batch_default leaves here: q4_gemv_awq_wide.cuh); act-order, up to five: the batch kernel
-  AwqFewPlan few;
-  BatchPlan act_few;
-  if (awq && cfg_in == nullptr && gate_up_act == 0 && x_perm == nullptr &&
-      (awq_few_default(w, M, dtype, false, &few) || (M <= 6 && (long)w->K * w->N >= (1L << 28) && awq_wide_default(w, M, dtype, false, &few)))) {
-    const size_t need = (size_t)Q4_WORKSPACE_COUNTER_BYTES + (cfg.splits > 1 ? (size_t)cfg.splits * M * w->N * sizeof(float) : 0);
-    if (workspace != nullptr && workspace_bytes >= need)
-      return launch_awq_few(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, few, stream);
-  }
-  if (act && cfg_in == nullptr && gate_up_act == 0 && x_perm == nullptr && batch_act_few_default(w, M, dtype, &act_few)) {
-    const size_t need = (size_t)Q4_WORKSPACE_COUNTER_BYTES + (cfg.splits > 1 ? (size_t)cfg.splits * M * w->N * sizeof(float) : 0);
-    if (workspace != nullptr && workspace_bytes >= need) return launch_batch_act(w, x, bias, y, M, dtype, 0, workspace, workspace_bytes, act_few, stream);
-  }
   const bool contiguous = !awq && !act;
   if (!contiguous || w->groupsize < 128) cfg.words = 4;  // only the contiguous-group kernel has narrow tiles
   if (gate_up_act != 0) cfg.words = 8;                    // four gate + four up words per lane

@@ -123,7 +123,7 @@ int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y,
   else launch_dtype<Q4_DTYPE_BF16>(p, plan.wn, plan.wk, gate_up_act != 0, grid, stream);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
-    set_error("q4_linear(AWQ, up to four rows): launch failed: %s", hipGetErrorString(err));
+    set_error("q4_linear(AWQ, %s rows): launch failed: %s", M > q4::kAwqFewRows ? "five to sixteen" : "up to four", hipGetErrorString(err));
     return Q4_ERR_LAUNCH;
   }
   return Q4_OK;

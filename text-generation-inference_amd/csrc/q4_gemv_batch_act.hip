@@ -89,8 +89,8 @@ static void act_wide(const q4_weight* w, int M, BatchPlan* plan) {
 // K splits are powers of two unless the estimate of another number is a tenth below theirs, with two row blocks a fifth (20 layer shapes x
 // 6, 16, 24 and 48 rows: 1.02-1.05 in geometric mean over powers of two alone, 5120 x 13824 at 48 rows 1.29, least 0.96; any number
 // whatever the estimates differ by: down to 0.91).
-// Plain launches of a few rows whose powers of two deal K out unevenly are the decode path's (launch_gemv), which runs this
-// kernel with any number of splits up to five rows (batch_act_few_default), us, gemv_gptq_act_kernel / so: 8192 x 10240, 4 rows 17.7 / 16.3,
+// Plain launches of a few rows whose powers of two deal K out unevenly are the decode path's; up to five rows they run on this
+// kernel all the same, with any number of splits (batch_act_few_default), us, gemv_gptq_act_kernel / so: 8192 x 10240, 4 rows 17.7 / 16.3,
 // 9344 x 18560 40.5 / 27.9, 4096 x 11008 15.5 / 11.4, 3584 x 4608 8.2 / 7.5; 18 shapes 1.14 in geometric mean, one row of very long K
 // 0.98 (18944 x 3584 15.4 / 15.7), left to the older kernel.  Groups of 32, whose tables leave room for fewer
 // workgroups, 8192 x 10240 1 row 19.6 / 22.2, 16 rows 22.4 / 23.3 (gated fp16 21.5 / 24.0 and 24.5 / 25.5, bf16 up to 2 rows; gated 9344 x
@@ -112,7 +112,7 @@ bool batch_act_default(const q4_weight* w, int M, int dtype, bool gate_up, Batch
   return !(dtype == Q4_DTYPE_F16 ? M <= 5 && uneven >= 1.11 : M <= 2 && uneven >= 1.19 && w->K >= 8192);
 }
 
-// Plain calls of a few rows that batch_act_default leaves to the decode path (launch_gemv): with any number of workgroups along K.
+// Plain calls of a few rows that batch_act_default leaves to the decode path (decode_few_default): with any number of workgroups along K.
 bool batch_act_few_default(const q4_weight* w, int M, int dtype, BatchPlan* plan) {
   double uneven;
   if ((dtype == Q4_DTYPE_F16 && M == 1 && w->K > 5 * w->N) || (w->num_groups >= 256 && (double)w->K * w->N >= 2.6e8)) return false;
