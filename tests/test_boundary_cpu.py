@@ -325,6 +325,13 @@ def test_k_waves_of_unsplit_batch_tiles(pkg, M, K, N, gs, gate_up, want):
     assert _all_tiles(pkg, M, K, N, gs, "f16", gate_up=gate_up) == ((M + 15) // 16 * 16, 128, want, 1)
 
 
+@pytest.mark.parametrize("M,K,N,gs,dtype,gate_up,want", [(8, 2560, 10112, 64, "f16", 0, (16, 64, 8, 1)), (5, 12800, 18816, 64, "bf16", 1, (16, 64, 8, 2)),
+                                                        (11, 8704, 3584, 128, "f16", 0, (16, 64, 8, 4)), (39, 18688, 10624, 128, "bf16", 1, (48, 64, 4, 3)), (48, 13440, 2304, 128, "bf16", 0, (48, 64, 8, 7))])
+def test_splits_of_the_act_order_batch_kernel(pkg, M, K, N, gs, dtype, gate_up, want):
+    """Powers of two unless another number is well ahead of them, eight waves kept at more than that."""
+    assert _all_tiles(pkg, M, K, N, gs, dtype, gate_up=gate_up, g_idx=True) == want
+
+
 FEW = "q4_linear(AWQ, up to four rows)"
 
 

@@ -86,9 +86,9 @@ static void act_wide(const q4_weight* w, int M, BatchPlan* plan) {
 // 32 and 128, both types, time of theirs over time of this one in geometric mean (least):
 //   1-5 rows 1.19 (0.96), 16 1.22 (1.00), 17 1.58 (1.07), 33 1.85 (1.35), 64 1.50 (1.15).  us, theirs / this one: 8192 x 57344
 //   gated 1 row 85.7 / 67.8, 33 rows 205 / 123; 28672 x 8192 4 rows 41.8 / 36.7, 33 rows 125 / 54; 4096 x 4096 16 rows 9.5 / 7.7.
-// K splits are powers of two unless the estimate of another number is a tenth below theirs, with two row blocks a fifth (20 layer shapes x
-// 6, 16, 24 and 48 rows: 1.02-1.05 in geometric mean over powers of two alone, 5120 x 13824 at 48 rows 1.29, least 0.96; any number
-// whatever the estimates differ by: down to 0.91).
+// K splits are powers of two unless the estimate of another number is a tenth below theirs, with two row blocks a fifth, and a fifth too
+// where it gives up to sixteen rows four waves in place of eight: 293 such calls 1.13 in geometric mean over powers of two alone (0.93-1.48); 30 more of four
+// waves for a tenth 0.99, 0.88 at worst (2560 x 10112 8 rows 9.5 / 10.8 us, 12800 x 18816 gated 5 bf16 rows 50.3 / 56.8).
 // Plain launches of a few rows whose powers of two deal K out unevenly are the decode path's; up to five rows they run on this
 // kernel all the same, with any number of splits (batch_act_few_default), us, gemv_gptq_act_kernel / so: 8192 x 10240, 4 rows 17.7 / 16.3,
 // 9344 x 18560 40.5 / 27.9, 4096 x 11008 15.5 / 11.4, 3584 x 4608 8.2 / 7.5; 18 shapes 1.14 in geometric mean, one row of very long K
@@ -101,7 +101,8 @@ bool batch_act_default(const q4_weight* w, int M, int dtype, bool gate_up, Batch
   const double pow2_us = act_plan(w, M, (M + 15) / 16, true, plan, &uneven);
   if (pow2_us < 0.0) return false;
   BatchPlan any;
-  if (act_plan(w, M, (M + 15) / 16, false, &any, &uneven_any) < (M > 16 && M <= 32 ? 0.8 : 0.9) * pow2_us) *plan = any;
+  const double any_us = act_plan(w, M, (M + 15) / 16, false, &any, &uneven_any);
+  if (any_us < ((M > 16 && M <= 32) || (M <= 16 && plan->wk == 8 && any.wk == 4) ? 0.8 : 0.9) * pow2_us) *plan = any;
   const double weights = (double)w->K * w->N;
   if (w->num_groups >= 256 && M <= 16 && weights >= 2.6e8 && M > 2) return false;
   if (w->num_groups >= 256 && M <= 16 && weights < 2.6e8 && uneven >= 1.19 && (!gate_up || (weights < 1.2e8 && (dtype == Q4_DTYPE_F16 || M <= 2))))
