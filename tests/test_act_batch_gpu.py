@@ -5,6 +5,8 @@ Bars: max|y - ref| / max|ref| <= 2e-3 in fp16 (output rounding 2^-11 plus the fp
 bf16 (three roundings of 2^-8).
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -142,3 +144,26 @@ def test_tiles_and_splits(pkg, oracle, gpu, K, N, gs, M, dtype, sym):
     hot[torch.arange(M), ks] = 1
     back = pkg.ops.linear(pk, hot).cpu().view(torch.int16).numpy().view(np.uint16)
     assert np.array_equal(back & 0x7FFF, w[ks.numpy()].view(np.uint16) & 0x7FFF)  # (a zero may have lost its sign)
+
+
+@pytest.mark.parametrize("M", [1, 4, 16])
+@pytest.mark.parametrize("sym", [False, True])
+def test_wide_gated_tiles_in_workgroups_along_k(pkg, gpu, M, sym):
+    """128-column tiles beyond one a CU: against the plain launch on 64 columns and the elementwise kernel, whose roundings are the same and whose
+    fp32 sums are in another order, so that an output is off by its sums' last place (2^-11 each) now and then."""
+    K, N, gs, g = 5120, 49152, 128, torch.Generator(device=gpu).manual_seed(M)
+    words = lambda *s: torch.randint(-(2**31), 2**31 - 1, s, dtype=torch.int32, device=gpu, generator=g)  # noqa: E731
+    qz = torch.full((K // gs, N // 8), 0x77777777, dtype=torch.int32, device=gpu) if sym else words(K // gs, N // 8)
+    sc = (torch.rand((K // gs, N), device=gpu, generator=g) * 0.01 + 0.001).half()
+    g_idx = (torch.arange(K, device=gpu) // gs)[torch.randperm(K, device=gpu, generator=g)].to(torch.int32)
+    pk = pkg.ops.make_packed(words(K // 8, N), qz, sc, g_idx, gs, 0)
+    tiles = (ctypes.c_int * 4)()
+    assert pkg._lib.load().q4_linear_tiles(ctypes.byref(pk.struct()), M, 0, 1, tiles) == 0 and tiles[1] == 128 and tiles[3] > 1
+    x = (torch.randn((M, K), device=gpu, generator=g) / 16).half()
+    got, sums = pkg.ops.linear_gate_up(pk, x, "silu"), pkg.ops.linear(pk, x)
+    assert torch.equal(got, pkg.ops.linear_gate_up(pk, x, "silu"))
+    want, (gate, up) = pkg.ops.act_mul(sums, "silu").double(), sums.double().chunk(2, dim=1)
+    # the sums' last place through the product (slope of silu at most 1.1), and the two roundings behind them
+    bar = 2.0**-10 * (1.1 * gate.abs() * up.abs() + torch.nn.functional.silu(gate).abs() * up.abs()) + 2.0**-9 * want.abs() + 2.0**-24
+    assert bool(((got.double() - want).abs() <= bar).all())
+    assert float((got != want).double().mean()) < 0.05

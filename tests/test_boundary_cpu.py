@@ -326,7 +326,8 @@ def test_k_waves_of_unsplit_batch_tiles(pkg, M, K, N, gs, gate_up, want):
 
 
 @pytest.mark.parametrize("M,K,N,gs,dtype,gate_up,want", [(8, 2560, 10112, 64, "f16", 0, (16, 64, 8, 1)), (5, 12800, 18816, 64, "bf16", 1, (16, 64, 8, 2)),
-                                                        (11, 8704, 3584, 128, "f16", 0, (16, 64, 8, 4)), (39, 18688, 10624, 128, "bf16", 1, (48, 64, 4, 3)), (48, 13440, 2304, 128, "bf16", 0, (48, 64, 8, 7))])
+                                                        (11, 8704, 3584, 128, "f16", 0, (16, 64, 8, 4)), (13, 2304, 50816, 128, "f16", 1, (16, 64, 4, 1)),
+                                                        (4, 8192, 57344, 128, "f16", 1, (16, 128, 4, 4)), (4, 4096, 28672, 128, "f16", 1, (16, 128, 8, 1)), (39, 18688, 10624, 128, "bf16", 1, (48, 64, 4, 3)), (48, 13440, 2304, 128, "bf16", 0, (48, 64, 8, 7))])
 def test_splits_of_the_act_order_batch_kernel(pkg, M, K, N, gs, dtype, gate_up, want):
     """Powers of two unless another number is well ahead of them, eight waves kept at more than that."""
     assert _all_tiles(pkg, M, K, N, gs, dtype, gate_up=gate_up, g_idx=True) == want

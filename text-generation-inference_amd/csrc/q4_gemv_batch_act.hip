@@ -70,9 +70,11 @@ static double act_plan(const q4_weight* w, int M, int mt, bool pow2, BatchPlan* 
 // waves, from one and a half on four waves, split along K as far as the cells allow (8192 x 57344, 4 rows, one
 // workgroup / two / four along K: one zero point 53.3 / 54.0 / 53.7 us, others 67.8 / 67.1 / 65.1; on 64 columns 57-60 and 64-66).  In
 // between (3584 x 37888, 296 tiles) a second round is nearly empty: 25.2 us, and 31.0 against 26.6 with several zero points.
+// Below 5120 rows of K a workgroup along K has too few words to its table: from 384 tiles on 0.93-1.10 of the 64-column tiles' speed, 27 calls 0.98 in
+// geometric mean (2304 x 50816 13 rows 23.6 us there, 25.4 here), from 5120 on 31 calls 1.06 (0.96-1.23), 192-256 tiles 1.06 (0.97-1.16).
 static void act_wide(const q4_weight* w, int M, BatchPlan* plan) {
   const int chunks = w->K / 128, tiles = w->N / 128;
-  if (w->N % 128 != 0 || tiles < 192 || (tiles > 256 && tiles < 384) || w->num_groups > 96 || chunks < 16) return;
+  if (w->N % 128 != 0 || tiles < 192 || (tiles > 256 && (tiles < 384 || w->K < 5120)) || w->num_groups > 96 || chunks < 16) return;
   int splits = 1;
   while (tiles > 256 && splits < 4 && (2L * splits - 1) * act_units(2, M) * tiles * 512 <= Q4_WORKSPACE_CELL_BYTES) splits *= 2;
   const int wk = tiles <= 256 ? 8 : 4;
