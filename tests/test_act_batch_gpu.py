@@ -115,7 +115,7 @@ def test_replays(pkg, oracle, gpu):
         assert torch.equal(pkg.ops.linear(pk, x), want[0])
 
 
-@pytest.mark.parametrize("K,N,gs", [(4096, 28672, 128), (2048, 24576, 64), (2176, 49152, 128), (5504, 192, 128), (4608, 4608, 128), (18944, 256, 256)])
+@pytest.mark.parametrize("K,N,gs", [(4096, 28672, 128), (2048, 24576, 64), (2176, 49152, 128), (5504, 192, 128), (4608, 4608, 128), (18944, 256, 256), (8192, 1280, 32), (2304, 1152, 32)])
 @pytest.mark.parametrize("M,dtype", [(1, "f16"), (3, "bf16"), (4, "f16"), (5, "f16"), (16, "f16"), (37, "bf16")])
 @pytest.mark.parametrize("sym", [False, True])
 def test_tiles_and_splits(pkg, oracle, gpu, K, N, gs, M, dtype, sym):

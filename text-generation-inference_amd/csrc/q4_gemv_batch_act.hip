@@ -94,9 +94,11 @@ static void act_wide(const q4_weight* w, int M, BatchPlan* plan) {
 // Plain launches of a few rows whose powers of two deal K out unevenly are the decode path's; up to five rows they run on this
 // kernel all the same, with any number of splits (batch_act_few_default), us, gemv_gptq_act_kernel / so: 8192 x 10240, 4 rows 17.7 / 16.3,
 // 9344 x 18560 40.5 / 27.9, 4096 x 11008 15.5 / 11.4, 3584 x 4608 8.2 / 7.5; 18 shapes 1.14 in geometric mean, one row of very long K
-// 0.98 (18944 x 3584 15.4 / 15.7), left to the older kernel.  Groups of 32, whose tables leave room for fewer
-// workgroups, 8192 x 10240 1 row 19.6 / 22.2, 16 rows 22.4 / 23.3 (gated fp16 21.5 / 24.0 and 24.5 / 25.5, bf16 up to 2 rows; gated 9344 x
-// 18560 is faster here, 1.1 and more), and 8192 x 57344 from 3 rows on, gated 5 rows 91.7 / 99.0.
+// 0.98 (18944 x 3584 15.4 / 15.7), left to the older kernel.  256 groups and more, whose tables leave room for fewer
+// workgroups, among them: 8192 x 10240 in groups of 32, 1 row 20.1 / 20.1 (22.2 in powers of two), 4 rows 19.9 / 19.2, bf16 20.9 / 19.9 and 22.1 /
+// 19.7; 94 calls of ten shapes, nearly all in groups of 32, 1.22 in geometric mean (1.00-1.78).  Left to the older kernel with such groups: 8192 x
+// 10240 16 rows 22.4 / 23.3 (gated fp16 1 row 21.5 / 24.0, 16 rows 24.5 / 25.5, bf16 up to 2 rows; gated 9344 x 18560 is faster here, 1.1 and more), and 8192 x
+// 57344 from 3 rows on, gated 5 rows 91.7 / 99.0.
 bool batch_act_default(const q4_weight* w, int M, int dtype, bool gate_up, BatchPlan* plan) {
   double uneven = 1.0, uneven_any = 1.0;
   if (M > 64 || !act_supported(w, M, gate_up)) return false;
