@@ -318,10 +318,10 @@ def _launched(pkg, w, M, dtype, gate_up=0, path=0):
     return lib.q4_last_error().decode().split(":")[0] if rc == pkg._lib.ERR_LAUNCH else rc
 
 
-@pytest.mark.parametrize("M,K,N,gs,gate_up,want", [(5, 13312, 27392, 64, 0, 8), (31, 3584, 28672, 64, 0, 8), (10, 3968, 28672, 64, 0, 4), (4, 4608, 30720, 64, 1, 4),
+@pytest.mark.parametrize("M,K,N,gs,gate_up,want", [(5, 13312, 27392, 64, 0, 8), (31, 3584, 28672, 64, 0, 8), (10, 3968, 28672, 64, 0, 8), (2, 3072, 24960, 64, 0, 8),
                                                   (1, 4096, 28672, 128, 1, 4), (31, 8192, 28672, 128, 0, 4), (5, 4096, 28672, 32, 0, 8)])
 def test_k_waves_of_unsplit_batch_tiles(pkg, M, K, N, gs, gate_up, want):
-    """Four waves for 128-column tiles that fill the chip, in groups of 64 over a short K and few rows only."""
+    """Four waves for 128-column tiles that fill the chip, eight in groups of 64 and 32 rows."""
     assert _all_tiles(pkg, M, K, N, gs, "f16", gate_up=gate_up) == ((M + 15) // 16 * 16, 128, want, 1)
 
 
