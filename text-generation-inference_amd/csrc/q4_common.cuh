@@ -234,7 +234,7 @@ size_t gemv_direct_workspace_bytes(const q4_weight* w, int M, int dtype, int spl
 bool gemv_direct_default(const q4_weight* w, int M, int dtype, int* wk, int* splits);
 int launch_gemv_direct(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, void* workspace,
                        size_t workspace_bytes, int wk, int splits, hipStream_t stream);
-// AWQ, one to four rows (q4_gemv_awq_few.cuh)
+// AWQ, up to four rows (q4_gemv_awq_few.cuh); its plan and launch also serve five to sixteen rows (q4_gemv_awq_wide.cuh)
 struct AwqFewPlan {
   int wn;      // column waves of a workgroup; 0: no plan
   int wk;      // K waves
@@ -242,7 +242,7 @@ struct AwqFewPlan {
 };
 bool awq_few_supported(const q4_weight* w, int M, bool gate_up);
 bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan);
-// five to sixteen rows (q4_gemv_awq_wide.cuh); launched by launch_awq_few
+// five to sixteen rows; launched by launch_awq_few
 bool awq_wide_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan);
 int launch_awq_few(const q4_weight* w, const void* x, const void* bias, void* y, int M, int dtype, int gate_up_act, void* workspace,
                    size_t workspace_bytes, const AwqFewPlan& plan, hipStream_t stream);

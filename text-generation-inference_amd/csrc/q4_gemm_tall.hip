@@ -59,10 +59,11 @@ static double tall_plan(bool awq, int dtype, int M, int K, int N, bool gate_up, 
   // Two halves of K in a workgroup, 128 columns: as many CUs at work with half the splits, whose fp32 partial sums (8 M N bytes each, out and in)
   // otherwise cost up to a third of a call; every fragment of x then serves half as many columns, which is why they end where two
   // splits and less would do.  Fitted to 15 layer shapes x 100-640 rows x all heights and splits, within 7 % where the workgroups are one round;
-  // where it puts them 2 % ahead they run.  188 such calls of 24 layer shapes at 65-1536 rows 1.17 in geometric mean (0.96-1.71), 150 of
-  // any shape 1.20 (0.99); us, before / so: 3584 x 8192 301 rows 35.7 / 30.2, bf16 35.1 / 30.9, 1024 x 8192 301 rows 17.4 / 12.8, 14336 x 4096 89
-  // rows 30.7 / 25.0, 3584 x 3584 1000 rows 40.3 / 35.5, 4096 x 6144 301 rows 29.9 / 30.0.  (A price on padded rows, which left the last one
-  // out, cost 90 calls that it changed 1.09 in geometric mean.  AWQ, whose words are loaded row by row, 0.75-1.1: not built in.)
+  // where it puts them 2 % ahead they run.  1319 such calls at 65-1536 rows, weights from memory, 1.15 in geometric mean (0.93-1.77, 15 below
+  // 0.97; 366 of serving models' layer shapes 1.12); us, before / so: 3584 x 8192 301 rows 33.9 / 28.9, bf16 35.2 / 30.3, 1024 x 8192 301 rows
+  // 17.5 / 12.8, 14336 x 4096 89 rows 30.5 / 24.9, 3584 x 3584 1000 rows 39.9 / 34.3, 209 rows 19.7 / 21.1, 4096 x 6144 301 rows 29.9 / 29.6 (a whole
+  // layer 0.995-1.00).  (A price on padded rows, which left the last two out, cost 90 calls that it changed 1.09 in geometric mean; a lead of 4 %
+  // instead of 2 cost 534 calls 1.07.  AWQ, whose words are loaded row by row, 0.75-1.1: not built in.)
   static const double kHalves[3][2] = {{0.54, 0.81}, {0.69, 1.00}, {0.85, 1.23}};  // (bf16: 0.065 more)
   const int KT = K / q4::kBK;
   for (int r = 3; r <= 5; ++r)

@@ -172,7 +172,7 @@ int launch_batch_act(const q4_weight* w, const void* x, const void* bias, void* 
   const bool few = act_few(w, M, plan.nq, plan.wk, plan.splits);
   const size_t lds = q4::batch_act_lds(w->num_groups, act_k_rows(w, plan.wk, plan.splits), plan.wk, mt, plan.nq, few);
   if (lds > kActLds) {
-    set_error("q4_linear(act-order batch kernel): %zu bytes of LDS needed without a workspace", lds);
+    set_error("q4_linear(act-order batch kernel): %zu bytes of LDS needed%s", lds, act_cells(workspace, workspace_bytes) ? "" : " without a workspace");
     return Q4_ERR_WORKSPACE;
   }
   BatchParams bp = {};
