@@ -28,7 +28,7 @@ def _case(pkg, oracle, gpu, K, N, gs, seed):
 
 # K: one chunk a wave, ragged deals (17, 43, 67 chunks), an odd number of workgroups along K; N: one tile, an odd number, pairs of tiles
 @pytest.mark.parametrize("K,N,gs", [(2048, 256, 128), (2176, 768, 128), (5504, 512, 256), (8576, 1280, 128), (4096, 28672, 128), (14336, 4096, -1),
-                                    (8192, 10240, 512), (2176, 16640, 128), (5504, 6400, 128)])
+                                    (8192, 10240, 512), (2176, 16640, 128), (5504, 6400, 128), (4992, 4096, 128)])
 @pytest.mark.parametrize("M,dtype", [(1, "f16"), (1, "bf16"), (2, "f16"), (3, "bf16"), (4, "f16"), (4, "bf16")])
 def test_plain(pkg, oracle, gpu, K, N, gs, M, dtype):
     gs = gs if gs == -1 or K % gs == 0 else 128

@@ -353,7 +353,7 @@ def test_a_forced_decode_path_runs_its_own_kernels(pkg, K, N, layout, g_idx, M, 
 
 
 # (K in whole 128-row chunks, one and more a wave; fewer and more units of 128 x 256 weights than the chip has SIMDs)
-@pytest.mark.parametrize("K,N,gate_up,dtype,few", [(2176, 4096, 0, 0, False), (2176, 16384, 0, 0, True), (3968, 8192, 0, 1, False), (2048, 512, 0, 0, True), (8320, 1024, 0, 1, True),
+@pytest.mark.parametrize("K,N,gate_up,dtype,few", [(2176, 4096, 0, 0, False), (2176, 16384, 0, 0, True), (2176, 8960, 0, 0, False), (2176, 9216, 0, 0, True), (3968, 8192, 0, 1, False), (2048, 512, 0, 0, True), (8320, 1024, 0, 1, True),
                                                    (2176, 4096, 1, 0, False), (2176, 20480, 1, 0, True), (11008, 2048, 1, 0, False), (11008, 3072, 1, 0, True),
                                                    (2048, 4096, 1, 0, True), (4096, 4096, 1, 1, False), (4096, 8192, 1, 1, True)])
 def test_awq_rows_of_small_ragged_layers(pkg, K, N, gate_up, dtype, few):

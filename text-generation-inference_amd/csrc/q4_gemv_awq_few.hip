@@ -60,10 +60,10 @@ static bool awq_few_plan(const q4_weight* w, int M, bool gate_up, AwqFewPlan* pl
 // 57344 0.95-1.03).  So are layers of fewer 16 KB units (128 rows x 256 columns) than the chip has SIMDs, about 1000, of which some wave walks
 // two: the CUs that have work then read twice what the batch kernel's 128-column tiles give them (chunks of K: us at one row, theirs / this one;
 // 2122 calls of 14 widths x 22 lengths).
-//   plain, up to 8192 rows of K   17 chunks x 4096 columns 0.91, bf16 0.85-0.86; 31 x 8192 0.96-0.98, 0.90-0.93; from 1000 units on 0.98-1.6,
-//                                 longer ones 1.00 and more whatever the units
+//   plain, up to 8192 rows of K   17 chunks x 4096 columns 0.91, bf16 0.85-0.86; 31 x 8192 bf16 0.90-0.93; fp16 from 600 units on (75 calls up to 1000,
+//                                 weights from memory, 1.07, least 1.00: 47 x 5120 10.1 / 8.7; below, 194 calls 0.96), bf16 from 1000; longer ones 1.00 and more whatever the units
 //   gated                         17 x 4096 0.81, 63 x 4096 0.89-0.92, 86 x 2048 0.93; fp16 from 1100 units on, bf16 from 1300, from 1000 beyond
-//                                 8192 rows; 18 x 16384 0.92-0.95, bf16 0.89-0.90
+//                                 8192 rows; 18 x 16384 0.92-0.95, bf16 0.89-0.90; weights from memory, 323 fp16 calls below the line 0.93
 //   gated bf16, one chunk a wave  4096 x 4096 0.91-0.94, 4096 x 6144 0.98-1.00: from 800 units on
 // (20480 columns in fp16 0.92-0.99 over 39-86 chunks, 19456 and 21504 1.1-1.3: kept.)
 bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewPlan* plan) {
@@ -73,7 +73,7 @@ bool awq_few_default(const q4_weight* w, int M, int dtype, bool gate_up, AwqFewP
   if (!awq_few_plan(w, M, gate_up, &own)) return false;
   const long chunks = w->K / 128, units = chunks * (w->N / 256);
   const bool bf16_gated = gate_up && dtype == Q4_DTYPE_BF16, one_each = chunks <= (long)own.wk * own.splits;
-  if (!one_each && units < (w->K > 8192 ? (gate_up ? 1000 : 0) : (bf16_gated ? 1300 : (gate_up ? 1100 : 1000)))) return false;
+  if (!one_each && units < (w->K > 8192 ? (gate_up ? 1000 : 0) : (bf16_gated ? 1300 : (gate_up ? 1100 : (dtype == Q4_DTYPE_BF16 ? 1000 : 600))))) return false;
   if (bf16_gated && one_each && w->K <= 4096 && units < 800) return false;
   *plan = own;
   return true;
